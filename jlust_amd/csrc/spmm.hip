@@ -9,20 +9,14 @@
 // from column-major B touches k cache lines 4*ldb bytes apart for k useful
 // values, so the kernel first re-lays B out row-major (Bt, n x ldt) in the
 // library's scratch buffer with an LDS-tiled transpose: one coalesced read
-// and one coalesced write of B.  Then:
-//   - a block owns SPMM_ROWS consecutive rows; each wave walks one row at a
-//     time, its 64 lanes covering a 64*VEC-column chunk (VEC consecutive
-//     columns per lane, one vector load per lane per nonzero, so one nonzero
-//     reads a contiguous 64*VEC*sizeof(T)-byte slice of Bt);
-//   - the row's col/val are read 64 at a time with one coalesced load and
-//     broadcast lane by lane (v_readlane), several B slices in flight;
-//   - results are staged in LDS and written to column-major C column by
-//     column (SPMM_ROWS consecutive values per column), so C writes are
-//     coalesced too.
+// and one coalesced write of B.  csr_spmm_rows_kernel then gathers whole rows
+// of Bt for several rows of A at once, and writes its results column by column
+// through LDS.  One column needs no copy (csr_spmm_col_kernel).
 #include "common.hpp"
 
 #include <cstdlib>
 #include <memory>
+#include <type_traits>
 #include <vector>
 
 namespace jlust {
@@ -32,7 +26,6 @@ constexpr int SPMM_BLOCK = 256;
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 constexpr int SPMM_ROWS = 32;
-constexpr int SPMM_UNROLL = 8;
 
 template <typename T>
 __device__ __forceinline__ T bcast(T v, int lane);
@@ -56,63 +49,65 @@ template <typename T> struct Vec<T, 1> { T v[1]; };
 template <typename T> struct alignas(2 * sizeof(T)) Vec<T, 2> { T v[2]; };
 template <typename T> struct alignas(4 * sizeof(T)) Vec<T, 4> { T v[4]; };
 
-// Bt[j*ldt + c] = B[j + c*ldb] for j < n, c < k (64 x 64 tiles through LDS).
-template <typename T>
-__global__ __launch_bounds__(256) void transpose_kernel(int64_t n, int64_t k,
-                                                        const T *__restrict__ B, int64_t ldb,
-                                                        T *__restrict__ Bt, int64_t ldt)
+// Bt[j*ldt + c] = B[j + c*ldb] for j < n, c < k, in tiles of CT columns and
+// 4096/CT rows through LDS: columns are read 64 rows at a time, rows written
+// VEC columns at a time.  CT is the smallest of 16, 32 and 64 that holds the
+// columns, so a narrow B's tile holds as many entries as a wide one's (262k
+// rows, f64, 20 columns: 19.4 us with 64-column tiles and one column per
+// write, 16.2 us).  Padding columns (ldt beyond k) take what the tile holds,
+// and are never used; row n of Bt is zeroed for the lanes of the rows kernel
+// that have no entry.
+template <typename T, int VEC, int CT>
+__global__ __launch_bounds__(256) void transpose_kernel(int64_t n, int64_t k, const T *__restrict__ B,
+                                                        int64_t ldb, T *__restrict__ Bt, int64_t ldt)
 {
-    __shared__ T tile[64][65];
-    const int tx = threadIdx.x & 63;
-    const int ty = threadIdx.x >> 6;
-    const int64_t j0 = (int64_t)blockIdx.x * 64;
-    const int64_t c0 = (int64_t)blockIdx.y * 64;
+    constexpr int JT = 4096 / CT;
+    constexpr int UR = CT / VEC;               // writes per row of the tile
+    __shared__ T tile[CT][JT + 1];
+    const int64_t j0 = (int64_t)blockIdx.x * JT;
+    const int64_t c0 = (int64_t)blockIdx.y * CT;
+    const int ncol = (int)min((int64_t)CT, k - c0);
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
-        const int cc = ty + 4 * s;
-        const int64_t j = j0 + tx, c = c0 + cc;
-        if (j < n && c < k) tile[cc][tx] = B[j + c * ldb];
+        const int i = threadIdx.x + 256 * s;
+        const int cc = i / JT, jj = i % JT;
+        if (j0 + jj < n && cc < ncol) tile[cc][jj] = B[j0 + jj + (c0 + cc) * ldb];
     }
     __syncthreads();
+    const int nwr = (int)min((int64_t)CT, ldt - c0);
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const int jj = ty + 4 * s;
-        const int64_t j = j0 + jj, c = c0 + tx;
-        if (j < n && c < k) Bt[j * ldt + c] = tile[tx][jj];
+    for (int s = 0; s < 16 / VEC; ++s) {
+        const int i = threadIdx.x + 256 * s;
+        const int jj = i / UR, cc = i % UR * VEC;
+        if (cc >= nwr || j0 + jj > n) continue;
+        Vec<T, VEC> v;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v.v[e] = j0 + jj < n ? tile[cc + e][jj] : T(0);
+        *reinterpret_cast<Vec<T, VEC> *>(Bt + (j0 + jj) * ldt + c0 + cc) = v;
     }
 }
 
-// Chunks of at most 32 columns: groups of KV lanes (KV the smallest power of
-// two >= the chunk's columns), one nonzero per group per step, so a wave
-// takes 64/KV nonzeros per step (64 at k = 1, where the kernel is a
-// wave-per-row SpMV).  Each lane loads its group's col/val itself (the
-// group's lanes read one address), gathers its column of the nonzero's Bt
-// row, and keeps its group's sum in nonzero order; the groups' sums are added
-// with xor-shuffles at the row's end.  U steps are loaded at once (indices
-// clamped into the row, products of the clamped copies dropped by a select;
-// U is chosen per call from the mean row length, so a short row issues no
-// clamped copies), and the next row's pointers are loaded before the current
-// row's nonzeros, so a wave's rows do not wait on each other's pointer loads.
-template <typename T, int KV, int U>
-__global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_group_kernel(
-    int64_t m, int64_t k, int32_t origin, const int32_t *__restrict__ rowptr,
-    const int32_t *__restrict__ colind, const T *__restrict__ val, const T *__restrict__ Bt,
-    int64_t ldt, T alpha, T beta, int beta_zero, T *__restrict__ C, int64_t ldc,
-    int skip_empty_rows, const int32_t *__restrict__ rowend, const uint8_t *__restrict__ row_skip)
+// One column: a wave per row, 64 entries per step, gathered from B's own
+// column.  U steps are loaded at once (indices clamped into the row, products
+// of the clamped copies dropped by a select; U is chosen per call from the mean
+// row length, so a short row issues no clamped copies), and the next row's
+// pointers are loaded before the current row's nonzeros, so a wave's rows do
+// not wait on each other's pointer loads.
+template <typename T, int U>
+__global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_col_kernel(
+    int64_t m, int32_t origin, const int32_t *__restrict__ rowptr, const int32_t *__restrict__ rowend,
+    const uint8_t *__restrict__ row_skip, const int32_t *__restrict__ colind, const T *__restrict__ val,
+    const T *__restrict__ B, T alpha, T beta, int beta_zero, T *__restrict__ C, int skip_empty_rows)
 {
-    constexpr int G = 64 / KV;                 // nonzeros per step
     constexpr int NW = SPMM_BLOCK / 64;
-    __shared__ T s_c[SPMM_ROWS][KV + 1];
+    __shared__ T s_c[SPMM_ROWS];
     __shared__ int s_empty[SPMM_ROWS];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int grp = lane / KV;
-    const int col = lane % KV;
     const int64_t row0 = (int64_t)blockIdx.x * SPMM_ROWS;
     const int nrows = (int)min((int64_t)SPMM_ROWS, m - row0);
-    const int64_t cl = col < k ? col : 0;      // clamped, in-bounds column
 
     int32_t lo_n = 0, hi_n = 0;
     if (wave < nrows) {
@@ -130,125 +125,302 @@ __global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_group_kernel(
         if (skip) hi = lo;                     // a split row: its segments compute it
         if (lane == 0) s_empty[rr] = skip ? 2 : hi <= lo;
         T acc = T(0);
-        for (int64_t p0 = lo + grp; p0 < hi; p0 += (int64_t)G * U) {
+        for (int64_t p0 = lo + lane; p0 < hi; p0 += (int64_t)64 * U) {
             int32_t c[U];
             T a[U], b[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int64_t p = min(p0 + (int64_t)u * G, hi - 1);
+                const int64_t p = min(p0 + (int64_t)u * 64, hi - 1);
                 c[u] = colind[p];
                 a[u] = val[p];
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) b[u] = Bt[(int64_t)(c[u] - origin) * ldt + cl];
+            for (int u = 0; u < U; ++u) b[u] = B[c[u] - origin];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const T s = acc + a[u] * b[u];
-                acc = p0 + (int64_t)u * G < hi ? s : acc;
+                acc = p0 + (int64_t)u * 64 < hi ? s : acc;
             }
         }
 #pragma unroll
-        for (int off = KV; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
-        if (lane < KV) s_c[rr][col] = acc;
+        for (int off = 1; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
+        if (lane == 0) s_c[rr] = acc;
     }
     __syncthreads();
-    const int ncols = (int)k;                  // k <= KV here
-    for (int idx = tid; idx < SPMM_ROWS * ncols; idx += SPMM_BLOCK) {
-        const int rr = idx % SPMM_ROWS;
-        const int cc = idx / SPMM_ROWS;
-        if (rr >= nrows) continue;
-        if (s_empty[rr] == 2 || (skip_empty_rows && s_empty[rr])) continue;
-        T *dst = C + (row0 + rr) + cc * ldc;
-        const T s = alpha * s_c[rr][cc];
-        *dst = beta_zero ? s : s + beta * *dst;
-    }
+    if (tid >= nrows || s_empty[tid] == 2 || (skip_empty_rows && s_empty[tid])) return;
+    T *dst = C + row0 + tid;
+    const T s = alpha * s_c[tid];
+    *dst = beta_zero ? s : s + beta * *dst;
 }
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_kernel(
-    int64_t m, int64_t k, int32_t origin, const int32_t *__restrict__ rowptr,
-    const int32_t *__restrict__ colind, const T *__restrict__ val, const T *__restrict__ Bt,
-    int64_t ldt, T alpha, T beta, int beta_zero, T *__restrict__ C, int64_t ldc,
-    int skip_empty_rows, const int32_t *__restrict__ rowend, const uint8_t *__restrict__ row_skip)
+// A set of rows for csr_spmm_rows_kernel: the matrix's rows (hi null: row r
+// ends where r + 1 starts), or the segments of a plan's split rows.
+template <typename T>
+struct SpmmJob {
+    int64_t rows = 0;
+    const int32_t *lo = nullptr, *hi = nullptr;
+    const uint8_t *skip = nullptr;       // rows left untouched
+    T alpha = T(0), beta = T(0);
+    T *C = nullptr;
+    int64_t ldc = 0;
+    int beta_zero = 1, skip_empty_rows = 0;
+    int R = 1;                           // rows per block, at most 64
+    unsigned blocks = 0;
+    unsigned run = 1;                    // consecutive blocks per XCD
+};
+
+// Most entries of a block staged at once, and most slices of rows among them:
+// a remainder per row, and one per 32 entries.
+constexpr int SPMM_STAGE = 2040;
+constexpr int SPMM_TASKS = 64 + SPMM_STAGE / 32 + 2;
+
+// How the columns lie over a wave, and the block's buffers.
+struct SpmmShape {
+    int64_t k;                           // columns of the pass
+    int64_t ldt;                         // row stride of Bt
+    int64_t zero_row;                    // Bt's row of zeros
+    int cols;                            // columns per blockIdx.y, a multiple of VEC
+    int L;                               // lanes per entry: cols / VEC
+    int slice_log2;                      // entries of a slice
+    int cld;                             // row stride of the result tile
+    int rmax;                            // rows of the result tile
+    int ch;                              // entries staged at once, above a slice
+    int xmax;                            // further slices of the staged rows
+};
+
+__device__ __forceinline__ int wave_min(int v)
 {
-    constexpr int KC = 64 * VEC;              // columns per chunk
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) v = min(v, __shfl_xor(v, off, 64));
+    return v;
+}
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
+
+// Row-split SpMM over the row-major copy of B.  A wave's 64 lanes form
+// NG = 64 / L groups; a group takes a row, each lane VEC columns of B's row per
+// entry, so one vector load of a wave serves NG entries of NG rows and no sum crosses lanes.  What bounds it is the gathers: L1 and L2 where rows share
+// columns, the fabric behind the L2s where they do not.
+//   - The block's entries (colind turned into an offset into Bt, and val) are
+//     staged in LDS with coalesced loads and read back by the groups: a load
+//     of col and val by each group would take as many address cycles as the
+//     gathers.  Groups past their row's end read a staged entry that points at
+//     Bt's row of zeros, so no product needs a select.
+//   - The unit of work is a slice of a row: 32 to 256 entries by the number of
+//     columns, counted from the row's start, so most rows are one.  A slice is
+//     summed by one group, and a row's slices are added in order: a
+//     row's sum depends on its own entries alone, not on the rows around it.
+//     Slices are dealt to the groups longest first (whole slices, then what
+//     remains of the rows in four classes of length), so that the groups of a
+//     wave end together.
+//   - The results pass through LDS and are written column by column.
+//   - Blocks are numbered so that an XCD takes `run` consecutive ones: rows
+//     that share columns then find B's rows in one L2 (the f64 mesh product
+//     below: 65 us with one block at a time per XCD, 60 us).
+// Measured against one row per wave (k > 32) and one entry per 2^i lanes
+// (k <= 32), both loading col and val from memory for every entry, in us per
+// product with B's copy: 27-point mesh of 262k rows, f64, k = 20: 297 -> 80,
+// f32, k = 64: 224 -> 124; 200k power-law rows of 14, f32, k = 100: 1380 -> 274
+// (segments of split rows included: 743 of the 1380); 8000 rows of 300, f32,
+// k = 20: 107 -> 34; 200k uniform rows of 16 (bound by the fabric), f64, k = 8:
+// 69 -> 63, k = 64: 291 -> 297.
+// 5 waves per SIMD at least, as many as the LDS of 5 blocks leaves (the f64 mesh
+// at k = 20: 71 us at 4).
+template <typename T, int VEC, int U, int ACC, bool BIG>
+__global__ __launch_bounds__(SPMM_BLOCK, 5) void csr_spmm_rows_kernel(
+    SpmmJob<T> ja, SpmmJob<T> jb, SpmmShape sh, int32_t origin, const int32_t *__restrict__ colind,
+    const T *__restrict__ val, const T *__restrict__ Bt0)
+{
     constexpr int NW = SPMM_BLOCK / 64;
-    __shared__ T s_c[SPMM_ROWS][KC + 1];
-    __shared__ int s_empty[SPMM_ROWS];
     using V = Vec<T, VEC>;
+    extern __shared__ __attribute__((aligned(16))) char s_mem[];
+    T *const s_val = reinterpret_cast<T *>(s_mem);                             // [ch + 1]
+    T *const s_c = s_val + sh.ch + 2;                                          // [rmax][cld]
+    T *const s_x = s_c + sh.rmax * sh.cld;                                     // [xmax][cld]
+    uint32_t *const s_off = reinterpret_cast<uint32_t *>(s_x + sh.xmax * sh.cld);   // [ch + 1]
+    __shared__ int s_task[SPMM_TASKS];
+
+    const bool second = blockIdx.x >= ja.blocks;
+    const SpmmJob<T> &j = second ? jb : ja;
+    unsigned lb = blockIdx.x - (second ? ja.blocks : 0u);
+    if (!second) {
+        const unsigned x = lb % NUM_XCD, i = lb / NUM_XCD;
+        lb = (i / j.run * NUM_XCD + x) * j.run + i % j.run;
+    }
+    const int64_t row0 = (int64_t)lb * j.R;
+    if (row0 >= j.rows) return;
+    const int nrows = (int)min((int64_t)j.R, j.rows - row0);
+    const int c0 = (int)blockIdx.y * sh.cols;
+    const int kk = (int)min((int64_t)sh.cols, sh.k - c0);
+    const T *const Bt = Bt0 + c0;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int64_t row0 = (int64_t)blockIdx.x * SPMM_ROWS;
-    const int nrows = (int)min((int64_t)SPMM_ROWS, m - row0);
+    const int L = sh.L, NG = 64 / L, NGB = NG * NW;
+    const int grp = lane / L, sub = lane - grp * L;
+    // The lane's first column; the last lanes of the last columns stay in Bt's row.
+    const int col = min(sub * VEC, (int)(sh.ldt - c0) - VEC);
+    const uint32_t colb = (uint32_t)(col * (int)sizeof(T));
 
-    for (int64_t c0 = 0; c0 < k; c0 += KC) {
-        const int64_t cl = c0 + (int64_t)lane * VEC;     // first column of this lane
-        const bool full = cl + VEC <= k;
-        for (int rr = wave; rr < nrows; rr += NW) {
-            const int64_t row = row0 + rr;
-            const int64_t lo = (int64_t)rowptr[row] - origin;
-            int64_t hi = (int64_t)(rowend ? rowend[row] : rowptr[row + 1]) - origin;
-            const bool skip = row_skip && row_skip[row];
-            if (skip) hi = lo;                 // a split row: its segments compute it
-            if (lane == 0 && c0 == 0) s_empty[rr] = skip ? 2 : hi <= lo;
-            T acc[VEC];
+    int lo = 0, hi = 0;
+    bool skip = false;
+    if (lane < nrows) {
+        lo = j.lo[row0 + lane] - origin;
+        hi = (j.hi ? j.hi[row0 + lane] : j.lo[row0 + lane + 1]) - origin;
+        skip = j.skip && j.skip[row0 + lane];
+        if (skip) lo = hi;
+    }
+    const bool empty = hi <= lo;
+    // A lane whose row is not followed by the next row's entries ends a run.
+    const int next = __shfl_down(lo, 1, 64);
+    const bool brk = lane == nrows - 1 || (lane < nrows && (next != hi || next < lo));
+    const bool whole = __popcll(__ballot(brk)) == 1;     // the rows' entries are one run
+    const int last = whole ? bcast_i(hi, nrows - 1) : wave_max(empty ? INT_MIN + 1 : hi);
+
+    const int ss = sh.slice_log2, S = 1 << ss;
+
+    // N steps of every group: entries p + s .. p + s + N - 1, those with s + u < n.
+    // ACC sums per column, entry u of a step into sum u mod ACC.
+    T acc[ACC][VEC];
+    auto steps = [&](auto N, int p, int s, int n) {
+        constexpr int NS = decltype(N)::value;
+        uint32_t off[NS];
+        T a[NS];
+        V b[NS];
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] = T(0);
-            for (int64_t p0 = lo; p0 < hi; p0 += 64) {
-                const int cnt = (int)min((int64_t)64, hi - p0);
-                int cidx = 0;
-                T cv = T(0);
-                if (lane < cnt) {
-                    cidx = colind[p0 + lane] - origin;
-                    cv = val[p0 + lane];
-                }
-                int q = 0;
-                for (; q + SPMM_UNROLL <= cnt; q += SPMM_UNROLL) {
-                    V b[SPMM_UNROLL];
-                    T a[SPMM_UNROLL];
+        for (int u = 0; u < NS; ++u) {
+            const int i = s + u < n ? p + s + u : sh.ch;
+            off[u] = s_off[i];
+            a[u] = s_val[i];
+        }
 #pragma unroll
-                    for (int u = 0; u < SPMM_UNROLL; ++u) {
-                        const int64_t j = bcast_i(cidx, q + u);
-                        a[u] = bcast(cv, q + u);
-                        if (full) {
-                            b[u] = *reinterpret_cast<const V *>(Bt + j * ldt + cl);
-                        } else {
+        for (int u = 0; u < NS; ++u) {
+            if (BIG)
+                b[u] = *reinterpret_cast<const V *>(Bt + (uint64_t)off[u] * (uint64_t)sh.ldt + col);
+            else
+                b[u] = *reinterpret_cast<const V *>(reinterpret_cast<const char *>(Bt) + (off[u] + colb));
+        }
 #pragma unroll
-                            for (int e = 0; e < VEC; ++e)
-                                b[u].v[e] = cl + e < k ? Bt[j * ldt + cl + e] : T(0);
-                        }
-                    }
+        for (int u = 0; u < NS; ++u)
 #pragma unroll
-                    for (int u = 0; u < SPMM_UNROLL; ++u)
+            for (int e = 0; e < VEC; ++e) acc[u % ACC][e] += a[u] * b[u].v[e];
+    };
+    auto row_sum = [&](int p, int n) {
+        int s = 0;
+        if (U == 8)
+            for (; __any(s + 4 < n); s += 8) steps(std::integral_constant<int, 8>(), p, s, n);
+        for (; __any(s + 2 < n); s += 4) steps(std::integral_constant<int, 4>(), p, s, n);
+        if (__any(s < n)) steps(std::integral_constant<int, 2>(), p, s, n);
+    };
+
+    int a = whole ? bcast_i(lo, 0) : wave_min(empty ? INT_MAX : lo);
+    while (a < last) {
+        // The next entries [a, b): from the first unfinished row on, no further
+        // than its run, the end of the rows and the buffer.
+        if (!whole) a = wave_min(!empty && hi > a ? max(lo, a) : INT_MAX);
+        if (a >= last) break;
+        int b = a + min(sh.ch, last - a);
+        if (!whole) b = min(b, wave_min(brk && hi > a ? hi : INT_MAX));
+        // The row that holds entry b is left before its start, or at the end of a slice.
+        const uint64_t left = __ballot(lo < b && b < hi);
+        if (left) {
+            const int to = hi - lo > S ? lo + ((b - lo) >> ss << ss) : lo;
+            b = max(bcast_i(max(to, max(lo, a)), __ffsll((unsigned long long)left) - 1), a + 1);
+        }
+        const int n = empty ? 0 : max(0, min(hi, b) - max(lo, a));
+        const int st = min(max(max(lo, a) - a, 0), sh.ch);
+
+        // The slices: full ones, the row's remainder, and those beyond the
+        // row's first, which have sums of their own until all are done.
+        const bool cont = lo < a;
+        const int full = n >> ss, rem = n & (S - 1);
+        const int more = n > 0 ? full + (rem > 0) - !cont : 0;
+        const uint64_t xrows = __ballot(more > 0);
+        int fbase = full, xbase = more, nfull = 0;
+        if (xrows || __any(full > 0)) {
 #pragma unroll
-                        for (int e = 0; e < VEC; ++e) acc[e] += a[u] * b[u].v[e];
-                }
-                for (; q < cnt; ++q) {
-                    const int64_t j = bcast_i(cidx, q);
-                    const T a = bcast(cv, q);
+            for (int off = 1; off < 64; off <<= 1) {
+                const int f = __shfl_up(fbase, off, 64), x = __shfl_up(xbase, off, 64);
+                fbase += lane >= off ? f : 0;
+                xbase += lane >= off ? x : 0;
+            }
+            nfull = bcast_i(fbase, 63);
+        }
+        fbase -= full;
+        xbase -= more;
+        int at = nfull, ntask = nfull;
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e)
-                        if (cl + e < k) acc[e] += a * Bt[j * ldt + cl + e];
+        for (int c = 3; c >= 0; --c) {
+            const uint64_t in = __ballot(rem > 0 && rem >> (ss - 2) == c);
+            if (rem >> (ss - 2) == c) at = ntask + __popcll(in & ((1ull << lane) - 1));
+            ntask += __popcll(in);
+        }
+        ntask = min(ntask, SPMM_TASKS);
+
+        __syncthreads();                       // the last entries are done with
+        // A slice is (first entry | entries | place of its sum: a row, or 64 + s_x's).
+        auto task = [&](int q, int i, int cnt) {
+            const int x = i - !cont;
+            const int place = x < 0 ? lane : 64 + min(xbase + x, sh.xmax - 1);
+            if (q < SPMM_TASKS) s_task[q] = (st + (i << ss)) | cnt << 11 | place << 20;
+        };
+        for (int i = wave; i < full; i += NW) task(fbase + i, i, S);
+        if (wave == 0 && rem > 0) task(at, full, rem);
+        for (int i = tid; i < b - a; i += SPMM_BLOCK) {
+            const uint32_t c = (uint32_t)(colind[a + i] - origin);
+            s_off[i] = BIG ? c : c * (uint32_t)(sh.ldt * sizeof(T));
+            s_val[i] = val[a + i];
+        }
+        if (tid == 0) {
+            s_off[sh.ch] = BIG ? (uint32_t)sh.zero_row : (uint32_t)(sh.zero_row * sh.ldt * sizeof(T));
+            s_val[sh.ch] = T(0);
+        }
+        __syncthreads();
+
+        int turn = 0;
+        for (int q0 = 0; q0 < ntask; q0 += NGB, ++turn) {
+            const int q = q0 + (turn & 1 ? NW - 1 - wave : wave) * NG + grp;
+            const int t = grp < NG && q < ntask ? s_task[q] : 0;
+            const int cnt = t >> 11 & 511;
+#pragma unroll
+            for (int h = 0; h < ACC; ++h)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) acc[h][e] = T(0);
+            row_sum(t & 2047, cnt);
+            // s_x follows s_c, rmax rows on.
+            const int place = t >> 20;
+            T *const dst = s_c + (place < 64 ? place : place - 64 + sh.rmax) * sh.cld + sub * VEC;
+            if (cnt > 0) {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    T v = acc[0][e] + acc[1][e];
+                    if (ACC == 4) v += acc[ACC - 2][e] + acc[ACC - 1][e];
+                    dst[e] = v;
                 }
             }
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) s_c[rr][lane * VEC + e] = acc[e];
         }
-        __syncthreads();
-        // Column-major write-out: SPMM_ROWS consecutive rows per column.
-        const int ncols = (int)min((int64_t)KC, k - c0);
-        for (int idx = tid; idx < SPMM_ROWS * ncols; idx += SPMM_BLOCK) {
-            const int rr = idx % SPMM_ROWS;
-            const int cc = idx / SPMM_ROWS;
-            if (rr >= nrows) continue;
-            if (s_empty[rr] == 2 || (skip_empty_rows && s_empty[rr])) continue;
-            T *dst = C + (row0 + rr) + (c0 + cc) * ldc;
-            const T s = alpha * s_c[rr][cc];
-            *dst = beta_zero ? s : s + beta * *dst;
+        if (xrows) {
+            __syncthreads();
+            uint64_t left_rows = xrows;
+            for (int i = 0; left_rows; ++i, left_rows &= left_rows - 1) {
+                if ((i & (NW - 1)) != wave) continue;
+                const int r = __ffsll((unsigned long long)left_rows) - 1;
+                const int x0 = bcast_i(xbase, r), cnt = min(bcast_i(more, r), sh.xmax - x0);
+                for (int c = lane; c < kk; c += 64) {
+                    T v = s_c[r * sh.cld + c];
+                    for (int h = 0; h < cnt; ++h) v += s_x[(x0 + h) * sh.cld + c];
+                    s_c[r * sh.cld + c] = v;
+                }
+            }
         }
-        __syncthreads();
+        a = b;
+    }
+    __syncthreads();
+    if (lane >= nrows || skip || (j.skip_empty_rows && empty)) return;
+    for (int c = wave; c < kk; c += NW) {
+        T *const dst = j.C + (row0 + lane) + (c0 + c) * j.ldc;
+        const T v = j.alpha * (empty ? T(0) : s_c[lane * sh.cld + c]);
+        *dst = j.beta_zero ? v : v + j.beta * *dst;
     }
 }
 
@@ -256,15 +428,6 @@ __global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_kernel(
 // the 256 MB MALL, else the widest multiple of 16 columns that does (at least
 // 16).  JLUST_HIP_SPMM_KCHUNK=c forces c columns per pass.
 constexpr size_t SPMM_MALL_BUDGET = (size_t)256 << 20;
-
-bool spmm_group()
-{
-    static const bool on = [] {
-        const char *e = getenv("JLUST_HIP_SPMM_GROUP");
-        return !(e && e[0] == '0');
-    }();
-    return on;
-}
 
 int64_t spmm_kchunk(int64_t n, int64_t k, size_t tsz)
 {
@@ -281,12 +444,11 @@ int64_t spmm_kchunk(int64_t n, int64_t k, size_t tsz)
 }
 
 // Long rows of a prepared plan: a row with more than SPMM_LONG_ROW entries
-// is cut into segments of SPMM_SEG entries, each a wave's work in the same
-// kernels (rowptr = segment starts, rowend = segment ends) writing one partial
-// row into the plan's workspace; spmm_long_reduce_kernel adds a row's
-// partials in segment order.  A wave otherwise walks a whole row alone, so a
-// 10^5-entry row of a power-law matrix would keep one wave busy for the whole
-// product.
+// is cut into segments of SPMM_SEG entries, each a row of its own in the same
+// launch (blocks after the rows') writing one partial row into the plan's
+// workspace; spmm_long_reduce_kernel adds a row's partials in segment order.
+// A block otherwise walks a whole row alone, so a 10^5-entry row of a power-law
+// matrix would keep one block busy long after the others.
 constexpr int64_t SPMM_LONG_ROW = 1024;
 constexpr int64_t SPMM_SEG = 256;
 
@@ -310,22 +472,46 @@ __global__ void spmm_long_reduce_kernel(int64_t nlong, int64_t kk, const int32_t
     *dst = beta_zero ? v : v + beta * *dst;
 }
 
-// How one column chunk of kk columns is computed: the group kernel (kk <= 32)
-// or the wide kernel; the group kernel's B copy is unpadded, the wide one's
-// rows padded to 16 bytes; one column gathers from B's own column.
+// How one column chunk of kk columns is computed: VEC columns per lane of the
+// rows kernel and the row stride of B's copy (whole vectors), or one column
+// from B itself.
+//   - 16 bytes per lane where L1 and L2 serve the gathers: half the loads of
+//     8 bytes (27-point mesh, k = 64: f32 105 against 146 us, f64 249 against
+//     321 us).
+//   - Fewer columns per lane below 13 (f32) and 5 (f64) of them, so that the
+//     block's groups do not outnumber the 64 rows its lanes hold (200k
+//     power-law rows, f32, k = 8: 71 us, 87 with 4 columns per lane; f64, k = 4
+//     likewise).
+//   - 8 bytes per lane for wide f32 chunks of a copy past 128 MB, where random
+//     rows come from the MALL: a wave's load then spans half as many rows
+//     (1M uniform rows of 32, 64 columns: 1.135 against 1.160 ms; a mesh would
+//     rather have 16).  f64 keeps 16: the mesh loses more than random rows
+//     gain (262k rows, k = 128: 519 -> 680 us; 200k uniform rows of 16: 585 ->
+//     567 us).
 struct SpmmChunk {
-    bool group;
     bool direct;
+    int vec;
     int64_t ldt;
 };
 
-SpmmChunk spmm_chunk_kind(int64_t kk)
+template <typename T>
+SpmmChunk spmm_chunk_kind(int64_t n, int64_t kk)
 {
+    constexpr int W16 = 16 / sizeof(T), W8 = 8 / sizeof(T);
     SpmmChunk c;
-    c.group = kk <= 32 && spmm_group();
-    c.direct = c.group && kk == 1;
-    c.ldt = c.group ? kk : (kk + 3) / 4 * 4;
+    c.direct = kk == 1;
+    c.vec = W16;
+    if (sizeof(T) == 4 && kk >= 48 && n * kk * 4 > (int64_t)128 << 20) c.vec = W8;
+    if (kk <= 12 && sizeof(T) == 4) c.vec = W8;
+    if (kk <= 4) c.vec = 1;
+    c.ldt = (kk + c.vec - 1) / c.vec * c.vec;
     return c;
+}
+
+// Elements of the row-major copy of a pass of at most kc of k columns.
+int64_t spmm_copy_elems(int64_t n, int64_t kc, int64_t k)
+{
+    return (n + 1) * ((min(kc, k > 0 ? k : 1) + 3) / 4 * 4);
 }
 
 // Row-major copy of columns [c0, c0+kk) of B into Bt (skipped when direct).
@@ -333,59 +519,141 @@ template <typename T>
 int spmm_copy_chunk(int64_t n, int64_t kk, const T *B, int64_t ldb, const SpmmChunk &ck, T *Bt, hipStream_t s)
 {
     if (n == 0 || ck.direct) return JLUST_STATUS_SUCCESS;
-    dim3 tgrid((unsigned)((n + 63) / 64), (unsigned)((kk + 63) / 64));
-    hipLaunchKernelGGL((transpose_kernel<T>), tgrid, dim3(256), 0, s, n, kk, B, ldb, Bt, ck.ldt);
+#define JLUST_TRANSPOSE(V, CT)                                                                             \
+    hipLaunchKernelGGL((transpose_kernel<T, V, CT>),                                                       \
+                       dim3((unsigned)(n / (4096 / CT) + 1), (unsigned)((kk + CT - 1) / CT)), dim3(256), 0, \
+                       s, n, kk, B, ldb, Bt, ck.ldt)
+#define JLUST_TRANSPOSE_CT(V)                \
+    do {                                     \
+        if (kk <= 16) JLUST_TRANSPOSE(V, 16); \
+        else if (kk <= 32) JLUST_TRANSPOSE(V, 32); \
+        else JLUST_TRANSPOSE(V, 64);         \
+    } while (0)
+    if (ck.vec == 1) JLUST_TRANSPOSE_CT(1);
+    else if (ck.vec == 2) JLUST_TRANSPOSE_CT(2);
+    else JLUST_TRANSPOSE_CT((16 / (int)sizeof(T)));
+#undef JLUST_TRANSPOSE_CT
+#undef JLUST_TRANSPOSE
     return check_launch("transpose_kernel");
 }
 
-// The product of one chunk over m rows (rows of A, or segments when rowend is
-// given): C[:, 0:kk] (ldc) = alpha * A[rows, :] * Bsrc + beta * C, rows
-// flagged in row_skip left untouched.  nnz_rows: the entries these rows hold
-// (for the group kernel's steps per load).
+// Rows per block of the rows kernel for `rows` rows of `mean` entries.  A round
+// gives each of the block's ngb groups one slice; as many rounds as 64 lanes
+// hold rows, fewer where the result tile would pass 9 KB (8 blocks per CU want
+// 20 KB each; columns of C still get whole 128-byte lines), where the staged
+// entries would not fit and where the rows would not make 1024 blocks.
 template <typename T>
-int spmm_chunk_launch(int64_t m, int64_t kk, int64_t nnz_rows, int32_t origin, const int32_t *rowptr,
-                      const int32_t *rowend, const uint8_t *row_skip, const int32_t *colind, const T *val,
-                      const T *Bsrc, const SpmmChunk &ck, T alpha, T beta, T *Cc, int64_t ldc,
-                      int skip_empty_rows, hipStream_t s)
+int spmm_rows_per_block(int64_t rows, int64_t mean, int ngb, int slice_log2, int cld)
+{
+    const int64_t slices = ((mean - 1) >> slice_log2) + 1;
+    const int64_t step = min(max(ngb / slices, (int64_t)1), (int64_t)64), line = 128 / sizeof(T);
+    int64_t r = 64 / step * step;
+    while (r > step && r - step >= line && r * cld * (int64_t)sizeof(T) > (9 << 10)) r -= step;
+    while (r > step && (r * mean > 1800 || rows / r < 1024)) r -= step;
+    return (int)r;
+}
+
+template <typename T, int VEC>
+int spmm_rows_launch(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, int32_t origin, SpmmJob<T> ja,
+                     SpmmJob<T> jb, const int32_t *colind, const T *val, const T *Bt, int64_t ldt, hipStream_t s)
+{
+    const int64_t ny = (kk + 64 * VEC - 1) / (64 * VEC);
+    SpmmShape sh;
+    sh.k = kk;
+    sh.ldt = ldt;
+    sh.zero_row = n;
+    sh.cols = (int)(((kk + ny - 1) / ny + VEC - 1) / VEC * VEC);
+    sh.L = sh.cols / VEC;
+    sh.cld = sh.cols | 1;
+    const int ngb = 64 / sh.L * (SPMM_BLOCK / 64);
+    sh.slice_log2 = sh.L <= 8 ? 5 : sh.L <= 16 ? 6 : sh.L <= 32 ? 7 : 8;
+    const int64_t mean_a = ja.rows ? nnz_rows / ja.rows + 1 : 1, mean_b = jb.rows ? nnz_seg / jb.rows + 1 : 1;
+    ja.R = spmm_rows_per_block<T>(ja.rows, mean_a, ngb, sh.slice_log2, sh.cld);
+    jb.R = spmm_rows_per_block<T>(jb.rows, mean_b, ngb, sh.slice_log2, sh.cld);
+    const int64_t nb = (ja.rows + ja.R - 1) / ja.R;
+    ja.run = (unsigned)((nb + 4 * NUM_XCD - 1) / (4 * NUM_XCD));
+    if (ja.run == 0) ja.run = 1;
+    ja.blocks = (unsigned)((nb + ja.run * NUM_XCD - 1) / (ja.run * NUM_XCD) * (ja.run * NUM_XCD));
+    jb.blocks = (unsigned)((jb.rows + jb.R - 1) / jb.R);
+    sh.rmax = max(ja.R, jb.rows ? jb.R : 1);
+    const int64_t want = max(ja.R * mean_a * 9 / 8, jb.rows ? jb.R * mean_b : 0) + 32;
+    sh.ch = (int)min(max(want, ((int64_t)1 << sh.slice_log2) + 32), (int64_t)SPMM_STAGE);
+    sh.xmax = (sh.ch >> sh.slice_log2) + 2;
+    const size_t lds = sizeof(T) * (size_t)(sh.ch + 2 + (sh.rmax + sh.xmax) * sh.cld) + 4 * (size_t)(sh.ch + 1);
+    const dim3 grid(ja.blocks + jb.blocks, (unsigned)ny);
+    // 8 entries in flight per group for long f64 rows (27-point mesh, k = 128:
+    // 558 -> 523 us), else 4: short rows would load past their ends (1M
+    // power-law rows of 5, f64, k = 64: 827 -> 752 us), and f32 gains nothing.
+    // Four sums per column up to 16 columns, else two: as many roundings in a
+    // chain as the kernels before had or fewer (27 entries, f32: 6.2e-8 relative
+    // error with four, 7.2e-8 with two, 9.4e-8 with one; four cost the f64 mesh
+    // at k = 20 8 % in registers).
+#define JLUST_ROWS(U, ACC, BIG)                                                                               \
+    hipLaunchKernelGGL((csr_spmm_rows_kernel<T, VEC, U, ACC, BIG>), grid, dim3(SPMM_BLOCK), lds, s, ja, jb, sh, \
+                       origin, colind, val, Bt)
+    const bool deep = sizeof(T) == 8 && mean_a > 20, wide = kk > 16;
+    if ((uint64_t)(n + 1) * (uint64_t)ldt * sizeof(T) > 0xffffff00ull) JLUST_ROWS(4, 4, true);
+    else if (deep && wide) JLUST_ROWS(8, 2, false);
+    else if (deep) JLUST_ROWS(8, 4, false);
+    else if (wide) JLUST_ROWS(4, 2, false);
+    else JLUST_ROWS(4, 4, false);
+#undef JLUST_ROWS
+    return check_launch("csr_spmm_rows_kernel");
+}
+
+template <typename T>
+int spmm_rows_pass(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, int32_t origin, const SpmmJob<T> &ja,
+                   const SpmmJob<T> &jb, const int32_t *colind, const T *val, const T *Bt, const SpmmChunk &ck,
+                   hipStream_t s)
+{
+    auto run = [&](auto V) {
+        return spmm_rows_launch<T, decltype(V)::value>(n, kk, nnz_rows, nnz_seg, origin, ja, jb, colind, val, Bt,
+                                                       ck.ldt, s);
+    };
+    if (ck.vec == 1) return run(std::integral_constant<int, 1>());
+    if (ck.vec == 2) return run(std::integral_constant<int, 2>());
+    return run(std::integral_constant<int, 16 / sizeof(T)>());
+}
+
+// The product of one column over m rows (rows of A, or segments when rowend
+// is given): C = alpha * A[rows, :] * B + beta * C, rows flagged in row_skip
+// left untouched.  nnz_rows: the entries these rows hold.
+template <typename T>
+int spmm_col_launch(int64_t m, int64_t nnz_rows, int32_t origin, const int32_t *rowptr, const int32_t *rowend,
+                    const uint8_t *row_skip, const int32_t *colind, const T *val, const T *B, T alpha, T beta, T *C,
+                    int skip_empty_rows, hipStream_t s)
 {
     if (m == 0) return JLUST_STATUS_SUCCESS;
     const dim3 grid((unsigned)((m + SPMM_ROWS - 1) / SPMM_ROWS));
     const int bz = beta == T(0);
-    const int64_t ldt = ck.ldt;
-    const int vec = (sizeof(T) == 4) ? (kk <= 64 ? 1 : kk <= 128 ? 2 : 4) : (kk <= 64 ? 1 : 2);
-#define JLUST_GROUP_U(KV, U)                                                                           \
-    hipLaunchKernelGGL((csr_spmm_group_kernel<T, KV, U>), grid, dim3(SPMM_BLOCK), 0, s, m, kk, origin,    \
-                       rowptr, colind, val, Bsrc, ldt, alpha, beta, bz, Cc, ldc, skip_empty_rows, rowend, \
-                       row_skip)
-#define JLUST_GROUP(KV)                                                                                \
-    do {                                                                                               \
-        const int64_t steps = (nnz_rows + m * (64 / KV) - 1) / (m * (64 / KV));  /* per row */          \
-        if (steps <= 1) JLUST_GROUP_U(KV, 1);                                                          \
-        else if (steps <= 2) JLUST_GROUP_U(KV, 2);                                                     \
-        else if (steps <= 4) JLUST_GROUP_U(KV, 4);                                                     \
-        else JLUST_GROUP_U(KV, 8);                                                                     \
-    } while (0)
-#define JLUST_WIDE(V)                                                                                  \
-    hipLaunchKernelGGL((csr_spmm_kernel<T, V>), grid, dim3(SPMM_BLOCK), 0, s, m, kk, origin, rowptr,      \
-                       colind, val, Bsrc, ldt, alpha, beta, bz, Cc, ldc, skip_empty_rows, rowend, row_skip)
-    if (ck.group) {
-        if (kk == 1) JLUST_GROUP(1);
-        else if (kk == 2) JLUST_GROUP(2);
-        else if (kk <= 4) JLUST_GROUP(4);
-        else if (kk <= 8) JLUST_GROUP(8);
-        else if (kk <= 16) JLUST_GROUP(16);
-        else JLUST_GROUP(32);
-    } else if (vec == 1) {
-        JLUST_WIDE(1);
-    } else if (vec == 2) {
-        JLUST_WIDE(2);
-    } else {
-        JLUST_WIDE(4);
+    const int64_t steps = (nnz_rows + m * 64 - 1) / (m * 64);     // per row
+#define JLUST_COL(U)                                                                                        \
+    hipLaunchKernelGGL((csr_spmm_col_kernel<T, U>), grid, dim3(SPMM_BLOCK), 0, s, m, origin, rowptr, rowend, \
+                       row_skip, colind, val, B, alpha, beta, bz, C, skip_empty_rows)
+    if (steps <= 1) JLUST_COL(1);
+    else if (steps <= 2) JLUST_COL(2);
+    else if (steps <= 4) JLUST_COL(4);
+    else JLUST_COL(8);
+#undef JLUST_COL
+    return check_launch("csr_spmm_col_kernel");
+}
+
+// One column chunk over the rows of ja and the segments of jb.
+template <typename T>
+int spmm_chunk(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, int32_t origin, const SpmmJob<T> &ja,
+               const SpmmJob<T> &jb, const int32_t *colind, const T *val, const T *B, int64_t ldb, T *Bt,
+               hipStream_t s)
+{
+    const SpmmChunk ck = spmm_chunk_kind<T>(n, kk);
+    if (ck.direct) {
+        for (const SpmmJob<T> *j : {&ja, &jb})
+            if (int st = spmm_col_launch<T>(j->rows, j == &ja ? nnz_rows : nnz_seg, origin, j->lo, j->hi, j->skip,
+                                            colind, val, B, j->alpha, j->beta, j->C, j->skip_empty_rows, s))
+                return st;
+        return JLUST_STATUS_SUCCESS;
     }
-#undef JLUST_WIDE
-#undef JLUST_GROUP
-#undef JLUST_GROUP_U
-    return check_launch(ck.group ? "csr_spmm_group_kernel" : "csr_spmm_kernel");
+    if (int st = spmm_copy_chunk<T>(n, kk, B, ldb, ck, Bt, s)) return st;
+    return spmm_rows_pass<T>(n, kk, nnz_rows, nnz_seg, origin, ja, jb, colind, val, Bt, ck, s);
 }
 
 int check_spmm_args(const char *who, int64_t m, int64_t n, int64_t k, int64_t nnz, int32_t origin,
@@ -430,18 +698,21 @@ int csr_spmm(int64_t m, int64_t n, int64_t k, int64_t nnz, int32_t origin,
     // gathers come from HBM, so B is processed in column chunks whose copy
     // fits (config 3: 2 chunks of 64 columns, 3.14 -> 2.56 ms).
     const int64_t kc = spmm_kchunk(n, k, sizeof(T));
-    const int64_t ldt_max = (min(kc, k) + 3) / 4 * 4;    // keeps every row of Bt 16-byte aligned
     void *ws = nullptr;
-    const int64_t nt = n > 0 ? n : 1;
-    if (int st = scratch(stream, sizeof(T) * (size_t)(nt * ldt_max), &ws)) return st;
+    if (int st = scratch(stream, sizeof(T) * (size_t)spmm_copy_elems(n, kc, k), &ws)) return st;
     T *Bt = (T *)ws;
+    SpmmJob<T> rows;
+    rows.rows = m;
+    rows.lo = rowptr;
+    rows.alpha = alpha;
+    rows.beta = beta;
+    rows.beta_zero = beta == T(0);
+    rows.ldc = ldc;
+    rows.skip_empty_rows = skip_empty_rows;
     for (int64_t c0 = 0; c0 < k; c0 += kc) {
-        const int64_t kk = min(kc, k - c0);
-        const SpmmChunk ck = spmm_chunk_kind(kk);
-        if (int st = spmm_copy_chunk<T>(n, kk, B + c0 * ldb, ldb, ck, Bt, s)) return st;
-        const T *Bsrc = ck.direct ? B + c0 * ldb : Bt;
-        if (int st = spmm_chunk_launch<T>(m, kk, nnz, origin, rowptr, nullptr, nullptr, colind, val, Bsrc, ck,
-                                          alpha, beta, C + c0 * ldc, ldc, skip_empty_rows, s))
+        rows.C = C + c0 * ldc;
+        if (int st = spmm_chunk<T>(n, min(kc, k - c0), nnz, 0, origin, rows, SpmmJob<T>(), colind, val, B + c0 * ldb,
+                                   ldb, Bt, s))
             return st;
     }
     return JLUST_STATUS_SUCCESS;
@@ -580,8 +851,7 @@ static int csr_spmm_plan_create_body(int64_t m, int64_t n, int64_t k, int64_t nn
     for (int32_t r : long_rows) skip[(size_t)r] = 1;
 
     // One allocation: B copy, row flags, segment tables, partial rows.
-    const int64_t ldt_max = (min(p->kc, k > 0 ? k : 1) + 3) / 4 * 4;
-    const size_t sz_bt = align_up(tsz * (size_t)(n > 0 ? n : 1) * (size_t)ldt_max, 256);
+    const size_t sz_bt = align_up(tsz * (size_t)spmm_copy_elems(n, p->kc, k), 256);
     const size_t sz_skip = p->nlong ? align_up((size_t)m, 256) : 0;
     const size_t sz_lr = align_up(sizeof(int32_t) * (size_t)(p->nlong + 1), 256);
     const size_t sz_sg = align_up(sizeof(int32_t) * (size_t)(p->nseg > 0 ? p->nseg : 1), 256);
@@ -671,19 +941,28 @@ static int spmm_plan_execute(jlust_spmm_plan_t p, int want_type, T alpha, const 
     T *Bt = (T *)p->Bt;
     T *part = (T *)p->part;
     const int bz = beta == T(0);
+    SpmmJob<T> rows, segs;
+    rows.rows = p->m;
+    rows.lo = p->rowptr;
+    rows.skip = p->row_skip;
+    rows.alpha = alpha;
+    rows.beta = beta;
+    rows.beta_zero = bz;
+    rows.ldc = ldc;
+    rows.skip_empty_rows = skip_empty_rows;
+    segs.rows = p->nseg;
+    segs.lo = p->seg_lo;
+    segs.hi = p->seg_hi;
+    segs.alpha = T(1);
+    segs.C = part;
+    segs.ldc = p->nseg;
     for (int64_t c0 = 0; c0 < p->k; c0 += p->kc) {
         const int64_t kk = min(p->kc, p->k - c0);
-        const SpmmChunk ck = spmm_chunk_kind(kk);
-        if (int st = spmm_copy_chunk<T>(p->n, kk, B + c0 * ldb, ldb, ck, Bt, s)) return st;
-        const T *Bsrc = ck.direct ? B + c0 * ldb : Bt;
-        if (int st = spmm_chunk_launch<T>(p->m, kk, p->nnz_rows, p->origin, p->rowptr, nullptr, p->row_skip,
-                                          p->colind, val, Bsrc, ck, alpha, beta, C + c0 * ldc, ldc,
-                                          skip_empty_rows, s))
+        rows.C = C + c0 * ldc;
+        if (int st = spmm_chunk<T>(p->n, kk, p->nnz_rows, p->nnz - p->nnz_rows, p->origin, rows, segs, p->colind, val,
+                                   B + c0 * ldb, ldb, Bt, s))
             return st;
         if (p->nseg == 0) continue;
-        if (int st = spmm_chunk_launch<T>(p->nseg, kk, p->nnz - p->nnz_rows, p->origin, p->seg_lo, p->seg_hi,
-                                          nullptr, p->colind, val, Bsrc, ck, T(1), T(0), part, p->nseg, 0, s))
-            return st;
         const int64_t t = p->nlong * kk;
         hipLaunchKernelGGL((spmm_long_reduce_kernel<T>), dim3((unsigned)((t + 255) / 256)), dim3(256), 0, s,
                            p->nlong, kk, p->long_rows, p->seg_first, part, p->nseg, alpha, beta, bz,
@@ -738,7 +1017,7 @@ extern "C" int jlust_hip_csr_spmm_plan_destroy(jlust_spmm_plan_t plan)
 namespace jlust {
 int preload_spmm()
 {
-    JLUST_PRELOAD_KERNEL(transpose_kernel<float>);
+    JLUST_PRELOAD_KERNEL((transpose_kernel<float, 4, 64>));
     return JLUST_STATUS_SUCCESS;
 }
 }  // namespace jlust

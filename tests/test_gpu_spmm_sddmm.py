@@ -66,6 +66,66 @@ def test_spmm_random(J, O, k, dtype):
     assert_within(C, ref, absref, dtype, f"k={k} ({strat})")
 
 
+def _rows_kernel_lengths(shape, m, rng):
+    if shape == "even":
+        return np.full(m, 9)
+    if shape == "sparse":                      # mostly empty rows, empty first and last blocks
+        lens = np.where(rng.random(m) < 0.1, rng.integers(1, 5, m), 0)
+        lens[:70] = lens[-70:] = 0
+        return lens
+    lens = rng.integers(0, 12, m)              # "uneven": rows past a group's share, past the
+    lens[[0, m // 3, m // 2]] = 90, 700, 5000  # staged entries, and past a plan's split
+    return lens
+
+
+@pytest.mark.parametrize("call", ["plain", "plan"])
+@pytest.mark.parametrize("shape,m", [("even", 1), ("even", 63), ("even", 64), ("even", 65), ("even", 4099),
+                                     ("sparse", 900), ("uneven", 300), ("uneven", 4099)])
+@pytest.mark.parametrize("k", [2, 4, 5, 12, 13, 17, 20, 100, 129, 260])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_spmm_rows_kernel_edges(J, O, dtype, k, shape, m, call):
+    """Blocks and groups of rows at their edges, rows cut by the staged
+    entries and into slices, empty and split rows; a B row that is not finite
+    reaches only the rows that hold its column."""
+    rng = np.random.default_rng(m + k)
+    n = 6000
+    rowptr, colind, val = random_csr(m, n - 1, lengths=_rows_kernel_lengths(shape, m, rng), seed=m, dtype=dtype)
+    B = np.asfortranarray(rng.standard_normal((n, k)).astype(dtype))
+    bad = int(colind[-1]) - 1 if colind.size else 0
+    Bbad = B.copy(order="F")
+    Bbad[bad], Bbad[n - 1] = np.inf, np.nan    # column n is in no row
+    ref, _ = O.csr_spmm(rowptr, colind, val, B)
+    absref = O.csr_spmm_absref(rowptr, colind, val, B)
+    rows = np.repeat(np.arange(m), np.diff(rowptr))
+    hit = np.zeros(m, bool)
+    hit[rows[colind == bad + 1]] = True
+    if call == "plain":
+        C, Cbad = (run_spmm(J, rowptr, colind, val, b, m, n) for b in (B, Bbad))
+    else:
+        A = J.csr_tensor(dev(rowptr), dev(colind), dev(val), (m, n))
+        h = J.prepare(J.HIPBackend(), J.SpMMOp, A, n_cols=k)
+        assert h.info()["split_rows"] == int((np.diff(rowptr) > 1024).sum())
+        C, Cbad = (host(J.execute(h, dev(b), J.dense_matrix(m, k, dtype=A.dtype, fill=float("nan"))).val)
+                   for b in (B, Bbad))
+    assert_within(C, ref, absref, dtype, f"{shape} m={m} k={k}")
+    np.testing.assert_array_equal(Cbad[~hit], C[~hit])
+    assert not np.isfinite(Cbad[hit]).any()
+
+
+def test_spmm_copy_beyond_32_bit_offsets(J):
+    """B's row-major copy past 4 GiB: rows are addressed in 64 bits."""
+    import torch
+    n, k, m = 34_000_000, 16, 200
+    B = torch.randn((k, n), dtype=torch.float64, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).t()
+    cols = torch.linspace(0, n - 1, m * 3, dtype=torch.float64).long().view(m, 3).cuda()
+    val = torch.randn(m * 3, dtype=torch.float64, device="cuda")
+    A = J.csr_tensor(torch.arange(0, 3 * m + 1, 3, dtype=torch.int32, device="cuda") + 1, cols.view(-1).int() + 1,
+                     val, (m, n))
+    C = J.matmul(A, B)
+    ref = (val.view(m, 3, 1) * B[cols]).sum(1)
+    assert (C - ref).abs().max() <= 1e-12 * (val.view(m, 3, 1).abs() * B[cols].abs()).sum(1).max()
+
+
 @pytest.mark.parametrize("alpha,beta", [(2.0, 0.0), (0.5, -1.5)])
 def test_spmm_alpha_beta_zero_based(J, O, alpha, beta):
     m, n, k = 1000, 1500, 128
