@@ -918,6 +918,23 @@ int jlust_hip_convert_analyze(const jlust_sparse *src, int32_t dst_format,
                               jlust_stream_t stream, jlust_convert_t *out,
                               int64_t *dst_nnz, int64_t *dst_nouter);
 
+/* The same analysis in the caller's device memory: jlust_hip_convert_workspace
+ * reports the bytes it takes, jlust_hip_convert_analyze_ws runs in ws (256-byte
+ * aligned, at least that many bytes), which the handle keeps pointers into:
+ * ws must stay valid until the last fill with it has run.  A program that
+ * converts often allocates ws from a pool of its own instead of paying a
+ * device allocation and release per conversion. */
+int jlust_hip_convert_workspace(const jlust_sparse *src, int32_t dst_format,
+                                int32_t dst_b1, int32_t dst_b2,
+                                int32_t dst_row_major_blocks, int value_type,
+                                int64_t *bytes);
+int jlust_hip_convert_analyze_ws(const jlust_sparse *src, int32_t dst_format,
+                                 int32_t dst_b1, int32_t dst_b2,
+                                 int32_t dst_row_major_blocks, int value_type,
+                                 void *ws, int64_t ws_bytes,
+                                 jlust_stream_t stream, jlust_convert_t *out,
+                                 int64_t *dst_nnz, int64_t *dst_nouter);
+
 /* Step 2: writes the target's buffers (caller-allocated with the sizes from
  * analyze; origin, extents and format equal to the source's and the analysed
  * target), stream-ordered. */

@@ -20,6 +20,7 @@
 //
 // Also: sparse_to_dense (ext/KernelAbstractionsExt/ops/conversion.jl:47-65)
 // and the index shift of materialize's origin change (CUDAExt.jl:199-220).
+#include <algorithm>
 #include <cstring>
 
 #include <hip/hip_runtime.h>
@@ -343,9 +344,34 @@ KeyLayout layout_for(int fmt, int64_t m, int64_t n, int b1, int b2, int row_majo
     return L;
 }
 
-// Segment id per position for CSR/CSC/DCSR (per value) and BSR (per block).
-int segments(const jlust_sparse *s, int32_t *seg, int64_t &len, void *&tmp, size_t &tmp_bytes,
-             hipStream_t st)
+int64_t segment_positions(const jlust_sparse *s)
+{
+    return s->format == JLUST_FORMAT_BSR ? s->nouter : s->nnz;
+}
+
+// The scans' and the sort's temporary storage over n items.
+int scan_bytes(int64_t n, size_t *need)
+{
+    int32_t *v = nullptr;
+    size_t a = 0, b = 0, c = 0;
+    JLUST_HIP_TRY(rocprim::inclusive_scan(nullptr, a, v, v, (size_t)n, rocprim::maximum<int32_t>(), (hipStream_t)0));
+    JLUST_HIP_TRY(rocprim::exclusive_scan(nullptr, b, v, v, 0, (size_t)n, rocprim::plus<int32_t>(), (hipStream_t)0));
+    JLUST_HIP_TRY(rocprim::inclusive_scan(nullptr, c, v, v, (size_t)n, rocprim::plus<int32_t>(), (hipStream_t)0));
+    *need = std::max(a, std::max(b, c));
+    return JLUST_STATUS_SUCCESS;
+}
+
+int sort_bytes(int64_t n, int begin_bit, int end_bit, size_t *need)
+{
+    uint64_t *k = nullptr;
+    int32_t *v = nullptr;
+    JLUST_HIP_TRY(rocprim::radix_sort_pairs(nullptr, *need, k, k, v, v, (size_t)n, begin_bit, end_bit, (hipStream_t)0));
+    return JLUST_STATUS_SUCCESS;
+}
+
+// Segment id per position for CSR/CSC/DCSR (per value) and BSR (per block);
+// tmp: scan_bytes of the positions.
+int segments(const jlust_sparse *s, int32_t *seg, int64_t &len, void *tmp, hipStream_t st)
 {
     int64_t nseg = 0;
     len = s->nnz;
@@ -369,12 +395,6 @@ int segments(const jlust_sparse *s, int32_t *seg, int64_t &len, void *&tmp, size
     size_t need = 0;
     JLUST_HIP_TRY(rocprim::inclusive_scan(nullptr, need, seg, seg, (size_t)len,
                                           rocprim::maximum<int32_t>(), st));
-    if (need > tmp_bytes) {
-        if (tmp) JLUST_HIP_TRY(hipFree(tmp));
-        tmp = nullptr;
-        JLUST_HIP_TRY(hipMalloc(&tmp, need));
-        tmp_bytes = need;
-    }
     JLUST_HIP_TRY(rocprim::inclusive_scan(tmp, need, seg, seg, (size_t)len,
                                           rocprim::maximum<int32_t>(), st));
     return JLUST_STATUS_SUCCESS;
@@ -392,7 +412,9 @@ struct jlust_convert {
     int64_t count = 0;          // entries after drop + dedup
     int64_t nruns = 0;          // DCSR rows / BSR blocks
     const void *src_val = nullptr;
-    void *mem = nullptr;        // the analysis workspace: keys, pos, head and run point into it
+    void *mem = nullptr;        // the analysis workspace if the handle owns it: keys, pos, head, run
+                                // and spare point into it
+    uint64_t *spare = nullptr;  // a buffer of as many words as there are stored values, free after analyse
     uint64_t *keys = nullptr;
     int32_t *pos = nullptr, *head = nullptr, *run = nullptr;   // pos null: the identity
 };
@@ -404,52 +426,74 @@ struct Workspace {
     ~Workspace() { if (p) (void)hipFree(p); }
 };
 
+// The bits an entry's key is sorted by: [begin, end), empty where target and
+// source share the identity ordering (convert.jl:331-349).  A source whose
+// segments run in the order of the target's minor coordinate (CSR rows to a
+// CSC target, CSC columns to a row-major one) holds equal majors in ascending
+// minor order already, so the stable sort need only order the major bits.
+bool sort_bits(const jlust_sparse *src, int dst_format, const KeyLayout &L, int *begin_bit, int *end_bit)
+{
+    if (dst_identity(dst_format) && src_ordered_identity(src->format)) return false;
+    const bool major_only = (src->format == JLUST_FORMAT_CSR && dst_format == JLUST_FORMAT_CSC) ||
+                            (src->format == JLUST_FORMAT_CSC && dst_identity(dst_format));
+    *end_bit = L.total_bits > 0 ? L.total_bits : 1;
+    *begin_bit = major_only && L.minor_bits + L.inner_bits < *end_bit ? L.minor_bits + L.inner_bits : 0;
+    return true;
+}
+
+// The analysis workspace: keys x2, positions x2, flags and their scan per
+// stored value, segments, two counters, and the library's temporary storage.
+struct AnalyzeLayout {
+    size_t tmp = 0, bytes = 0;
+};
+
+int analyze_layout(const jlust_sparse *src, int dst_format, const KeyLayout &L, AnalyzeLayout *out)
+{
+    const int64_t N = src->nnz;
+    *out = AnalyzeLayout();
+    if (N == 0) return JLUST_STATUS_SUCCESS;
+    size_t scan = 0, sort = 0;
+    if (int e = scan_bytes(std::max(N, segment_positions(src)), &scan)) return e;
+    int begin_bit = 0, end_bit = 0;
+    if (sort_bits(src, dst_format, L, &begin_bit, &end_bit))
+        if (int e = sort_bytes(N, begin_bit, end_bit, &sort)) return e;
+    out->tmp = (std::max(scan, sort) + 255) / 256 * 256;
+    out->bytes = out->tmp + 8 * (size_t)N * 2 + 4 * (size_t)N * 4 + 4 * (size_t)segment_positions(src) + 256;
+    return JLUST_STATUS_SUCCESS;
+}
+
+// ws: analyze_layout's bytes, the caller's (the handle keeps pointers into it).
 template <typename T>
-int analyze(const jlust_sparse *src, jlust_convert *h, hipStream_t st)
+int analyze(const jlust_sparse *src, jlust_convert *h, void *ws, const AnalyzeLayout &al, hipStream_t st)
 {
     const int64_t N = src->nnz;
     KeyLayout &L = h->L;
     if (N == 0) return JLUST_STATUS_SUCCESS;
-    // Workspace: seg (per value or block), keys x2, pos x2, flags, scan.
-    Workspace ws, tmpw;
-    size_t tmp_bytes = 0;
     const size_t n = (size_t)N;
-    const size_t nseg_len = (size_t)(src->format == JLUST_FORMAT_BSR ? src->nouter : N) + 1;
-    const size_t bytes = 8 * n * 2 + 4 * n * 4 + 4 * nseg_len + 64;
-    JLUST_HIP_TRY(hipMalloc(&ws.p, bytes));
-    char *b = (char *)ws.p;
+    char *b = (char *)ws;
+    void *tmp = b;                    b += al.tmp;
     uint64_t *k0 = (uint64_t *)b;     b += 8 * n;
     uint64_t *k1 = (uint64_t *)b;     b += 8 * n;
     int32_t *p0 = (int32_t *)b;       b += 4 * n;
     int32_t *p1 = (int32_t *)b;       b += 4 * n;
     int32_t *flag = (int32_t *)b;     b += 4 * n;
     int32_t *idx = (int32_t *)b;      b += 4 * n;
-    int32_t *seg = (int32_t *)b;      b += 4 * nseg_len;
-    int32_t *bad = (int32_t *)b;      // bad[0]: a coordinate out of range; bad[1]: values dropped
+    int32_t *bad = (int32_t *)b;      b += 64;   // bad[0]: a coordinate out of range; bad[1]: values dropped
+    int32_t *seg = (int32_t *)b;
     JLUST_HIP_TRY(hipMemsetAsync(bad, 0, 2 * sizeof(int32_t), st));
 
     int64_t seglen = 0;
-    if (int e = segments(src, seg, seglen, tmpw.p, tmp_bytes, st)) return e;
+    if (int e = segments(src, seg, seglen, tmp, st)) return e;
     hipLaunchKernelGGL((decompose_kernel<T>), dim3(cv_grid(N)), dim3(CV_BLOCK), 0, st, *src, seg, L, k0,
                        flag, bad, bad + 1);
     if (int e = check_launch("decompose_kernel")) return e;
 
-    auto ensure = [&](size_t need) -> int {
-        if (need > tmp_bytes) {
-            if (tmpw.p) JLUST_HIP_TRY(hipFree(tmpw.p));
-            tmpw.p = nullptr;
-            JLUST_HIP_TRY(hipMalloc(&tmpw.p, need));
-            tmp_bytes = need;
-        }
-        return JLUST_STATUS_SUCCESS;
-    };
     // count of flagged items (exclusive scan + last flag), read back.
     auto count_flags = [&](int64_t len, int64_t *out) -> int {
         size_t need = 0;
         JLUST_HIP_TRY(rocprim::exclusive_scan(nullptr, need, flag, idx, 0, (size_t)len,
                                               rocprim::plus<int32_t>(), st));
-        if (int e = ensure(need)) return e;
-        JLUST_HIP_TRY(rocprim::exclusive_scan(tmpw.p, need, flag, idx, 0, (size_t)len,
+        JLUST_HIP_TRY(rocprim::exclusive_scan(tmp, need, flag, idx, 0, (size_t)len,
                                               rocprim::plus<int32_t>(), st));
         int32_t last[2] = {0, 0};
         JLUST_HIP_TRY(hipMemcpyAsync(&last[0], idx + len - 1, 4, hipMemcpyDeviceToHost, st));
@@ -481,28 +525,21 @@ int analyze(const jlust_sparse *src, jlust_convert *h, hipStream_t st)
     }
     if (K == 0) return JLUST_STATUS_SUCCESS;
 
-    // 2. sort by level coordinates unless target and source share the
-    // identity ordering (convert.jl:331-349).
-    const bool sort = !(dst_identity(h->dst_format) && src_ordered_identity(src->format));
-    if (sort) {
+    // 2. sort by level coordinates.
+    int begin_bit = 0, end_bit = 0;
+    if (sort_bits(src, h->dst_format, L, &begin_bit, &end_bit)) {
         if (!pc) {                                  // the positions to carry: 0..K-1
             hipLaunchKernelGGL(iota_kernel, dim3(cv_grid(K)), dim3(CV_BLOCK), 0, st, K, p1);
             if (int e = check_launch("iota_kernel")) return e;
             pc = p1;
         }
         uint64_t *ko = kc == k0 ? k1 : k0;
-        // A source whose segments run in the order of the target's minor
-        // coordinate (CSR rows to a CSC target, CSC columns to a row-major
-        // one) holds equal majors in ascending minor order already, so the
-        // stable sort need only order the major bits.
-        const bool major_only = (src->format == JLUST_FORMAT_CSR && h->dst_format == JLUST_FORMAT_CSC) ||
-                                (src->format == JLUST_FORMAT_CSC && dst_identity(h->dst_format));
-        const int end_bit = L.total_bits > 0 ? L.total_bits : 1;
-        const int begin_bit = major_only && L.minor_bits + L.inner_bits < end_bit ? L.minor_bits + L.inner_bits : 0;
         size_t need = 0;
         JLUST_HIP_TRY(rocprim::radix_sort_pairs(nullptr, need, kc, ko, pc, p0, (size_t)K, begin_bit, end_bit, st));
-        if (int e = ensure(need)) return e;
-        JLUST_HIP_TRY(rocprim::radix_sort_pairs(tmpw.p, need, kc, ko, pc, p0, (size_t)K, begin_bit, end_bit, st));
+        Workspace more;                             // fewer entries than N may take another sort
+        if (need > al.tmp) JLUST_HIP_TRY(hipMalloc(&more.p, need));
+        JLUST_HIP_TRY(rocprim::radix_sort_pairs(more.p ? more.p : tmp, need, kc, ko, pc, p0, (size_t)K, begin_bit,
+                                                end_bit, st));
         kc = ko;
         pc = p0;
     } else if (h->dst_format == JLUST_FORMAT_CSR) {
@@ -544,9 +581,8 @@ int analyze(const jlust_sparse *src, jlust_convert *h, hipStream_t st)
     // 4. the handle keeps the workspace: keys, positions, and (DCSR rows /
     // BSR blocks) run heads and ids in the flag and index arrays, free now.
     const size_t c = (size_t)C;
-    h->mem = ws.p;
-    ws.p = nullptr;
     h->keys = kc;
+    h->spare = kc == k0 ? k1 : k0;
     h->pos = pc;
     h->head = flag;
     h->run = idx;
@@ -562,8 +598,7 @@ int analyze(const jlust_sparse *src, jlust_convert *h, hipStream_t st)
         if (int e = check_launch("head_kernel")) return e;
         size_t need = 0;
         JLUST_HIP_TRY(rocprim::inclusive_scan(nullptr, need, h->head, h->run, c, rocprim::plus<int32_t>(), st));
-        if (int e = ensure(need)) return e;
-        JLUST_HIP_TRY(rocprim::inclusive_scan(tmpw.p, need, h->head, h->run, c, rocprim::plus<int32_t>(), st));
+        JLUST_HIP_TRY(rocprim::inclusive_scan(tmp, need, h->head, h->run, c, rocprim::plus<int32_t>(), st));
         int32_t nr = 0;
         JLUST_HIP_TRY(hipMemcpyAsync(&nr, h->run + C - 1, 4, hipMemcpyDeviceToHost, st));
         JLUST_HIP_TRY(hipStreamSynchronize(st));
@@ -621,7 +656,7 @@ int fill(const jlust_convert *h, const jlust_sparse *d, hipStream_t st)
         const int64_t nv = nb * L.b1 * L.b2;
         int32_t *brow = nullptr;
         if (nb > 0) {
-            JLUST_HIP_TRY(hipMallocAsync((void **)&brow, 4 * (size_t)nb, st));
+            brow = (int32_t *)h->spare;              // nb blocks, of one stored value or more each
             hipLaunchKernelGGL((zero_kernel<T>), dim3(cv_grid(nv)), dim3(CV_BLOCK), 0, st, nv, (T *)d->val);
             if (int e = check_launch("zero_kernel")) return e;
             hipLaunchKernelGGL((fill_bsr_kernel<T>), dim3(cv_grid(C)), dim3(CV_BLOCK), 0, st, C, h->keys, h->pos,
@@ -631,7 +666,6 @@ int fill(const jlust_convert *h, const jlust_sparse *d, hipStream_t st)
         hipLaunchKernelGGL(lower_bound_ptr_kernel, dim3(cv_grid(L.major_dim + 1)), dim3(CV_BLOCK), 0, st, nb,
                            (const uint64_t *)nullptr, brow, L, L.major_dim, o, d->pos2);
         if (int e = check_launch("lower_bound_ptr_kernel")) return e;
-        if (brow) JLUST_HIP_TRY(hipFreeAsync(brow, st));
     }
     }
     return JLUST_STATUS_SUCCESS;
@@ -680,15 +714,12 @@ bool src_ptrs_ok(const jlust_sparse *s)
 
 }  // namespace
 
-extern "C" int jlust_hip_convert_analyze(const jlust_sparse *src, int32_t dst_format, int32_t dst_b1,
-                                         int32_t dst_b2, int32_t dst_row_major_blocks, int value_type,
-                                         jlust_stream_t stream, jlust_convert_t *out, int64_t *dst_nnz,
-                                         int64_t *dst_nouter)
+namespace {
+
+// The checks and the key layout of an analysis.
+int analyze_args(const jlust_sparse *src, int32_t dst_format, int32_t dst_b1, int32_t dst_b2,
+                 int32_t dst_row_major_blocks, int value_type, KeyLayout *L)
 {
-    clear_error();
-    if (!out || !dst_nnz || !dst_nouter)
-        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: null output pointer");
-    *out = nullptr;
     if (int st = check_sparse(src, "convert_analyze")) return st;
     if (!check_format(dst_format))
         return fail(JLUST_STATUS_UNSUPPORTED_FORMAT, "convert_analyze: unknown target format %d", dst_format);
@@ -700,7 +731,29 @@ extern "C" int jlust_hip_convert_analyze(const jlust_sparse *src, int32_t dst_fo
         return fail(JLUST_STATUS_INVALID_ARGUMENT,
                     "convert_analyze: BSR block size %d x %d does not tile %lld x %lld", dst_b1, dst_b2,
                     (long long)src->m, (long long)src->n);
+    *L = layout_for(dst_format, src->m, src->n, dst_b1, dst_b2, dst_row_major_blocks);
+    if (L->total_bits > 64)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: coordinates need more than 64 key bits");
+    return JLUST_STATUS_SUCCESS;
+}
+
+// ws null: the handle allocates its workspace and frees it when destroyed.
+int convert_analyze(const jlust_sparse *src, int32_t dst_format, int32_t dst_b1, int32_t dst_b2,
+                    int32_t dst_row_major_blocks, int value_type, void *ws, size_t ws_bytes, hipStream_t stream,
+                    jlust_convert_t *out, int64_t *dst_nnz, int64_t *dst_nouter)
+{
+    clear_error();
+    if (!out || !dst_nnz || !dst_nouter)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: null output pointer");
+    *out = nullptr;
+    KeyLayout L;
+    if (int st = analyze_args(src, dst_format, dst_b1, dst_b2, dst_row_major_blocks, value_type, &L)) return st;
     if (int st = require_device(nullptr)) return st;
+    AnalyzeLayout al;
+    if (int st = analyze_layout(src, dst_format, L, &al)) return st;
+    if (ws && ws_bytes < al.bytes)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: workspace of %zu bytes, %zu needed", ws_bytes,
+                    al.bytes);
     auto *h = new jlust_convert();
     h->dst_format = dst_format;
     h->origin = src->origin;
@@ -708,13 +761,15 @@ extern "C" int jlust_hip_convert_analyze(const jlust_sparse *src, int32_t dst_fo
     h->m = src->m;
     h->n = src->n;
     h->src_val = src->val;
-    h->L = layout_for(dst_format, src->m, src->n, dst_b1, dst_b2, dst_row_major_blocks);
-    if (h->L.total_bits > 64) {
-        delete h;
-        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: coordinates need more than 64 key bits");
+    h->L = L;
+    int st = JLUST_STATUS_SUCCESS;
+    if (!ws && al.bytes) {
+        const hipError_t e = hipMalloc(&h->mem, al.bytes);
+        if (e != hipSuccess) st = hip_fail(e, "hipMalloc(convert workspace)");
+        ws = h->mem;
     }
-    const int st = value_type == 0 ? analyze<double>(src, h, (hipStream_t)stream)
-                                   : analyze<float>(src, h, (hipStream_t)stream);
+    if (!st)
+        st = value_type == 0 ? analyze<double>(src, h, ws, al, stream) : analyze<float>(src, h, ws, al, stream);
     if (st) {
         if (h->mem) (void)hipFree(h->mem);
         delete h;
@@ -724,6 +779,43 @@ extern "C" int jlust_hip_convert_analyze(const jlust_sparse *src, int32_t dst_fo
     *dst_nouter = (dst_format == JLUST_FORMAT_DCSR || dst_format == JLUST_FORMAT_BSR) ? h->nruns : 0;
     *out = h;
     return JLUST_STATUS_SUCCESS;
+}
+
+}  // namespace
+
+extern "C" int jlust_hip_convert_analyze(const jlust_sparse *src, int32_t dst_format, int32_t dst_b1,
+                                         int32_t dst_b2, int32_t dst_row_major_blocks, int value_type,
+                                         jlust_stream_t stream, jlust_convert_t *out, int64_t *dst_nnz,
+                                         int64_t *dst_nouter)
+{
+    return convert_analyze(src, dst_format, dst_b1, dst_b2, dst_row_major_blocks, value_type, nullptr, 0,
+                           (hipStream_t)stream, out, dst_nnz, dst_nouter);
+}
+
+extern "C" int jlust_hip_convert_workspace(const jlust_sparse *src, int32_t dst_format, int32_t dst_b1,
+                                           int32_t dst_b2, int32_t dst_row_major_blocks, int value_type,
+                                           int64_t *bytes)
+{
+    clear_error();
+    if (!bytes) return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_workspace: null output pointer");
+    KeyLayout L;
+    if (int st = analyze_args(src, dst_format, dst_b1, dst_b2, dst_row_major_blocks, value_type, &L)) return st;
+    if (int st = require_device(nullptr)) return st;
+    AnalyzeLayout al;
+    if (int st = analyze_layout(src, dst_format, L, &al)) return st;
+    *bytes = (int64_t)al.bytes;
+    return JLUST_STATUS_SUCCESS;
+}
+
+extern "C" int jlust_hip_convert_analyze_ws(const jlust_sparse *src, int32_t dst_format, int32_t dst_b1,
+                                            int32_t dst_b2, int32_t dst_row_major_blocks, int value_type,
+                                            void *ws, int64_t ws_bytes, jlust_stream_t stream,
+                                            jlust_convert_t *out, int64_t *dst_nnz, int64_t *dst_nouter)
+{
+    if (ws_bytes < 0 || (ws_bytes > 0 && !ws) || (uintptr_t)ws % 256)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: workspace null or not 256-byte aligned");
+    return convert_analyze(src, dst_format, dst_b1, dst_b2, dst_row_major_blocks, value_type, ws, (size_t)ws_bytes,
+                           (hipStream_t)stream, out, dst_nnz, dst_nouter);
 }
 
 extern "C" int jlust_hip_convert_fill(jlust_convert_t h, const jlust_sparse *dst, jlust_stream_t stream)
@@ -768,18 +860,21 @@ extern "C" int jlust_hip_sparse_to_dense(const jlust_sparse *src, int value_type
     const int64_t N = src->nnz;
     if (N == 0) return JLUST_STATUS_SUCCESS;
     const KeyLayout L = layout_for(JLUST_FORMAT_CSR, src->m, src->n, 1, 1, 1);
-    Workspace ws, tmpw;
+    Workspace ws;
     size_t tmp_bytes = 0;
+    if (int st = scan_bytes(segment_positions(src), &tmp_bytes)) return st;
+    tmp_bytes = (tmp_bytes + 255) / 256 * 256;
     const size_t nseg_len = (size_t)(src->format == JLUST_FORMAT_BSR ? src->nouter : N) + 1;
-    JLUST_HIP_TRY(hipMalloc(&ws.p, 8 * (size_t)N + 4 * (size_t)N + 4 * nseg_len + 64));
+    JLUST_HIP_TRY(hipMalloc(&ws.p, tmp_bytes + 8 * (size_t)N + 4 * (size_t)N + 4 * nseg_len + 64));
     char *b = (char *)ws.p;
+    void *tmp = b;                      b += tmp_bytes;
     uint64_t *k = (uint64_t *)b;        b += 8 * (size_t)N;
     int32_t *keep = (int32_t *)b;       b += 4 * (size_t)N;
     int32_t *seg = (int32_t *)b;        b += 4 * nseg_len;
     int32_t *bad = (int32_t *)b;
     JLUST_HIP_TRY(hipMemsetAsync(bad, 0, 4, s));
     int64_t seglen = 0;
-    if (int st = segments(src, seg, seglen, tmpw.p, tmp_bytes, s)) return st;
+    if (int st = segments(src, seg, seglen, tmp, s)) return st;
     if (value_type == 0)
         hipLaunchKernelGGL((decompose_kernel<double>), dim3(cv_grid(N)), dim3(CV_BLOCK), 0, s, *src, seg, L, k,
                            keep, bad, nullptr);

@@ -254,3 +254,40 @@ def test_config5_bsr_round_trip_full_size(J):
     assert np.array_equal(host(b.pos_buffers[1]), cfg["browptr"])
     assert np.array_equal(host(b.crd_buffers[1]), cfg["bcolind"])
     assert np.array_equal(host(b.val).view(np.uint32), cfg["val"].view(np.uint32))
+
+
+@pytest.mark.parametrize("dst", ["CSC", "COO", "DCSR", "BSR"])
+def test_workspace_of_the_caller(J, CO, dst):
+    """convert_analyze (the handle's own workspace) and convert_analyze_ws
+    (the caller's) analyse alike; a workspace that is too small or not
+    aligned is refused."""
+    import ctypes
+    import torch
+    from jlust_amd import _lib
+    from jlust_amd import convert as CV
+    csr, _ = random_source(CO, 3, 1, np.float64)
+    u = to_ust(J, csr)
+    fid, b1, b2, rm = CV._format_id(fmt_of(J, dst, 4, 2))
+    L, src = _lib.lib(), CV._descriptor(u)
+    args = (ctypes.byref(src), fid, b1, b2, int(rm), 0)
+    stream = CV._stream(u.val.device)
+
+    def run(ws, size):
+        h, nz, no = ctypes.c_void_p(), ctypes.c_int64(-1), ctypes.c_int64(-1)
+        tail = (stream, ctypes.byref(h), ctypes.byref(nz), ctypes.byref(no))
+        st = (L.jlust_hip_convert_analyze(*args, *tail) if size is None else
+              L.jlust_hip_convert_analyze_ws(*args, ws, size, *tail))
+        if h.value:
+            L.jlust_hip_convert_destroy(h)
+        return st, nz.value, no.value
+
+    need = ctypes.c_int64()
+    assert L.jlust_hip_convert_workspace(*args, ctypes.byref(need)) == 0 and need.value > 0
+    buf = torch.empty(need.value + 256, dtype=torch.uint8, device="cuda")
+    own = run(None, None)
+    assert own[0] == 0 and run(buf.data_ptr(), need.value) == own
+    assert run(buf.data_ptr(), need.value - 1)[0] != 0
+    assert run(buf.data_ptr() + 8, need.value)[0] != 0
+    assert run(None, need.value)[0] != 0
+    got = J.convert_format(u, fmt_of(J, dst, 4, 2))
+    assert got.val.numel() == own[1]
