@@ -11,7 +11,7 @@
 // library's scratch buffer with an LDS-tiled transpose: one coalesced read
 // and one coalesced write of B.  csr_spmm_rows_kernel then gathers whole rows
 // of Bt for several rows of A at once, and writes its results column by column
-// through LDS.  One column needs no copy (csr_spmm_col_kernel).
+// through LDS.  One column needs no copy (csr_spmm_group_kernel).
 #include "common.hpp"
 
 #include <cstdlib>
@@ -87,27 +87,37 @@ __global__ __launch_bounds__(256) void transpose_kernel(int64_t n, int64_t k, co
     }
 }
 
-// One column: a wave per row, 64 entries per step, gathered from B's own
-// column.  U steps are loaded at once (indices clamped into the row, products
-// of the clamped copies dropped by a select; U is chosen per call from the mean
-// row length, so a short row issues no clamped copies), and the next row's
-// pointers are loaded before the current row's nonzeros, so a wave's rows do
-// not wait on each other's pointer loads.
-template <typename T, int U>
-__global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_col_kernel(
-    int64_t m, int32_t origin, const int32_t *__restrict__ rowptr, const int32_t *__restrict__ rowend,
-    const uint8_t *__restrict__ row_skip, const int32_t *__restrict__ colind, const T *__restrict__ val,
-    const T *__restrict__ B, T alpha, T beta, int beta_zero, T *__restrict__ C, int skip_empty_rows)
+// One column, and 2 to 4 columns of long rows: groups of KV lanes (KV the
+// smallest power of two >= the columns), one nonzero per group per step, so a
+// wave takes 64/KV nonzeros per step (64 at k = 1, where the kernel is a
+// wave-per-row SpMV).  Each lane loads its group's col/val itself (the group's
+// lanes read one address), gathers its column of the nonzero's Bt row, and
+// keeps its group's sum in nonzero order; the groups' sums are added with
+// xor-shuffles at the row's end.  U steps are loaded at once (indices clamped
+// into the row, products of the clamped copies dropped by a select; U is
+// chosen per call from the mean row length, so a short row issues no clamped
+// copies), and the next row's pointers are loaded before the current row's
+// nonzeros, so a wave's rows do not wait on each other's pointer loads.
+template <typename T, int KV, int U>
+__global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_group_kernel(
+    int64_t m, int64_t k, int32_t origin, const int32_t *__restrict__ rowptr,
+    const int32_t *__restrict__ colind, const T *__restrict__ val, const T *__restrict__ Bt,
+    int64_t ldt, T alpha, T beta, int beta_zero, T *__restrict__ C, int64_t ldc,
+    int skip_empty_rows, const int32_t *__restrict__ rowend, const uint8_t *__restrict__ row_skip)
 {
+    constexpr int G = 64 / KV;                 // nonzeros per step
     constexpr int NW = SPMM_BLOCK / 64;
-    __shared__ T s_c[SPMM_ROWS];
+    __shared__ T s_c[SPMM_ROWS][KV + 1];
     __shared__ int s_empty[SPMM_ROWS];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
+    const int grp = lane / KV;
+    const int col = lane % KV;
     const int64_t row0 = (int64_t)blockIdx.x * SPMM_ROWS;
     const int nrows = (int)min((int64_t)SPMM_ROWS, m - row0);
+    const int64_t cl = col < k ? col : 0;      // clamped, in-bounds column
 
     int32_t lo_n = 0, hi_n = 0;
     if (wave < nrows) {
@@ -125,32 +135,38 @@ __global__ __launch_bounds__(SPMM_BLOCK) void csr_spmm_col_kernel(
         if (skip) hi = lo;                     // a split row: its segments compute it
         if (lane == 0) s_empty[rr] = skip ? 2 : hi <= lo;
         T acc = T(0);
-        for (int64_t p0 = lo + lane; p0 < hi; p0 += (int64_t)64 * U) {
+        for (int64_t p0 = lo + grp; p0 < hi; p0 += (int64_t)G * U) {
             int32_t c[U];
             T a[U], b[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int64_t p = min(p0 + (int64_t)u * 64, hi - 1);
+                const int64_t p = min(p0 + (int64_t)u * G, hi - 1);
                 c[u] = colind[p];
                 a[u] = val[p];
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) b[u] = B[c[u] - origin];
+            for (int u = 0; u < U; ++u) b[u] = Bt[(int64_t)(c[u] - origin) * ldt + cl];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const T s = acc + a[u] * b[u];
-                acc = p0 + (int64_t)u * 64 < hi ? s : acc;
+                acc = p0 + (int64_t)u * G < hi ? s : acc;
             }
         }
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
-        if (lane == 0) s_c[rr] = acc;
+        for (int off = KV; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
+        if (lane < KV) s_c[rr][col] = acc;
     }
     __syncthreads();
-    if (tid >= nrows || s_empty[tid] == 2 || (skip_empty_rows && s_empty[tid])) return;
-    T *dst = C + row0 + tid;
-    const T s = alpha * s_c[tid];
-    *dst = beta_zero ? s : s + beta * *dst;
+    const int ncols = (int)k;                  // k <= KV here
+    for (int idx = tid; idx < SPMM_ROWS * ncols; idx += SPMM_BLOCK) {
+        const int rr = idx % SPMM_ROWS;
+        const int cc = idx / SPMM_ROWS;
+        if (rr >= nrows) continue;
+        if (s_empty[rr] == 2 || (skip_empty_rows && s_empty[rr])) continue;
+        T *dst = C + (row0 + rr) + cc * ldc;
+        const T s = alpha * s_c[rr][cc];
+        *dst = beta_zero ? s : s + beta * *dst;
+    }
 }
 
 // A set of rows for csr_spmm_rows_kernel: the matrix's rows (hi null: row r
@@ -206,7 +222,7 @@ __device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 //     gathers.  Groups past their row's end read a staged entry that points at
 //     Bt's row of zeros, so no product needs a select.
 //   - The unit of work is a slice of a row: 32 to 256 entries by the number of
-//     columns, counted from the row's start, so most rows are one.  A slice is
+//     columns, counted from the row's start, so most rows are one. A slice is
 //     summed by one group, and a row's slices are added in order: a
 //     row's sum depends on its own entries alone, not on the rows around it.
 //     Slices are dealt to the groups longest first (whole slices, then what
@@ -488,18 +504,26 @@ __global__ void spmm_long_reduce_kernel(int64_t nlong, int64_t kk, const int32_t
 //     rather have 16).  f64 keeps 16: the mesh loses more than random rows
 //     gain (262k rows, k = 128: 519 -> 680 us; 200k uniform rows of 16: 585 ->
 //     567 us).
+//   - The group kernel for one column, and for 2 to 4 (f64: 2) where rows hold
+//     more than 48 entries on average: so few columns leave the rows kernel's
+//     slices too few for its groups (200 entries a row, band of +-150, f32:
+//     k = 2 86.9 against 50.9 us, k = 4 99.4 against 74.7 us; f64: k = 2 92.8
+//     against 68.6, k = 4 107.7 against 125.9; with 27 entries, f32, k = 4,
+//     27.6 against 54.2 us).
 struct SpmmChunk {
-    bool direct;
+    bool group;                          // the group kernel
+    bool direct;                         // B's own column, no copy
     int vec;
     int64_t ldt;
 };
 
 template <typename T>
-SpmmChunk spmm_chunk_kind(int64_t n, int64_t kk)
+SpmmChunk spmm_chunk_kind(int64_t n, int64_t kk, int64_t mean)
 {
     constexpr int W16 = 16 / sizeof(T), W8 = 8 / sizeof(T);
     SpmmChunk c;
     c.direct = kk == 1;
+    c.group = c.direct || (kk <= (sizeof(T) == 4 ? 4 : 2) && mean > 48);
     c.vec = W16;
     if (sizeof(T) == 4 && kk >= 48 && n * kk * 4 > (int64_t)128 << 20) c.vec = W8;
     if (kk <= 12 && sizeof(T) == 4) c.vec = W8;
@@ -514,23 +538,24 @@ int64_t spmm_copy_elems(int64_t n, int64_t kc, int64_t k)
     return (n + 1) * ((min(kc, k > 0 ? k : 1) + 3) / 4 * 4);
 }
 
-// Row-major copy of columns [c0, c0+kk) of B into Bt (skipped when direct).
+// Row-major copy of kk columns of B into Bt, vec columns per write (ldt a
+// multiple of vec).
 template <typename T>
-int spmm_copy_chunk(int64_t n, int64_t kk, const T *B, int64_t ldb, const SpmmChunk &ck, T *Bt, hipStream_t s)
+int spmm_copy_chunk(int64_t n, int64_t kk, const T *B, int64_t ldb, T *Bt, int64_t ldt, int vec, hipStream_t s)
 {
-    if (n == 0 || ck.direct) return JLUST_STATUS_SUCCESS;
+    if (n == 0) return JLUST_STATUS_SUCCESS;
 #define JLUST_TRANSPOSE(V, CT)                                                                             \
     hipLaunchKernelGGL((transpose_kernel<T, V, CT>),                                                       \
                        dim3((unsigned)(n / (4096 / CT) + 1), (unsigned)((kk + CT - 1) / CT)), dim3(256), 0, \
-                       s, n, kk, B, ldb, Bt, ck.ldt)
+                       s, n, kk, B, ldb, Bt, ldt)
 #define JLUST_TRANSPOSE_CT(V)                \
     do {                                     \
         if (kk <= 16) JLUST_TRANSPOSE(V, 16); \
         else if (kk <= 32) JLUST_TRANSPOSE(V, 32); \
         else JLUST_TRANSPOSE(V, 64);         \
     } while (0)
-    if (ck.vec == 1) JLUST_TRANSPOSE_CT(1);
-    else if (ck.vec == 2) JLUST_TRANSPOSE_CT(2);
+    if (vec == 1) JLUST_TRANSPOSE_CT(1);
+    else if (vec == 2) JLUST_TRANSPOSE_CT(2);
     else JLUST_TRANSPOSE_CT((16 / (int)sizeof(T)));
 #undef JLUST_TRANSPOSE_CT
 #undef JLUST_TRANSPOSE
@@ -615,27 +640,34 @@ int spmm_rows_pass(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, int
     return run(std::integral_constant<int, 16 / sizeof(T)>());
 }
 
-// The product of one column over m rows (rows of A, or segments when rowend
-// is given): C = alpha * A[rows, :] * B + beta * C, rows flagged in row_skip
-// left untouched.  nnz_rows: the entries these rows hold.
+// The product of one narrow chunk over m rows (rows of A, or segments when
+// rowend is given) by the group kernel: C[:, 0:kk] (ldc) = alpha * A[rows, :] *
+// Bsrc + beta * C, rows flagged in row_skip left untouched.  nnz_rows: the
+// entries these rows hold (for the steps per load).
 template <typename T>
-int spmm_col_launch(int64_t m, int64_t nnz_rows, int32_t origin, const int32_t *rowptr, const int32_t *rowend,
-                    const uint8_t *row_skip, const int32_t *colind, const T *val, const T *B, T alpha, T beta, T *C,
-                    int skip_empty_rows, hipStream_t s)
+int spmm_group_launch(int64_t m, int64_t kk, int64_t nnz_rows, int32_t origin, const SpmmJob<T> &j,
+                      const int32_t *colind, const T *val, const T *Bsrc, int64_t ldt, hipStream_t s)
 {
     if (m == 0) return JLUST_STATUS_SUCCESS;
     const dim3 grid((unsigned)((m + SPMM_ROWS - 1) / SPMM_ROWS));
-    const int bz = beta == T(0);
-    const int64_t steps = (nnz_rows + m * 64 - 1) / (m * 64);     // per row
-#define JLUST_COL(U)                                                                                        \
-    hipLaunchKernelGGL((csr_spmm_col_kernel<T, U>), grid, dim3(SPMM_BLOCK), 0, s, m, origin, rowptr, rowend, \
-                       row_skip, colind, val, B, alpha, beta, bz, C, skip_empty_rows)
-    if (steps <= 1) JLUST_COL(1);
-    else if (steps <= 2) JLUST_COL(2);
-    else if (steps <= 4) JLUST_COL(4);
-    else JLUST_COL(8);
-#undef JLUST_COL
-    return check_launch("csr_spmm_col_kernel");
+#define JLUST_GROUP_U(KV, U)                                                                                \
+    hipLaunchKernelGGL((csr_spmm_group_kernel<T, KV, U>), grid, dim3(SPMM_BLOCK), 0, s, m, kk, origin, j.lo, \
+                       colind, val, Bsrc, ldt, j.alpha, j.beta, j.beta_zero, j.C, j.ldc, j.skip_empty_rows,  \
+                       j.hi, j.skip)
+#define JLUST_GROUP(KV)                                                                                \
+    do {                                                                                               \
+        const int64_t steps = (nnz_rows + m * (64 / KV) - 1) / (m * (64 / KV));  /* per row */          \
+        if (steps <= 1) JLUST_GROUP_U(KV, 1);                                                          \
+        else if (steps <= 2) JLUST_GROUP_U(KV, 2);                                                     \
+        else if (steps <= 4) JLUST_GROUP_U(KV, 4);                                                     \
+        else JLUST_GROUP_U(KV, 8);                                                                     \
+    } while (0)
+    if (kk == 1) JLUST_GROUP(1);
+    else if (kk == 2) JLUST_GROUP(2);
+    else JLUST_GROUP(4);
+#undef JLUST_GROUP
+#undef JLUST_GROUP_U
+    return check_launch("csr_spmm_group_kernel");
 }
 
 // One column chunk over the rows of ja and the segments of jb.
@@ -644,15 +676,16 @@ int spmm_chunk(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, int32_t
                const SpmmJob<T> &jb, const int32_t *colind, const T *val, const T *B, int64_t ldb, T *Bt,
                hipStream_t s)
 {
-    const SpmmChunk ck = spmm_chunk_kind<T>(n, kk);
-    if (ck.direct) {
-        for (const SpmmJob<T> *j : {&ja, &jb})
-            if (int st = spmm_col_launch<T>(j->rows, j == &ja ? nnz_rows : nnz_seg, origin, j->lo, j->hi, j->skip,
-                                            colind, val, B, j->alpha, j->beta, j->C, j->skip_empty_rows, s))
-                return st;
-        return JLUST_STATUS_SUCCESS;
+    // The mean over all entries, so that a plan and a plain call choose alike.
+    const int64_t mean = ja.rows ? (nnz_rows + nnz_seg) / ja.rows : 0;
+    const SpmmChunk ck = spmm_chunk_kind<T>(n, kk, mean);
+    if (!ck.direct)
+        if (int st = spmm_copy_chunk<T>(n, kk, B, ldb, Bt, ck.ldt, ck.vec, s)) return st;
+    if (ck.group) {
+        const T *Bsrc = ck.direct ? B : Bt;
+        if (int st = spmm_group_launch<T>(ja.rows, kk, nnz_rows, origin, ja, colind, val, Bsrc, ck.ldt, s)) return st;
+        return spmm_group_launch<T>(jb.rows, kk, nnz_seg, origin, jb, colind, val, Bsrc, ck.ldt, s);
     }
-    if (int st = spmm_copy_chunk<T>(n, kk, B, ldb, ck, Bt, s)) return st;
     return spmm_rows_pass<T>(n, kk, nnz_rows, nnz_seg, origin, ja, jb, colind, val, Bt, ck, s);
 }
 
@@ -719,6 +752,15 @@ int csr_spmm(int64_t m, int64_t n, int64_t k, int64_t nnz, int32_t origin,
 }
 
 }  // namespace
+
+int spmm_row_major_copy(int value_type, int64_t n, int64_t k, const void *B, int64_t ldb, void *Bt, int64_t ldt,
+                        hipStream_t s)
+{
+    if (value_type == 0)
+        return spmm_copy_chunk<double>(n, k, (const double *)B, ldb, (double *)Bt, ldt, ldt % 2 ? 1 : 2, s);
+    return spmm_copy_chunk<float>(n, k, (const float *)B, ldb, (float *)Bt, ldt, ldt % 2 ? 1 : ldt % 4 ? 2 : 4, s);
+}
+
 }  // namespace jlust
 
 using namespace jlust;
