@@ -788,20 +788,43 @@ int jlust_hip_bsr_expand_csr_i32(int64_t mb, int64_t b1, int64_t b2,
                                  void *val_out, jlust_stream_t stream);
 
 /*
+ * C = alpha*A*B + beta*C for square blocks of 2 to 8 rows on the blocks as
+ * stored: *taken = 1 if the product ran, 0 if it is left to
+ * jlust_hip_bsr_expand_csr_i32 + the CSR entry points (another shape, k < 2,
+ * a copy of B past 4 GiB, block-rows far longer than the mean, or a browptr
+ * that is not canonical).  Arguments as jlust_hip_bsr_spmm_*.  Reads the
+ * longest block-row back, so it synchronises `stream` (not capturable; a plan
+ * is).
+ */
+int jlust_hip_bsr_spmm_small_f64_i32(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_t nnzb,
+                                     int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                                     const double *val, int row_major_blocks, int64_t k, double alpha,
+                                     const double *B, int64_t ldb, double beta, double *C, int64_t ldc,
+                                     jlust_stream_t stream, int32_t *taken);
+int jlust_hip_bsr_spmm_small_f32_i32(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_t nnzb,
+                                     int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                                     const float *val, int row_major_blocks, int64_t k, float alpha,
+                                     const float *B, int64_t ldb, float beta, float *C, int64_t ldc,
+                                     jlust_stream_t stream, int32_t *taken);
+
+/*
  * Prepared BSR SpMM, the BSR analyse handle (the cuSPARSE SpMM handle
  * contract, ext/CUDAExt/ops/spmm.jl:8-70: analysis and workspace once,
  * execute many times, update_values! for new values of the same pattern).
  * 16 x 16 blocks keep the MFMA kernels (fp32, with 16-byte aligned values
- * for BSRRight, or fp64) and read the caller's buffers in place.  Any other
+ * for BSRRight, or fp64) and read the caller's buffers in place, and so do
+ * square blocks of 2 to 8 rows whose longest block-row holds at most 64 blocks
+ * or 4 times the mean (k >= 2; the plan owns a copy of B).  Any other
  * b1 x b2 shape is expanded to CSR once (jlust_hip_bsr_expand_csr_i32's
  * layout; the plan owns it) and runs through a CSR SpMM plan over it for k
  * columns.  create synchronises `stream` (browptr's ends are read back and
  * the CSR plan analyses its rows); update_values re-expands only the values,
- * stream-ordered, on the expansion path, and is a pointer swap on the MFMA
- * path.  execute: B (nb*b2) x k (ldb), C (mb*b1) x k (ldc), column-major;
+ * stream-ordered, on the expansion path, and is a pointer swap on the other
+ * two.  execute: B (nb*b2) x k (ldb), C (mb*b1) x k (ldc), column-major;
  * C = alpha*A*B + beta*C (beta == 0: C write-only).  info: path 0 = MFMA,
- * 1 = CSR expansion.  The plan keeps browptr, bcolind (and, on the MFMA path,
- * the values) by pointer: the caller keeps them alive.
+ * 1 = CSR expansion, 2 = small square blocks as stored.  The plan keeps
+ * browptr, bcolind (and, on paths 0 and 2, the values) by pointer: the caller
+ * keeps them alive.
  */
 int jlust_hip_bsr_spmm_plan_create(int64_t mb, int64_t nb, int64_t b1,
                                    int64_t b2, int64_t nnzb, int32_t origin,

@@ -1,0 +1,339 @@
+// bsr_small.hip -- BSR SpMM C = alpha*A*B + beta*C for square blocks of 2 to 8
+// rows (gfx950, wave64), on the blocks as stored.
+//
+// Computes what bsr_spmm.hip computes for these shapes through a CSR
+// expansion (ext/KernelAbstractionsExt/ops/spmm.jl:397-423 over the expanded
+// rows), without the expansion: one column index per block instead of one per
+// entry, and every gathered row of B used for all of the block's rows.
+//
+// B is re-laid row-major (spmm_row_major_copy).  A wave's 64 lanes form NG =
+// 64 / L groups; a group takes a block-row, each lane CPL columns of C for its
+// B block-row rows in registers.  A group's next SB blocks are loaded by its
+// own lanes, a stage ahead, and kept in LDS column by column, from where every
+// lane of the group reads the same 16 bytes; waves share nothing, so nothing
+// waits on a barrier.  Results pass through the wave's LDS and are written as
+// runs of consecutive rows of C.
+//
+// What bounds it is L1: a block gathers B rows of CPL * L columns, and the LDS
+// reads of its values serve NG block-rows at once.  Measured per product, with
+// B's copy: 27-point mesh of 60,680 block-rows of 4 x 4 f64 blocks, k = 24:
+// 955 us through the CSR expansion and the SpMM kernels before, 295 through
+// the present ones, 134 here (2.2 TB/s of compulsory bytes); a plain call,
+// which expanded A every time (440 us), saves that too.  8 x 8 f64, 30,690
+// block-rows, k = 24: 1886 -> 235 us.
+#include <algorithm>
+
+#include "common.hpp"
+
+namespace jlust {
+namespace {
+
+constexpr int BS_BLOCK = 256;
+constexpr int BS_WAVES = BS_BLOCK / 64;
+constexpr int BS_STAGE = 8;              // values a lane loads per stage
+
+template <typename T, int N>
+struct alignas(sizeof(T) * N < 16 ? sizeof(T) * N : 16) Pack {
+    T v[N];
+};
+
+// Orders a wave's LDS accesses (its lanes exchange values through LDS).
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+struct SmallShape {
+    int64_t mb;
+    int64_t ldt;
+    int k;
+    int cols;                            // columns per blockIdx.y
+    int L;                               // lanes per group: cols / CPL or more
+    int sb;                              // blocks per stage
+    int gs;                              // values of a group's stage in LDS
+    int wave_vals;                       // values of a wave's stage or result tile in LDS
+    int wave_stride;                     // values from one wave's LDS to the next
+    int32_t origin;
+    int row_major;
+    unsigned run;                        // consecutive workgroups per XCD
+};
+
+template <typename T, int B, int CPL>
+__global__ __launch_bounds__(BS_BLOCK) void bsr_small_spmm_kernel(
+    SmallShape sh, const int32_t *__restrict__ browptr, const int32_t *__restrict__ bcolind,
+    const T *__restrict__ val, const T *__restrict__ Bt0, T alpha, T beta, int beta_zero, T *__restrict__ C,
+    int64_t ldc)
+{
+    constexpr int V16 = 16 / sizeof(T);
+    constexpr int W = CPL < V16 ? CPL : V16;               // columns per load of B
+    constexpr int AW = B <= 2 ? 2 : V16 < 4 ? 2 : 4;       // values per read of A
+    constexpr int BP = (B + AW - 1) / AW * AW;             // a block row in LDS
+    constexpr int BB = B * B;
+    extern __shared__ __attribute__((aligned(16))) char s_mem[];
+
+    const unsigned x = blockIdx.x % NUM_XCD, i0 = blockIdx.x / NUM_XCD;
+    const int64_t wg = (int64_t)(i0 / sh.run * NUM_XCD + x) * sh.run + i0 % sh.run;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int L = sh.L, NG = 64 / L;
+    const int64_t R0 = (wg * BS_WAVES + wave) * NG;
+    if (R0 >= sh.mb) return;
+    const int grp = lane / L, sub = lane - grp * L;
+    T *const s_a = reinterpret_cast<T *>(s_mem) + wave * sh.wave_stride;
+    uint32_t *const s_off = reinterpret_cast<uint32_t *>(s_a + sh.wave_vals);
+    const int c0 = (int)blockIdx.y * sh.cols;
+    const int kk = min(sh.cols, sh.k - c0);
+    const uint32_t col = (uint32_t)(c0 + min(sub * CPL, (int)sh.ldt - c0 - CPL)) * (uint32_t)sizeof(T);
+    const uint32_t row_bytes = (uint32_t)(sh.ldt * sizeof(T));
+
+    const bool live = grp < NG && R0 + grp < sh.mb;
+    int64_t q0 = 0;
+    int n = 0;
+    if (live) {
+        q0 = (int64_t)browptr[R0 + grp] - sh.origin;
+        n = max(browptr[R0 + grp + 1] - sh.origin - (int)q0, 0);
+    }
+    const T *const va = val + q0 * BB;
+    T *const a_dst = s_a + grp * sh.gs;
+
+    // A stage: blocks s0 .. s0 + sb - 1 of the group, element e = sub + t * L.
+    T st[BS_STAGE];
+    uint32_t oc = 0;
+    auto load_stage = [&](int s0) {
+        const int cnt = min(sh.sb, n - s0);
+        const T *const p = va + (int64_t)s0 * BB;
+#pragma unroll
+        for (int t = 0; t < BS_STAGE; ++t)
+            if (sub + t * L < cnt * BB) st[t] = p[sub + t * L];
+        if (sub < cnt) oc = (uint32_t)(bcolind[q0 + s0 + sub] - sh.origin) * (uint32_t)B * row_bytes;
+    };
+    auto store_stage = [&](int s0) {
+        const int cnt = min(sh.sb, n - s0);
+#pragma unroll
+        for (int t = 0; t < BS_STAGE; ++t) {
+            const int e = sub + t * L;
+            if (e < cnt * BB) {
+                const int blk = e / BB, w = e % BB, r = w / B, c = w % B;
+                const int ii = sh.row_major ? r : c, jj = sh.row_major ? c : r;
+                a_dst[(blk * B + ii) * BP + jj] = st[t];
+            }
+        }
+        if (sub < cnt) s_off[grp * sh.sb + sub] = oc;
+    };
+
+    T acc[B][CPL];
+#pragma unroll
+    for (int r = 0; r < B; ++r)
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) acc[r][c] = T(0);
+
+    load_stage(0);
+    for (int s0 = 0; __any(s0 < n); s0 += sh.sb) {
+        wave_sync();
+        store_stage(s0);
+        wave_sync();
+        load_stage(s0 + sh.sb);
+        const int top = min(sh.sb, n - s0);
+        for (int u = 0; __any(u < top); ++u) {
+            if (u >= top) continue;
+            const char *const bp = reinterpret_cast<const char *>(Bt0);
+            const uint32_t off = s_off[grp * sh.sb + u] + col;
+            Pack<T, W> b[B][CPL / W];
+#pragma unroll
+            for (int jj = 0; jj < B; ++jj)
+#pragma unroll
+                for (int v = 0; v < CPL / W; ++v)
+                    b[jj][v] = *reinterpret_cast<const Pack<T, W> *>(
+                        bp + (off + (uint32_t)jj * row_bytes + (uint32_t)(v * W * sizeof(T))));
+            // A row of the block's own product first, then into the row's sum: a
+            // chain of one rounding per block (as few as the expanded rows'
+            // split sums).
+#pragma unroll
+            for (int r = 0; r < B; ++r) {
+                T a[BP];
+#pragma unroll
+                for (int v = 0; v < BP / AW; ++v) {
+                    const Pack<T, AW> p = *reinterpret_cast<const Pack<T, AW> *>(a_dst + (u * B + r) * BP + v * AW);
+#pragma unroll
+                    for (int e = 0; e < AW; ++e) a[v * AW + e] = p.v[e];
+                }
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) {
+                    T t = a[0] * b[0][c / W].v[c % W];
+#pragma unroll
+                    for (int jj = 1; jj < B; ++jj) t += a[jj] * b[jj][c / W].v[c % W];
+                    acc[r][c] += t;
+                }
+            }
+        }
+    }
+
+    // Column c of every lane: the wave's rows, one run per column of C.
+    const int nr = (int)min((int64_t)NG, sh.mb - R0) * B, ts = NG * B + 1;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        wave_sync();
+        if (grp < NG) {
+#pragma unroll
+            for (int r = 0; r < B; ++r) s_a[sub * ts + grp * B + r] = acc[r][c];
+        }
+        wave_sync();
+        for (int s = 0; s < L; ++s) {
+            if (s * CPL + c >= kk) break;
+            T *const dst = C + R0 * B + (int64_t)(c0 + s * CPL + c) * ldc;
+            for (int r = lane; r < nr; r += 64) {
+                const T v = alpha * s_a[s * ts + r];
+                dst[r] = beta_zero ? v : v + beta * dst[r];
+            }
+        }
+    }
+}
+
+// longest[0] = the longest block-row, longest[1] set where browptr decreases.
+__global__ void block_row_longest_kernel(int64_t mb, const int32_t *__restrict__ browptr, int32_t *__restrict__ longest)
+{
+    int32_t len = 0;
+    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < mb; r += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t d = (int64_t)browptr[r + 1] - browptr[r];
+        if (d < 0) longest[1] = 1;
+        len = max(len, (int32_t)min(d, (int64_t)INT32_MAX));
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) len = max(len, __shfl_xor(len, off, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(longest, len);
+}
+
+__global__ void clear_pair_kernel(int32_t *p)
+{
+    if (threadIdx.x < 2) p[threadIdx.x] = 0;
+}
+
+template <typename T>
+constexpr int MAX_COLS = 16 / (int)sizeof(T);
+
+// Columns per lane: 16 bytes, fewer while a group has less than 4 lanes.
+template <typename T>
+int small_cpl(int64_t k)
+{
+    int c = MAX_COLS<T>;
+    while (c > 1 && (k + c - 1) / c < 4) c /= 2;
+    return c;
+}
+
+template <typename T, int B, int CPL>
+int launch(const SmallShape &base, const int32_t *browptr, const int32_t *bcolind, const T *val, const T *Bt, T alpha,
+           T beta, T *C, int64_t ldc, hipStream_t s)
+{
+    SmallShape sh = base;
+    const int64_t ny = (sh.k + 64 * CPL - 1) / (64 * CPL);
+    sh.cols = (int)(((sh.k + ny - 1) / ny + CPL - 1) / CPL * CPL);
+    // Lanes beyond the columns where a stage would not hold a block otherwise.
+    sh.L = max(sh.cols / CPL, (B * B + BS_STAGE - 1) / BS_STAGE);
+    const int NG = 64 / sh.L;
+    constexpr int V16 = 16 / (int)sizeof(T), AW = B <= 2 ? 2 : V16 < 4 ? 2 : 4, BP = (B + AW - 1) / AW * AW;
+    sh.sb = max(1, min(min(8, sh.L), BS_STAGE * sh.L / (B * B)));
+    // A group's stage starts an odd number of 16-byte units after the last one's.
+    sh.gs = (sh.sb * B * BP + V16 - 1) / V16 * V16;
+    if (sh.gs / V16 % 2 == 0) sh.gs += V16;
+    sh.wave_vals = (max(NG * sh.gs, sh.L * (NG * B + 1)) + V16 - 1) / V16 * V16;
+    sh.wave_stride = (sh.wave_vals + NG * sh.sb * 4 / (int)sizeof(T) + V16) / V16 * V16;
+    const size_t per_wave = sizeof(T) * (size_t)sh.wave_stride;
+    const int64_t wgs = (sh.mb + (int64_t)BS_WAVES * NG - 1) / (BS_WAVES * NG);
+    sh.run = (unsigned)((wgs + 4 * NUM_XCD - 1) / (4 * NUM_XCD));
+    const dim3 grid((unsigned)((wgs + (int64_t)sh.run * NUM_XCD - 1) / ((int64_t)sh.run * NUM_XCD) * sh.run * NUM_XCD),
+                    (unsigned)ny);
+    hipLaunchKernelGGL((bsr_small_spmm_kernel<T, B, CPL>), grid, dim3(BS_BLOCK), per_wave * BS_WAVES, s, sh, browptr,
+                       bcolind, val, Bt, alpha, beta, beta == T(0), C, ldc);
+    return check_launch("bsr_small_spmm_kernel");
+}
+
+template <typename T, int B>
+int launch_cpl(int cpl, const SmallShape &sh, const int32_t *browptr, const int32_t *bcolind, const T *val,
+               const T *Bt, T alpha, T beta, T *C, int64_t ldc, hipStream_t s)
+{
+    constexpr int M = MAX_COLS<T>;
+#define JLUST_CPL(N) \
+    if (cpl == N) return launch<T, B, (N <= M ? N : M)>(sh, browptr, bcolind, val, Bt, alpha, beta, C, ldc, s);
+    JLUST_CPL(4)
+    JLUST_CPL(2)
+#undef JLUST_CPL
+    return launch<T, B, 1>(sh, browptr, bcolind, val, Bt, alpha, beta, C, ldc, s);
+}
+
+}  // namespace
+
+bool bsr_small_shape(int64_t nb, int64_t b1, int64_t b2, int64_t k, size_t tsz)
+{
+    if (b1 != b2 || b1 < 2 || b1 > 8 || k < 2) return false;
+    // Offsets into B's copy are 32-bit.
+    return (uint64_t)(nb * b2 + 1) * (uint64_t)(k + 8) * tsz < 0xff000000ull;
+}
+
+size_t bsr_small_copy_bytes(int64_t nb, int64_t b, int64_t k, size_t tsz)
+{
+    return tsz * (size_t)(nb * b + 1) * (size_t)((k + 7) / 8 * 8);
+}
+
+int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *browptr, hipStream_t s, bool *even)
+{
+    *even = false;
+    if (mb == 0 || nnzb == 0) return JLUST_STATUS_SUCCESS;
+    void *ws = nullptr;
+    if (int st = scratch((jlust_stream_t)s, 64, &ws)) return st;
+    int32_t *d = (int32_t *)ws, h[2] = {0, 0}, ends[2] = {0, 0};
+    hipLaunchKernelGGL(clear_pair_kernel, dim3(1), dim3(64), 0, s, d);
+    hipLaunchKernelGGL(block_row_longest_kernel, dim3((unsigned)min((mb + 255) / 256, (int64_t)512)), dim3(256), 0, s,
+                       mb, browptr, d);
+    if (int st = check_launch("block_row_longest_kernel")) return st;
+    JLUST_HIP_TRY(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
+    JLUST_HIP_TRY(hipMemcpyAsync(&ends[0], browptr, 4, hipMemcpyDeviceToHost, s));
+    JLUST_HIP_TRY(hipMemcpyAsync(&ends[1], browptr + mb, 4, hipMemcpyDeviceToHost, s));
+    JLUST_HIP_TRY(hipStreamSynchronize(s));
+    if (ends[0] != origin || (int64_t)ends[1] - origin != nnzb || h[1]) return JLUST_STATUS_SUCCESS;
+    *even = h[0] <= std::max<int64_t>(64, 4 * nnzb / mb);
+    return JLUST_STATUS_SUCCESS;
+}
+
+template <typename T>
+int bsr_small_spmm(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                   const T *val, int row_major, int64_t k, T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                   T *Bt, hipStream_t s)
+{
+    if (mb == 0 || k == 0) return JLUST_STATUS_SUCCESS;
+    const int cpl = small_cpl<T>(k);
+    SmallShape sh{};
+    sh.mb = mb;
+    sh.k = (int)k;
+    sh.ldt = (k + cpl - 1) / cpl * cpl;
+    sh.origin = origin;
+    sh.row_major = row_major;
+    if (int st = spmm_row_major_copy(sizeof(T) == 8 ? 0 : 1, nb * b, k, B, ldb, Bt, sh.ldt, s)) return st;
+#define JLUST_B(N) \
+    case N: return launch_cpl<T, N>(cpl, sh, browptr, bcolind, val, Bt, alpha, beta, C, ldc, s);
+    switch (b) {
+        JLUST_B(2)
+        JLUST_B(3)
+        JLUST_B(4)
+        JLUST_B(5)
+        JLUST_B(6)
+        JLUST_B(7)
+        JLUST_B(8)
+    }
+#undef JLUST_B
+    return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_small_spmm: block size %lld", (long long)b);
+}
+
+template int bsr_small_spmm<double>(int64_t, int64_t, int64_t, int32_t, const int32_t *, const int32_t *,
+                                    const double *, int, int64_t, double, const double *, int64_t, double, double *,
+                                    int64_t, double *, hipStream_t);
+template int bsr_small_spmm<float>(int64_t, int64_t, int64_t, int32_t, const int32_t *, const int32_t *, const float *,
+                                   int, int64_t, float, const float *, int64_t, float, float *, int64_t, float *,
+                                   hipStream_t);
+
+int preload_bsr_small()
+{
+    JLUST_PRELOAD_KERNEL(block_row_longest_kernel);
+    return JLUST_STATUS_SUCCESS;
+}
+
+}  // namespace jlust

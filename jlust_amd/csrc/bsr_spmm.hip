@@ -2414,9 +2414,11 @@ extern "C" int jlust_hip_bsr_expand_csr_i32(int64_t mb, int64_t b1, int64_t b2, 
 // A prepared BSR SpMM (the analyse-once handle of the C ABI; the cuSPARSE SpMM
 // handle contract, ext/CUDAExt/ops/spmm.jl:8-70, for BSR).  16 x 16 blocks,
 // Float32 or Float64, keep the MFMA kernels and the caller's buffers
-// (update_values swaps the value pointer).  Any other block shape is
-// expanded to CSR once (the plan owns the expansion) and runs through a CSR
-// SpMM plan over it; update_values re-expands the values only, on the stream.
+// (update_values swaps the value pointer), and so do square blocks of 2 to 8
+// rows whose block-rows are of even length (bsr_small.hip; the plan owns the
+// copy of B).  Any other block shape is expanded to CSR once (the plan owns
+// the expansion) and runs through a CSR SpMM plan over it; update_values
+// re-expands the values only, on the stream.
 static size_t bsr_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 struct jlust_bsr_plan {
@@ -2426,8 +2428,8 @@ struct jlust_bsr_plan {
     const int32_t *browptr = nullptr;
     const int32_t *bcolind = nullptr;
     const void *val = nullptr;
-    bool mfma = false;
-    void *mem = nullptr;                // expansion: rowptr | colind | values
+    bool mfma = false, small = false;
+    void *mem = nullptr;                // expansion: rowptr | colind | values; or B's copy (small)
     int32_t *rowptr = nullptr;
     int32_t *colind = nullptr;
     void *cval = nullptr;
@@ -2474,8 +2476,12 @@ static int bsr_spmm_plan_create_body(int64_t mb, int64_t nb, int64_t b1, int64_t
     // blocks need 16-byte aligned values; fp64 takes any alignment).
     p->mfma = b1 == BSR_BS && b2 == BSR_BS &&
               (value_type == 0 || !row_major_blocks || (uintptr_t)val % 16 == 0);
-    if (!p->mfma) {
-        const size_t tsz = value_type == 0 ? sizeof(double) : sizeof(float);
+    const size_t tsz = value_type == 0 ? sizeof(double) : sizeof(float);
+    if (!p->mfma && bsr_small_shape(nb, b1, b2, k, tsz))
+        if (int st = bsr_small_pattern(mb, nnzb, origin, browptr, (hipStream_t)stream, &p->small)) return st;
+    if (p->small) {
+        JLUST_HIP_TRY(hipMalloc(&p->mem, bsr_small_copy_bytes(nb, b1, k, tsz)));
+    } else if (!p->mfma) {
         const size_t nz = (size_t)(total > 0 ? total : 1);
         const size_t sz_rp = bsr_align_up(sizeof(int32_t) * (size_t)(mb * b1 + 1), 256);
         const size_t sz_ci = bsr_align_up(sizeof(int32_t) * nz, 256);
@@ -2520,7 +2526,7 @@ extern "C" int jlust_hip_bsr_spmm_plan_update_values(jlust_bsr_plan_t plan, cons
     if (plan->mfma && plan->value_type == 1 && plan->row_major && (uintptr_t)val % 16 != 0)
         return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_plan_update_values: block values must be 16-byte aligned");
     plan->val = val;
-    if (plan->mfma) return JLUST_STATUS_SUCCESS;     // the kernels read the values in place
+    if (plan->mfma || plan->small) return JLUST_STATUS_SUCCESS;     // the kernels read the values in place
     int dev = 0;
     if (int st = require_device(&dev)) return st;
     if (dev != plan->device)
@@ -2528,6 +2534,85 @@ extern "C" int jlust_hip_bsr_spmm_plan_update_values(jlust_bsr_plan_t plan, cons
                     "bsr_spmm_plan_update_values: plan belongs to device %d, current device is %d", plan->device, dev);
     return bsr_expand_entries(plan->mb, plan->b1, plan->b2, plan->nnzb, plan->origin, plan->browptr, plan->bcolind,
                               val, plan->value_type, plan->row_major, nullptr, plan->cval, (hipStream_t)stream);
+}
+
+// The dense operands of a product on small blocks: the checks of the CSR plan.
+static int bsr_small_dense_args(int64_t m, int64_t n, int64_t k, const void *B, int64_t ldb, const void *C, int64_t ldc)
+{
+    using namespace jlust;
+    if (ldb < (n > 0 ? n : 1) || ldc < (m > 0 ? m : 1))
+        return fail(JLUST_STATUS_INVALID_ARGUMENT,
+                    "bsr_spmm: leading dimensions too small (ldb=%lld < %lld or ldc=%lld < %lld)", (long long)ldb,
+                    (long long)n, (long long)ldc, (long long)m);
+    if (bad_ptr(B, n * k) || bad_ptr(C, m * k))
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm: null device pointer");
+    return JLUST_STATUS_SUCCESS;
+}
+
+template <typename T>
+static int bsr_small_execute(jlust_bsr_plan_t p, T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                             jlust_stream_t stream)
+{
+    using namespace jlust;
+    if (int st = bsr_small_dense_args(p->mb * p->b1, p->nb * p->b2, p->k, B, ldb, C, ldc)) return st;
+    int dev = 0;
+    if (int st = require_device(&dev)) return st;
+    if (dev != p->device)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT,
+                    "bsr_spmm_plan_execute: plan belongs to device %d, current device is %d", p->device, dev);
+    return bsr_small_spmm<T>(p->mb, p->nb, p->b1, p->origin, p->browptr, p->bcolind, (const T *)p->val, p->row_major,
+                             p->k, alpha, B, ldb, beta, C, ldc, (T *)p->mem, (hipStream_t)stream);
+}
+
+template <typename T>
+static int bsr_small_call(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_t nnzb, int32_t origin,
+                          const int32_t *browptr, const int32_t *bcolind, const T *val, int row_major_blocks, int64_t k,
+                          T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, jlust_stream_t stream,
+                          int32_t *taken)
+{
+    using namespace jlust;
+    clear_error();
+    if (!taken) return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_small: null taken");
+    *taken = 0;
+    if (mb < 0 || nb < 0 || b1 <= 0 || b2 <= 0 || nnzb < 0 || k < 0)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_small: negative extent or block size");
+    if (int st = check_origin(origin)) return st;
+    if (mb * b1 >= INT32_MAX || nb * b2 >= INT32_MAX || nnzb * b1 * b2 >= (int64_t)INT32_MAX - 1)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_small: extents exceed the Int32 index range");
+    if ((mb > 0 && !browptr) || bad_ptr(bcolind, nnzb) || bad_ptr(val, nnzb))
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_small: null device pointer");
+    if (int st = require_device(nullptr)) return st;
+    if (!bsr_small_shape(nb, b1, b2, k, sizeof(T))) return JLUST_STATUS_SUCCESS;
+    hipStream_t s = (hipStream_t)stream;
+    bool even = false;
+    if (int st = bsr_small_pattern(mb, nnzb, origin, browptr, s, &even)) return st;
+    if (!even) return JLUST_STATUS_SUCCESS;
+    if (int st = bsr_small_dense_args(mb * b1, nb * b2, k, B, ldb, C, ldc)) return st;
+    void *Bt = nullptr;
+    if (int st = scratch(stream, bsr_small_copy_bytes(nb, b1, k, sizeof(T)), &Bt)) return st;
+    *taken = 1;
+    return bsr_small_spmm<T>(mb, nb, b1, origin, browptr, bcolind, val, row_major_blocks ? 1 : 0, k, alpha, B, ldb,
+                             beta, C, ldc, (T *)Bt, s);
+}
+
+extern "C" int jlust_hip_bsr_spmm_small_f64_i32(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_t nnzb,
+                                                int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                                                const double *val, int row_major_blocks, int64_t k, double alpha,
+                                                const double *B, int64_t ldb, double beta, double *C, int64_t ldc,
+                                                jlust_stream_t stream, int32_t *taken)
+{
+    return bsr_small_call<double>(mb, nb, b1, b2, nnzb, origin, browptr, bcolind, val, row_major_blocks, k, alpha, B,
+                                  ldb, beta, C, ldc, stream, taken);
+}
+
+extern "C" int jlust_hip_bsr_spmm_small_f32_i32(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_t nnzb,
+                                                int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                                                const float *val, int row_major_blocks, int64_t k, float alpha,
+                                                const float *B, int64_t ldb, float beta, float *C, int64_t ldc,
+                                                jlust_stream_t stream, int32_t *taken)
+{
+    return bsr_small_call<float>(mb, nb, b1, b2, nnzb, origin, browptr, bcolind, val, row_major_blocks, k, alpha, B,
+                                 ldb, beta, C, ldc, stream, taken);
 }
 
 extern "C" int jlust_hip_bsr_spmm_plan_execute_f32(jlust_bsr_plan_t plan, float alpha, const float *B, int64_t ldb,
@@ -2538,6 +2623,7 @@ extern "C" int jlust_hip_bsr_spmm_plan_execute_f32(jlust_bsr_plan_t plan, float 
     if (!plan) return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_plan_execute: null plan");
     if (plan->value_type != 1)
         return fail(JLUST_STATUS_UNSUPPORTED_VALUE_TYPE, "bsr_spmm_plan_execute: plan was created for Float64 values");
+    if (plan->small) return bsr_small_execute<float>(plan, alpha, B, ldb, beta, C, ldc, stream);
     if (!plan->mfma)
         return jlust_hip_csr_spmm_plan_execute_f32(plan->csr, alpha, B, ldb, beta, C, ldc, 0, stream);
     return bsr_spmm(plan->mb, plan->nb, BSR_BS, plan->nnzb, plan->origin, plan->browptr, plan->bcolind,
@@ -2552,6 +2638,7 @@ extern "C" int jlust_hip_bsr_spmm_plan_execute_f64(jlust_bsr_plan_t plan, double
     if (!plan) return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_plan_execute: null plan");
     if (plan->value_type != 0)
         return fail(JLUST_STATUS_UNSUPPORTED_VALUE_TYPE, "bsr_spmm_plan_execute: plan was created for Float32 values");
+    if (plan->small) return bsr_small_execute<double>(plan, alpha, B, ldb, beta, C, ldc, stream);
     if (!plan->mfma)
         return jlust_hip_csr_spmm_plan_execute_f64(plan->csr, alpha, B, ldb, beta, C, ldc, 0, stream);
     return bsr_spmm_f64(plan->mb, plan->nb, BSR_BS, plan->nnzb, plan->origin, plan->browptr, plan->bcolind,
@@ -2562,7 +2649,7 @@ extern "C" int jlust_hip_bsr_spmm_plan_info(jlust_bsr_plan_t plan, int32_t *path
 {
     jlust::clear_error();
     if (!plan) return jlust::fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_plan_info: null plan");
-    if (path) *path = plan->mfma ? 0 : 1;
+    if (path) *path = plan->mfma ? 0 : plan->small ? 2 : 1;
     return JLUST_STATUS_SUCCESS;
 }
 

@@ -121,6 +121,23 @@ int perm_gather(int value_type, int64_t nnz, const int32_t *perm, const void *sr
 // update_values.
 int spmm_plan_adopt_reorder(jlust_spmm_plan_t plan, void *mem, const int32_t *perm, void *val_copy);
 
+// Bt[j*ldt + c] = B[j + c*ldb] for j < n, c < k, and a row n of zeros
+// (spmm.hip); value_type 0 = f64, 1 = f32.  Bt holds (n + 1) * ldt values.
+int spmm_row_major_copy(int value_type, int64_t n, int64_t k, const void *B, int64_t ldb, void *Bt, int64_t ldt,
+                        hipStream_t s);
+
+// BSR SpMM on small square blocks (bsr_small.hip): whether a shape is one of
+// its; the bytes of B's copy (Bt); whether browptr runs from the origin to
+// nnzb + origin without decreasing and has no block-row much longer than the
+// others (*even; synchronises s); the product.
+bool bsr_small_shape(int64_t nb, int64_t b1, int64_t b2, int64_t k, size_t tsz);
+size_t bsr_small_copy_bytes(int64_t nb, int64_t b, int64_t k, size_t tsz);
+int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *browptr, hipStream_t s, bool *even);
+template <typename T>
+int bsr_small_spmm(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                   const T *val, int row_major, int64_t k, T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                   T *Bt, hipStream_t s);
+
 // ---------------------------------------------------------------- preload
 
 // The runtime loads a translation unit's device code on the first launch of
@@ -137,6 +154,7 @@ int preload_convert(hipStream_t s);
 int preload_spmm();
 int preload_sddmm();
 int preload_bsr();
+int preload_bsr_small();
 int preload_coo_spmv();
 int preload_coo_csc();
 int preload_assemble();

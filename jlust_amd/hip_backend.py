@@ -533,6 +533,22 @@ def _spmm(u_A: USTensor, u_B: USTensor, u_C: USTensor, alpha, beta, skip_empty_r
     if is_bsr(u_A.format):
         b1, b2, row_major, browptr, bcolind, mb, nb = _bsr_parts(u_A)
         if (b1, b2) != (16, 16) or (suf == "f32" and row_major and nonzeros(u_A).data_ptr() % 16):
+            if b1 == b2 and b1 <= 8 and not skip_empty_rows:
+                # Small square blocks as stored, unless the library leaves the
+                # pattern to the expansion.
+                v = nonzeros(u_A)
+                if not v.is_contiguous():
+                    raise NonCanonicalStorage("value buffers must be contiguous")
+                dev = _check_same_device(browptr, bcolind, v, B, C)
+                taken = ctypes.c_int32(0)
+                with _on(dev):
+                    st = getattr(L, f"jlust_hip_bsr_spmm_small_{suf}_i32")(
+                        mb, nb, b1, b2, bcolind.numel(), u_A.origin.offset, _ptr(browptr), _ptr(bcolind), _ptr(v),
+                        int(row_major), k, float(alpha), _ptr(B), leading_dim(B), float(beta), _ptr(C),
+                        leading_dim(C), _stream(dev), ctypes.byref(taken))
+                _lib.check(st, "bsr_spmm_small", u_A.format, _BE, T)
+                if taken.value:
+                    return u_C
             # Blocks other than 16 x 16 (the MFMA kernels serve 16 x 16 blocks
             # only), and fp32 row-major blocks whose values are not 16-byte
             # aligned (the fp32 MFMA kernels load a block row as one float4):
@@ -1472,8 +1488,9 @@ class HIPBSRSpMMHandle(AbstractKernelHandle):
     """Prepared BSR SpMM (jlust_hip_bsr_spmm_plan_*): prepare(HIPBackend(),
     SpMMOp, A::BSR; n_cols=k) -> execute(h, B, C) -> update_values!(h, A), the
     cuSPARSE SpMM handle contract (ext/CUDAExt/ops/spmm.jl:8-70) for BSR.
-    16 x 16 blocks run the MFMA kernels (fp32 or fp64) on A's buffers; any
-    other block shape is expanded to CSR once and runs through a CSR SpMM
+    16 x 16 blocks run the MFMA kernels (fp32 or fp64) on A's buffers, square
+    blocks of 2 to 8 rows in block-rows of even length a kernel of their own;
+    any other block shape is expanded to CSR once and runs through a CSR SpMM
     plan over the expansion.  A's values are read as they are at the
     call: on the expansion path, values written in place through torch since
     the plan last read them (the value tensor's version counter moved) are
@@ -1565,13 +1582,14 @@ class HIPBSRSpMMHandle(AbstractKernelHandle):
         return self
 
     def info(self) -> dict:
-        """The path the plan chose: "mfma" or "csr_expansion"."""
+        """The path the plan chose: "mfma", "blocks" (small square blocks as
+        stored) or "csr_expansion"."""
         if not self._plan.value:
             return {}
         path = ctypes.c_int32()
         st = _lib.lib().jlust_hip_bsr_spmm_plan_info(self._plan, ctypes.byref(path))
         _lib.check(st, "bsr_spmm_plan_info", self.u_A.format, _BE, self.T)
-        return {"path": "mfma" if path.value == 0 else "csr_expansion"}
+        return {"path": ("mfma", "csr_expansion", "blocks")[path.value]}
 
     def _destroy(self):
         plan, self._plan = getattr(self, "_plan", None), ctypes.c_void_p(0)

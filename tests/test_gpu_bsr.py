@@ -639,3 +639,47 @@ def test_bsr_long_rows_two_halves(J, O, k, beta):
     rp, ci, v = O.bsr_to_csr(browptr, bcolind, val, 16)
     absref = O.csr_spmm_absref(rp, ci, v, B, 0.75, beta, C0)
     assert_within(C, ref, absref, np.float32, f"long rows k={k} beta={beta}")
+
+
+@pytest.mark.parametrize("row_major", [True, False])
+@pytest.mark.parametrize("b", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_bsr_small_blocks(J, O, dtype, b, row_major):
+    """Square blocks of 2 to 8 rows as stored: widths at the edges of a lane's
+    columns and of a wave's, block-rows of 0 to 40 blocks (several stages),
+    values at an odd offset, padded leading dimensions, alpha and beta; exact on
+    integers, the plan equal to the plain call.  A block-row far longer than the
+    others goes through the expansion, with the same result."""
+    import torch
+    tdt = torch.float64 if dtype == np.float64 else torch.float32
+    rng = np.random.default_rng(10 * b + row_major)
+    for k, long_row in ((2, 0), (3, 0), (7, 0), (8, 0), (13, 0), (24, 0), (65, 0), (130, 0), (300, 0), (24, 200)):
+        mb, nb = (70, 250) if k < 100 else (9, 250)
+        counts = rng.integers(0, 6, mb)
+        counts[mb // 2], counts[0], counts[-1] = 40, 0, 33
+        if long_row:
+            counts[3] = long_row
+        bc = np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in counts]) + 1
+        bp = (np.r_[0, np.cumsum(counts)] + 1).astype(np.int32)
+        bc = bc.astype(np.int32)
+        flat = rng.integers(-4, 5, bc.size * b * b).astype(dtype)
+        vals = torch.empty(flat.size + 1, dtype=tdt, device="cuda")[1:]
+        vals.copy_(dev(flat))
+        A = J.bsr_tensor(dev(bp), dev(bc), vals, (mb * b, nb * b), (b, b), row_major)
+        B = np.asfortranarray(rng.integers(-3, 4, (nb * b, k)).astype(dtype))
+        C0 = np.asfortranarray(rng.integers(-3, 4, (mb * b, k)).astype(dtype))
+        Bd = torch.zeros((k, nb * b + 3), dtype=tdt, device="cuda").t()[1:nb * b + 1]
+        Bd.copy_(dev(B))
+        whole = torch.full((k, mb * b + 5), 7.0, dtype=tdt, device="cuda").t()
+        C = whole[3:mb * b + 3]
+        C.copy_(dev(C0))
+        J.execute(J.SpMMOp, A, Bd, C, alpha=2.0, beta=-1.0)
+        ref = O.bsr_spmm(bp, bc, flat, b, B, 2.0, -1.0, C0.copy(order="F"), row_major_blocks=row_major, b2=b)
+        np.testing.assert_array_equal(host(C), ref, err_msg=f"k={k}")
+        assert (whole[:3] == 7).all() and (whole[mb * b + 3:] == 7).all()
+        h = J.prepare(J.HIPBackend(), J.SpMMOp, A, n_cols=k)
+        assert h.info()["path"] == ("csr_expansion" if long_row else "blocks"), (k, long_row)
+        C2 = J.dense_matrix(mb * b, k, dtype=tdt, fill=float("nan"))
+        J.execute(h, Bd, C2)
+        ref = O.bsr_spmm(bp, bc, flat, b, B, 1.0, 0.0, C0.copy(order="F"), row_major_blocks=row_major, b2=b)
+        np.testing.assert_array_equal(host(C2), ref, err_msg=f"plan k={k}")
