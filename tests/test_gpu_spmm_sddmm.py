@@ -385,3 +385,51 @@ def test_sddmm_k_beyond_lds(J, O, mask_kind, dtype, K):
             h = J.prepare(J.HIPBackend(), J.SDDMMOp, Cs, n_inner=K)
             J.execute(J.SDDMMOp, h, dev(A), dev(Bm), Cs, alpha=0.5, beta=1.5)
         assert_within(host(cv), ref[perm], absref[perm], dtype, f"{mask_kind} {how} K={K}")
+
+
+@pytest.mark.parametrize("pad", [0, 1, 4])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_sddmm_every_width(J, O, dtype, pad):
+    """K at every edge of a lane's vector and a group's steps, columns of B at
+    any alignment (pad), as CSR, COO and CSC masks, plain and prepared; a
+    column of B that is not finite reaches only its entries."""
+    import torch
+    rng = np.random.default_rng(pad)
+    m, n = 300, 250
+    rowptr, colind, _ = random_csr(m, n, lengths=np.r_[0, rng.integers(0, 12, m - 2), 240], seed=pad, dtype=dtype)
+    nnz = colind.size
+    tdt = torch.float64 if dtype == np.float64 else torch.float32
+    rows = np.repeat(np.arange(m), np.diff(rowptr))
+    perm = rng.permutation(nnz)
+    order = np.lexsort((rows, colind))
+    colptr = (np.r_[0, np.cumsum(np.bincount(colind - 1, minlength=n))] + 1).astype(np.int32)
+    bad = int(colind[nnz // 2]) - 1
+    masks = {"csr": (np.arange(nnz), lambda v: J.csr_tensor(dev(rowptr), dev(colind), v, (m, n))),
+             "coo": (perm, lambda v: J.coo_tensor(dev((rows[perm] + 1).astype(np.int32)), dev(colind[perm]), v, (m, n))),
+             "csc": (order, lambda v: J.csc_tensor(dev(colptr), dev((rows[order] + 1).astype(np.int32)), v, (m, n)))}
+    for K in (1, 2, 3, 4, 5, 6, 7, 8, 9, 15, 16, 17, 31, 33, 50, 63, 65, 79, 95, 96, 97, 100, 111, 112, 113, 127, 128,
+              129, 161, 193, 225, 255, 257):
+        A = np.asfortranarray(rng.standard_normal((m, K)).astype(dtype))
+        B = np.asfortranarray(rng.standard_normal((K, n)).astype(dtype))
+        Bbad = B.copy(order="F")
+        Bbad[:, bad] = np.inf
+        ref = O.csr_sddmm(rowptr, colind, A, B, 0.5, 0.0, np.zeros(nnz, dtype), None)
+        absref = O.csr_sddmm_absref(rowptr, colind, A, B, 0.5, 0.0, np.zeros(nnz, dtype), None)
+        Bd = torch.empty((n, K + pad), dtype=tdt, device="cuda").fill_(float("nan")).t()[:K]
+        Bd.copy_(dev(B))
+        Bbd = torch.empty((n, K + pad), dtype=tdt, device="cuda").fill_(float("nan")).t()[:K]
+        Bbd.copy_(dev(Bbad))
+        for name, (sel, make) in masks.items():
+            for call in ("plain", "plan"):
+                C = make(torch.full((nnz,), float("nan"), dtype=tdt, device="cuda"))
+                h = J.prepare(J.HIPBackend(), J.SDDMMOp, C, n_inner=K) if call == "plan" else None
+                run = (lambda b: J.execute(h, dev(A), b, alpha=0.5)) if h else \
+                    (lambda b: J.execute(J.SDDMMOp, dev(A), b, C, alpha=0.5))
+                run(Bd)
+                got = host(J.nonzeros(C)).copy()
+                assert_within(got, ref[sel], absref[sel], dtype, f"{name} {call} K={K}")
+                run(Bbd)
+                hit = (colind - 1 == bad)[sel]
+                gbad = host(J.nonzeros(C))
+                np.testing.assert_array_equal(gbad[~hit], got[~hit], err_msg=f"{name} {call} K={K}")
+                assert not np.isfinite(gbad[hit]).any()
