@@ -745,8 +745,10 @@ int jlust_hip_bsr_spmm_f64_i32(int64_t mb, int64_t nb, int64_t bs,
  * y = alpha*A*x + beta*y for BSR of any b1 x b2 block shape (A (mb*b1) x
  * (nb*b2), storage as for jlust_hip_bsr_spmm_f32_i32 with bs = b1 x b2
  * blocks).  The reference's EmitterBackend claims SpMV for every sparse
- * format (KernelAbstractionsExt.jl:31-37).  Each scalar row sums its entries
- * in the order of its row in the CSR expansion below.  Block ranges and block
+ * format (KernelAbstractionsExt.jl:31-37).  A block-row's sum is made of
+ * partial sums added in storage order, the same on every call (segments of at
+ * most 32 blocks; square blocks of 2 to 8 rows: runs of 1024 / b rows and
+ * blocks).  Block ranges and block
  * columns are clamped to the stored blocks and to [0, nb), so a malformed
  * browptr or bcolind gives wrong sums, never an out-of-bounds read; they are
  * not validated here (the expansion validates browptr's ends).
@@ -853,9 +855,8 @@ int jlust_hip_bsr_spmm_plan_destroy(jlust_bsr_plan_t plan);
  * (ext/KernelAbstractionsExt/ops/spmv.jl:518-544, the handle execute(h, x, y)
  * and update_values! run on; the reference analyses nothing for it).  Any
  * block shape, either block order, Float64 or Float32 (value_type 0 / 1).
- * create builds the segment table of jlust_hip_bsr_spmv_*_i32 once (block-
- * rows cut into segments of at most 32 blocks; the plan owns it and the
- * per-segment sums) and synchronises `stream`; it reads browptr's ends back
+ * create builds the table of jlust_hip_bsr_spmv_*_i32's segments or runs once
+ * (the plan owns it and their partial sums) and synchronises `stream`; it reads browptr's ends back
  * and returns JLUST_STATUS_NONCANONICAL_STORAGE unless they are origin and
  * nnzb + origin.  execute: y = alpha*A*x + beta*y (beta == 0: y write-only),
  * stream-ordered; one plan must not run on two streams at once (the partial

@@ -1902,6 +1902,226 @@ __global__ __launch_bounds__(256) void bsr16_spmv_seg_kernel(int64_t mb, int64_t
     }
 }
 
+// Square blocks of 2 to 8 rows: the matrix as one list of items -- a row
+// start, then that row's blocks, item browptr[R] + R being the start of
+// block-row R -- cut into runs of BSRMV_ITEMS(b), a workgroup each, so that
+// long rows, short ones and empty ones cost what they hold (an equal share of
+// the blocks alone would leave a stretch of empty rows to one workgroup).
+// bsr_spmv_starts_kernel finds each run's first row; a run's blocks then
+// follow from that row's number.
+//
+// What bounds it: the values, once (8 TB/s nominal).  A thread takes row r of
+// one block, so that a wave's loads cover one stretch of the values in either
+// order of the blocks, and holds BSRMV_M of them in flight.  (A thread per
+// scalar row, as for the other shapes below, reads at the distance of a
+// segment, one block at a time.  Mesh of 101,520 nodes, 27 blocks of 3 x 3
+// f64 a row, 209 MB: residual 134.5 us with the segments, 46.8 with the runs;
+// 60,680 nodes, f64, plain calls, 2 / 4 / 8 rows a block: 37 / 59 / 373 to
+// 30 / 41 / 151 us row-major, 37 / 59 / 235 to 31 / 41 / 152 column-major.)
+// The blocks' sums go to LDS, and a thread per scalar row adds them in storage
+// order over four partial sums.  A row that ends in a later run leaves its
+// part in tail[run], each run that goes on with a row begun before it leaves
+// carry[run], and a second kernel adds those in order: the same sums on every
+// call.
+constexpr int BSRMV_M = 4;                 // rows of blocks per thread
+template <int B> constexpr int BSRMV_ITEMS = 256 * BSRMV_M / B;
+
+int64_t bsr_spmv_run_items(int64_t b) { return 256 * BSRMV_M / b; }
+int64_t bsr_spmv_runs(int64_t mb, int64_t nnzb, int64_t b)
+{
+    const int64_t t = bsr_spmv_run_items(b);
+    return (mb + nnzb + t - 1) / t;
+}
+bool bsr_spmv_is_square_small(int64_t b1, int64_t b2) { return b1 == b2 && b1 >= 2 && b1 <= 8; }
+
+// first[w] = the first block-row whose start is at item w * items or later
+// (first[nruns] = mb).  A canonical browptr sets each of them once; every
+// reader clamps what it reads.
+__global__ __launch_bounds__(256) void bsr_spmv_starts_kernel(int64_t mb, int64_t nnzb, int32_t origin,
+                                                              const int32_t *__restrict__ browptr, int64_t items,
+                                                              int64_t nruns, int32_t *__restrict__ first)
+{
+    const int64_t R = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (R > mb) return;
+    auto at = [&](int64_t i) { return min(max((int64_t)browptr[i] - origin, (int64_t)0), nnzb) + i; };
+    // The runs that start after row R - 1's start and no later than row R's.
+    const int64_t w0 = R == 0 ? 0 : at(R - 1) / items + 1;
+    const int64_t w1 = R == mb ? nruns : min(at(R) / items, nruns);
+    for (int64_t w = w0; w <= w1; ++w) first[w] = (int32_t)R;
+}
+
+template <typename T, int B, bool RM>
+__global__ __launch_bounds__(256) void bsr_spmv_items_kernel(int64_t mb, int64_t nb, int64_t nnzb, int32_t origin,
+                                                             const int32_t *__restrict__ browptr,
+                                                             const int32_t *__restrict__ bcolind,
+                                                             const T *__restrict__ val, T alpha,
+                                                             const T *__restrict__ x, T beta, T *__restrict__ y,
+                                                             const int32_t *__restrict__ first,
+                                                             T *__restrict__ carry, T *__restrict__ tail)
+{
+    constexpr int ITEMS = BSRMV_ITEMS<B>;
+    __shared__ T part[ITEMS * B];
+    const int64_t w = blockIdx.x, d0 = w * ITEMS, d1 = min(d0 + ITEMS, mb + nnzb);
+    const int64_t R0 = min(max((int64_t)first[w], (int64_t)0), mb);
+    const int64_t R1 = min(max((int64_t)first[w + 1], R0), mb);
+    const int64_t q0 = min(max(d0 - R0, (int64_t)0), nnzb);
+    const int64_t q1 = min(max(d1 - R1, q0), min(q0 + ITEMS, nnzb));
+    const int n = (int)(q1 - q0) * B, tid = threadIdx.x;
+    T vv[BSRMV_M][B], xx[BSRMV_M][B];
+    int32_t col[BSRMV_M];
+    auto at = [&](int u) { return min(tid + 256 * u, n - 1); };    // threads past the end: the last row again
+    if (n > 0) {
+#pragma unroll
+        for (int u = 0; u < BSRMV_M; ++u) col[u] = bcolind[q0 + at(u) / B];
+#pragma unroll
+        for (int u = 0; u < BSRMV_M; ++u) {
+            const int r = at(u) % B;
+            const T *v = val + (q0 + at(u) / B) * (B * B);
+            if (RM) {
+                __builtin_memcpy(vv[u], v + r * B, sizeof(vv[u]));
+            } else {
+#pragma unroll
+                for (int s = 0; s < B; ++s) vv[u][s] = v[s * B + r];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < BSRMV_M; ++u)
+            __builtin_memcpy(xx[u], x + min(max((int64_t)col[u] - origin, (int64_t)0), nb - 1) * B, sizeof(xx[u]));
+    }
+    // The pointers of this thread's first row, on their way meanwhile.
+    auto start = [&](int64_t R) { return min(max((int64_t)browptr[R] - origin, q0), q1); };
+    const int64_t nrows = R1 - R0;
+    const int64_t mine = min(R0 + tid / B, mb);
+    const int64_t p0 = browptr[mine], p1 = browptr[min(mine + 1, mb)];
+    const int64_t c1 = R0 > 0 ? start(R0) : q0;          // blocks of the row before
+#pragma unroll
+    for (int u = 0; u < BSRMV_M; ++u) {
+        const int i = tid + 256 * u;
+        if (i < n) {
+            T acc = T(0);
+#pragma unroll
+            for (int s = 0; s < B; ++s) acc += vv[u][s] * xx[u][s];
+            part[i] = acc;
+        }
+    }
+    __syncthreads();
+    // Blocks a to b of the run, row r of each: four sums, then one.
+    auto sum = [&](int64_t a, int64_t b, int r) {
+        T acc[4] = {T(0), T(0), T(0), T(0)};
+        const T *p = part + (a - q0) * B + r;
+        int k = (int)(b - a);
+        for (; k >= 8; k -= 8, p += 8 * B) {
+            T t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t[u] = p[u * B];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc[u & 3] += t[u];
+        }
+        for (; k > 0; --k, p += B) acc[k & 3] += *p;
+        return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    };
+    for (int64_t t = tid; t < nrows * B; t += 256) {
+        const int64_t R = R0 + t / B;
+        const int r = (int)(t % B);
+        const int64_t b0 = t == tid ? p0 : browptr[R], b1 = t == tid ? p1 : browptr[R + 1];
+        const int64_t a = min(max(b0 - origin, q0), q1), e = min(max(b1 - origin, a), q1);
+        const T acc = sum(a, e, r);
+        if (b1 - origin > q1) {
+            if (R == R1 - 1) tail[w * B + r] = acc;
+        } else {
+            T *yr = y + R * B + r;
+            *yr = beta == T(0) ? alpha * acc : alpha * acc + beta * *yr;
+        }
+    }
+    // A row begun in an earlier run: the last B threads, which have no row of
+    // their own unless the run's rows are mostly empty.
+    if (tid >= 256 - B && c1 > q0) carry[w * B + tid - (256 - B)] = sum(q0, c1, tid - (256 - B));
+}
+
+// y of the rows that go over several runs: the run of the row's start and the
+// runs after it, in order.
+template <typename T>
+__global__ __launch_bounds__(256) void bsr_spmv_runs_fix_kernel(int64_t mb, int64_t nnzb, int64_t B, int32_t origin,
+                                                                const int32_t *__restrict__ browptr, int64_t items,
+                                                                int64_t nruns, const int32_t *__restrict__ first,
+                                                                const T *__restrict__ carry,
+                                                                const T *__restrict__ tail, T alpha, T beta,
+                                                                T *__restrict__ y)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t w = t / B, r = t % B;
+    if (w >= nruns) return;
+    const int64_t R0 = min(max((int64_t)first[w], (int64_t)0), mb);
+    const int64_t R1 = min(max((int64_t)first[w + 1], R0), mb);
+    if (R1 == R0) return;
+    const int64_t end = min((int64_t)browptr[R1] - origin, nnzb) + R1 - 1;   // the row's last item
+    const int64_t w1 = min(end / items, nruns - 1);
+    if (w1 <= w) return;
+    T acc = tail[w * B + r];
+    int64_t k = w + 1;
+    for (; k + 8 <= w1 + 1; k += 8) {
+        T p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p[u] = carry[(k + u) * B + r];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc += p[u];
+    }
+    for (; k <= w1; ++k) acc += carry[k * B + r];
+    T *yr = y + (R1 - 1) * B + r;
+    *yr = beta == T(0) ? alpha * acc : alpha * acc + beta * *yr;
+}
+
+int bsr_spmv_starts(int64_t mb, int64_t nnzb, int64_t b, int32_t origin, const int32_t *browptr, int32_t *first,
+                    jlust_stream_t stream)
+{
+    hipLaunchKernelGGL(bsr_spmv_starts_kernel, dim3((unsigned)(mb / 256 + 1)), dim3(256), 0, (hipStream_t)stream, mb,
+                       nnzb, origin, browptr, bsr_spmv_run_items(b), bsr_spmv_runs(mb, nnzb, b), first);
+    return check_launch("bsr_spmv_starts_kernel");
+}
+
+template <typename T, int B>
+void bsr_spmv_items_launch(int64_t mb, int64_t nb, int64_t nnzb, int32_t origin, const int32_t *browptr,
+                           const int32_t *bcolind, const T *val, int row_major_blocks, T alpha, const T *x, T beta,
+                           T *y, const int32_t *first, T *carry, T *tail, int64_t nruns, hipStream_t s)
+{
+    if (row_major_blocks)
+        hipLaunchKernelGGL((bsr_spmv_items_kernel<T, B, true>), dim3((unsigned)nruns), dim3(256), 0, s, mb, nb, nnzb,
+                           origin, browptr, bcolind, val, alpha, x, beta, y, first, carry, tail);
+    else
+        hipLaunchKernelGGL((bsr_spmv_items_kernel<T, B, false>), dim3((unsigned)nruns), dim3(256), 0, s, mb, nb,
+                           nnzb, origin, browptr, bcolind, val, alpha, x, beta, y, first, carry, tail);
+}
+
+// The product over first (nruns + 1 rows); part holds 2 * nruns * b sums.
+template <typename T>
+int bsr_spmv_items(int64_t mb, int64_t nb, int64_t b, int64_t nnzb, int32_t origin, const int32_t *browptr,
+                   const int32_t *bcolind, const T *val, int row_major_blocks, T alpha, const T *x, T beta, T *y,
+                   const int32_t *first, T *part, jlust_stream_t stream)
+{
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t nruns = bsr_spmv_runs(mb, nnzb, b);
+    T *carry = part, *tail = part + nruns * b;
+#define JLUST_BSRMVI(B)                                                                                  \
+    case B:                                                                                              \
+        bsr_spmv_items_launch<T, B>(mb, nb, nnzb, origin, browptr, bcolind, val, row_major_blocks, alpha, x, beta, \
+                                    y, first, carry, tail, nruns, s);                                    \
+        break
+    switch (b) {
+        JLUST_BSRMVI(2);
+        JLUST_BSRMVI(3);
+        JLUST_BSRMVI(4);
+        JLUST_BSRMVI(5);
+        JLUST_BSRMVI(6);
+        JLUST_BSRMVI(7);
+        JLUST_BSRMVI(8);
+    }
+#undef JLUST_BSRMVI
+    if (int st = check_launch("bsr_spmv_items_kernel")) return st;
+    hipLaunchKernelGGL(bsr_spmv_runs_fix_kernel<T>, dim3((unsigned)((nruns * b + 255) / 256)), dim3(256), 0, s, mb,
+                       nnzb, b, origin, browptr, bsr_spmv_run_items(b), nruns, first, carry, tail, alpha, beta, y);
+    return check_launch("bsr_spmv_runs_fix_kernel");
+}
+
 // Blocks of any other shape: a thread per (segment, scalar row), blocks in
 // storage order and each block's row in column order, as bsr_spmv_kernel
 // (a block-row of one segment gets that kernel's sum).
@@ -2040,6 +2260,17 @@ int bsr_spmv_segments(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_t nn
                       const int32_t *browptr, const int32_t *bcolind, const T *val, int row_major_blocks, T alpha,
                       const T *x, T beta, T *y, jlust_stream_t stream)
 {
+    if (bsr_spmv_is_square_small(b1, b2)) {
+        // Scratch: first (nruns + 1), then carry and tail.
+        const int64_t nruns = bsr_spmv_runs(mb, nnzb, b1);
+        const size_t off = ((size_t)(nruns + 1) * sizeof(int32_t) + 255) / 256 * 256;
+        void *ws = nullptr;
+        if (int st = scratch(stream, off + (size_t)(2 * nruns * b1) * sizeof(T), &ws)) return st;
+        int32_t *first = (int32_t *)ws;
+        if (int st = bsr_spmv_starts(mb, nnzb, b1, origin, browptr, first, stream)) return st;
+        return bsr_spmv_items<T>(mb, nb, b1, nnzb, origin, browptr, bcolind, val, row_major_blocks, alpha, x, beta,
+                                 y, first, (T *)((char *)ws + off), stream);
+    }
     // Scratch: the scan's own part, then segstart (mb + 1), segrow (nsegmax),
     // part (b1 sums per segment).
     const int64_t nsegmax = bsr_spmv_nsegmax(mb, nnzb);
@@ -2678,7 +2909,7 @@ struct jlust_bsr_spmv_plan {
     const int32_t *bcolind = nullptr;
     const void *val = nullptr;
     void *mem = nullptr;                // segstart | segrow | partial sums
-    int32_t *segstart = nullptr;
+    int32_t *segstart = nullptr;        // or the runs' first rows
     int32_t *segrow = nullptr;
     void *part = nullptr;
 };
@@ -2732,15 +2963,20 @@ static int bsr_spmv_plan_create_body(int64_t mb, int64_t nb, int64_t b1, int64_t
                         "bsr_spmv_plan_create: browptr runs from %d to %d, expected %d to %lld", ends[0], ends[1],
                         origin, (long long)(nnzb + origin));
         const size_t tsz = value_type == 0 ? sizeof(double) : sizeof(float);
-        p->nsegmax = bsr_spmv_nsegmax(mb, nnzb);
-        const size_t sz_st = bsr_align_up(sizeof(int32_t) * (size_t)(mb + 1), 256);
-        const size_t sz_rw = bsr_align_up(sizeof(int32_t) * (size_t)p->nsegmax, 256);
-        JLUST_HIP_TRY(hipMalloc(&p->mem, sz_st + sz_rw + bsr_align_up(tsz * (size_t)(p->nsegmax * b1), 256)));
+        // The segment table, or the runs' first rows (square blocks of 2 to 8
+        // rows: nsegmax runs of two sums a row, in segstart alone).
+        const bool small = bsr_spmv_is_square_small(b1, b2);
+        p->nsegmax = small ? bsr_spmv_runs(mb, nnzb, b1) : bsr_spmv_nsegmax(mb, nnzb);
+        const size_t sz_st = bsr_align_up(sizeof(int32_t) * (size_t)((small ? p->nsegmax : mb) + 1), 256);
+        const size_t sz_rw = small ? 0 : bsr_align_up(sizeof(int32_t) * (size_t)p->nsegmax, 256);
+        JLUST_HIP_TRY(hipMalloc(&p->mem, sz_st + sz_rw +
+                                             bsr_align_up(tsz * (size_t)(p->nsegmax * b1) * (small ? 2 : 1), 256)));
         char *b = (char *)p->mem;
         p->segstart = (int32_t *)b;
         p->segrow = (int32_t *)(b + sz_st);
         p->part = b + sz_st + sz_rw;
-        int st = bsr_spmv_table(mb, nnzb, origin, browptr, p->segstart, p->segrow, p->nsegmax, stream);
+        int st = small ? bsr_spmv_starts(mb, nnzb, b1, origin, browptr, p->segstart, stream)
+                       : bsr_spmv_table(mb, nnzb, origin, browptr, p->segstart, p->segrow, p->nsegmax, stream);
         if (!st) {
             const hipError_t e = hipStreamSynchronize(s);  // the plan may then run on any stream
             if (e != hipSuccess) st = hip_fail(e, "bsr_spmv_plan_create");
@@ -2797,6 +3033,10 @@ static int bsr_spmv_plan_execute(jlust_bsr_spmv_plan_t plan, int value_type, T a
         return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmv_plan_execute: plan belongs to device %d, current device is %d",
                     plan->device, dev);
     if (plan->mb == 0) return JLUST_STATUS_SUCCESS;
+    if (bsr_spmv_is_square_small(plan->b1, plan->b2))
+        return bsr_spmv_items<T>(plan->mb, plan->nb, plan->b1, plan->nnzb, plan->origin, plan->browptr,
+                                 plan->bcolind, (const T *)plan->val, plan->row_major, alpha, x, beta, y,
+                                 plan->segstart, (T *)plan->part, stream);
     return bsr_spmv_run<T>(plan->mb, plan->nb, plan->b1, plan->b2, plan->nnzb, plan->origin, plan->browptr,
                            plan->bcolind, (const T *)plan->val, plan->row_major, alpha, x, beta, y, plan->segstart,
                            plan->segrow, (T *)plan->part, plan->nsegmax, stream);

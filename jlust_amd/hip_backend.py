@@ -732,8 +732,12 @@ class _CachedBSRPlan:
                 mb, nb, b1, b2, bcolind.numel(), u_A.origin.offset, 0 if suf == "f64" else 1, int(row_major),
                 _ptr(browptr), _ptr(bcolind), _ptr(vals), _stream(dev), ctypes.byref(self.plan))
         _lib.check(st, "bsr_spmv_plan_create", u_A.format, _BE, vals.dtype)
-        nseg = mb + (bcolind.numel() + 31) // 32         # segments of at most 32 blocks
-        self.bytes = 4 * (mb + 1) + 4 * nseg + nseg * b1 * vals.element_size()
+        if b1 == b2 and 2 <= b1 <= 8:                    # runs of 1024 // b rows and blocks
+            nrun = -(-(mb + bcolind.numel()) // (1024 // b1))
+            self.bytes = 4 * (nrun + 1) + 2 * nrun * b1 * vals.element_size()
+        else:
+            nseg = mb + (bcolind.numel() + 31) // 32     # segments of at most 32 blocks
+            self.bytes = 4 * (mb + 1) + 4 * nseg + nseg * b1 * vals.element_size()
         self.kind = "bsr_segments"
         self.what = "bsr_spmv_plan_execute"
         self.refs = (weakref.ref(idx1), weakref.ref(idx2), weakref.ref(vals))

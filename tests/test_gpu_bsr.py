@@ -683,3 +683,53 @@ def test_bsr_small_blocks(J, O, dtype, b, row_major):
         J.execute(h, Bd, C2)
         ref = O.bsr_spmm(bp, bc, flat, b, B, 1.0, 0.0, C0.copy(order="F"), row_major_blocks=row_major, b2=b)
         np.testing.assert_array_equal(host(C2), ref, err_msg=f"plan k={k}")
+
+
+@pytest.mark.parametrize("b", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("row_major", [True, False])
+def test_bsr_spmv_runs_of_items(J, O, b, dtype, row_major):
+    """SpMV of square blocks of 2 to 8 rows: runs of items = 1024 // b row
+    starts and blocks.  A row that ends with its run and one that ends one
+    item later, rows that start at a run's last item, a row over several runs,
+    more empty rows than a run holds, an empty last row, one run alone and no
+    blocks at all; values and x at an odd offset, alpha / beta, the plan's
+    result equal to the plain call's."""
+    import torch
+    items = 1024 // b
+    rng = np.random.default_rng(b + 10 * row_major)
+    origin = 1 if row_major else 0
+    og = J.OneBased() if origin else J.ZeroBased()
+    cases = {
+        "run ends with a row": [items // 2 - 1, items - items // 2 - 1, items - 1, 3, 0],
+        "one block over": [items // 2 - 1, items - items // 2, 5, items, 2],
+        "start is a run's last item": [items - 2, 7, 0, 3 * items + 11, items - 10, 1],
+        "empty rows": [3] + [0] * (2 * items + 5) + [4 * items, 0, 1, 0],
+        "one run": [1, 0, 2],
+        "no blocks": [0, 0, 0],
+    }
+    for name, lens in cases.items():
+        lens = np.asarray(lens)
+        mb, nb = len(lens), max(int(lens.max()), 4)
+        bcols = [np.sort(rng.choice(nb, int(n), replace=False)) for n in lens]
+        bp = (np.r_[0, np.cumsum(lens)] + origin).astype(np.int32)
+        bc = (np.concatenate(bcols) + origin).astype(np.int32)
+        flat = rng.standard_normal(bc.size * b * b).astype(dtype)
+        x = rng.uniform(-1, 1, nb * b).astype(dtype)
+        y0 = rng.uniform(-1, 1, mb * b).astype(dtype)
+        rp, ci, v = O.bsr_to_csr(bp, bc, flat, b, origin, row_major, b)
+        vals, xs = dev(np.r_[np.zeros(1, dtype), flat])[1:], dev(np.r_[np.zeros(1, dtype), x])[1:]
+        A = J.bsr_tensor(dev(bp), dev(bc), vals, (mb * b, nb * b), (b, b), row_major, og)
+        h = J.prepare(J.HIPBackend(), J.SpMVOp, A)
+        for alpha, beta in ((1.0, 0.0), (-0.5, 1.5)):
+            ys = []
+            for call in (lambda y: J.execute(J.SpMVOp, A, xs, y, alpha=alpha, beta=beta),
+                         lambda y: J.execute(h, xs, y, alpha=alpha, beta=beta)):
+                y = dev(y0.copy()) if beta else torch.full((mb * b,), float("nan"), dtype=A.dtype, device="cuda")
+                call(y)
+                ys.append(host(y))
+            yb = y0 if beta else None
+            ref = O.csr_spmv(rp, ci, v, x, alpha, beta, yb, origin)
+            absref = O.csr_spmv_absref(rp, ci, v, x, alpha, beta, yb, origin)
+            assert_within(ys[0], ref, absref, dtype, f"{name}, beta={beta}")
+            np.testing.assert_array_equal(ys[1], ys[0], err_msg=f"{name}, plan")
