@@ -959,6 +959,22 @@ int jlust_hip_convert_analyze_ws(const jlust_sparse *src, int32_t dst_format,
                                  jlust_stream_t stream, jlust_convert_t *out,
                                  int64_t *dst_nnz, int64_t *dst_nouter);
 
+/* CSR to CSC, CSC to CSR and CSC to COO in one call, without a handle: the
+ * entries move to the target's buffers in two or three passes.  workspace
+ * reports the device bytes of ws (256-byte aligned); 0: not a conversion of
+ * this kind, or one the two steps do better.  dst: origin and extents of src,
+ * nnz = src->nnz, its buffers allocated for that many entries.  *count: the
+ * entries written (fewer than nnz where zeros were dropped or coordinates
+ * repeated), or -1 if src's segment pointers are not canonical or the
+ * conversion is not of this kind: dst is then undefined, use the two steps.
+ * Results as theirs, bit for bit.  Synchronises `stream`. */
+int jlust_hip_convert_direct_workspace(const jlust_sparse *src,
+                                       int32_t dst_format, int value_type,
+                                       int64_t *bytes);
+int jlust_hip_convert_direct(const jlust_sparse *src, const jlust_sparse *dst,
+                             int value_type, void *ws, int64_t ws_bytes,
+                             jlust_stream_t stream, int64_t *count);
+
 /* Step 2: writes the target's buffers (caller-allocated with the sizes from
  * analyze; origin, extents and format equal to the source's and the analysed
  * target), stream-ordered. */

@@ -94,6 +94,47 @@ def _stream(dev):
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
+def _convert_direct(u: USTensor, fmt: TensorFormat, src: Sparse, fid: int, dev):
+    """CSR to CSC, CSC to CSR or COO in one call (jlust_hip_convert_direct), or
+    None where the two steps of convert_format do it."""
+    L = _lib.lib()
+    vt, nz = _VT[u.val.dtype], u.val.numel()
+    need, count = ctypes.c_int64(), ctypes.c_int64()
+    _lib.check(L.jlust_hip_convert_direct_workspace(ctypes.byref(src), fid, vt, ctypes.byref(need)),
+               "convert_direct", fmt)
+    if need.value == 0:
+        return None
+    m, n = u.extents
+    i32 = dict(dtype=torch.int32, device=dev)
+    ws = torch.empty(need.value, dtype=torch.uint8, device=dev)
+    val, crd = torch.empty(nz, dtype=u.val.dtype, device=dev), torch.empty(nz, **i32)
+    dst = Sparse(format=fid, origin=u.origin.offset, m=m, n=n, b1=1, b2=1, nnz=nz)
+    dst.val, dst.crd2 = val.data_ptr(), crd.data_ptr()
+    if fid == FMT_COO:
+        pos1, rows = torch.empty(2, **i32), torch.empty(nz, **i32)
+        dst.pos1, dst.crd1 = pos1.data_ptr(), rows.data_ptr()
+    else:
+        ptr = torch.empty((m if fid == FMT_CSR else n) + 1, **i32)
+        dst.pos2 = ptr.data_ptr()
+    st = L.jlust_hip_convert_direct(ctypes.byref(src), ctypes.byref(dst), vt, _ptr(ws), need.value, _stream(dev),
+                                    ctypes.byref(count))
+    _lib.check(st, "convert_direct", fmt)
+    c = count.value
+    if c < 0:
+        return None
+
+    def cut(t):                                  # zeros dropped, coordinates merged
+        return t if c == nz else t[:c].clone()
+
+    if fid == FMT_COO:
+        out = (pos1, None), (cut(rows), cut(crd)), cut(val)
+    else:
+        out = (None, ptr), (None, cut(crd)), cut(val)
+    if fid == FMT_COO or c < nz:                 # work of this call is still running
+        torch.cuda.current_stream(dev).synchronize()
+    return USTensor((m, n), fmt, *out, None, u.origin)
+
+
 def convert_format(u: USTensor, fmt: TensorFormat, index_type=None, value_type=None) -> USTensor:
     """src/convert.jl:302-388 on the device: a new tensor in `fmt` with u's origin."""
     if index_type not in (None, torch.int32):
@@ -106,6 +147,10 @@ def convert_format(u: USTensor, fmt: TensorFormat, index_type=None, value_type=N
     src = _descriptor(u)
     fid, b1, b2, rm = _format_id(fmt)
     L = _lib.lib()
+    with torch.cuda.device(dev):
+        direct = _convert_direct(u, fmt, src, fid, dev)
+    if direct is not None:
+        return direct
     h = ctypes.c_void_p()
     nnz_out, nouter = ctypes.c_int64(), ctypes.c_int64()
     with torch.cuda.device(dev):

@@ -15,8 +15,9 @@
 // Pipeline on the device: per-entry coordinates (segment ids by scatter +
 // max-scan), zero-drop compaction, stable LSD radix sort (rocPRIM) of packed
 // level keys with source positions as values, adjacent-key dedup, then the
-// target's pos/crd/val from the sorted keys.  Integer work only; values are
-// moved as bits.
+// target's pos/crd/val from the sorted keys.  CSR to CSC and CSC to CSR or COO
+// move whole entries by coordinate instead (convert_direct).  Integer work
+// only; values are moved as bits.
 //
 // Also: sparse_to_dense (ext/KernelAbstractionsExt/ops/conversion.jl:47-65)
 // and the index shift of materialize's origin change (CUDAExt.jl:199-220).
@@ -288,6 +289,399 @@ __global__ void shift_kernel(int64_t n, int32_t *__restrict__ dst, const int32_t
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i] + delta;
+}
+
+// --------------------------------------------- CSR <-> CSC and CSC -> COO
+//
+// A conversion that orders the entries by the source's inner coordinate and
+// keeps their order otherwise (sort_bits' major_only) is a stable sort of
+// (coordinate, segment, value) by the coordinate.  The general path sorts
+// 64-bit keys with positions and then fetches each value from where it was
+// stored: 16M f64 entries take 480 us of sorting, 326 of random 8-byte reads
+// and 250 of passes that make and check the keys.  Here an entry moves whole,
+// 16 bytes, in passes of up to CS_BITS bits (two for up to 4M columns), the
+// first of which reads the source and the last of which writes the target.
+//
+// What bounds it: memory, 32 bytes an entry and pass.  A workgroup takes
+// CS_TILE consecutive entries, ranks them by digit (equal digits of a wave
+// found by ballots, in order; waves by a table in LDS), puts them in digit
+// order in LDS and writes each digit's stretch at its place, found by a scan
+// of the tiles' digit counts.  The larger the tile, the longer the stretches:
+// 8,192 entries leave 8 of each of 1,024 digits, 64 bytes of values.
+// Consecutive tiles go to the same XCD, so that their stretches, which are
+// neighbours, meet in one L2.
+//
+// 16M f64 entries of 1,000,003 columns (512 MB of traffic a pass): the first
+// pass' count 67 us, the second's 21, each move 166 (3.1 TB/s; 16 entries a
+// thread without spills, two tiles a CU; 1,024 threads of 8 in 64 registers
+// took 195, with spills 285), scans 18, repeats 24, pointers 28: a whole
+// conversion 556 us, 1,201 by the general path.  10,007 rows of 9: 126 us, 260
+// there, both mostly launches.
+constexpr int CS_THREADS = 512, CS_WAVES = CS_THREADS / 64, CS_ITEMS = 16;
+constexpr int CS_TILE = CS_THREADS * CS_ITEMS;
+constexpr int CC_THREADS = 1024, CC_ITEMS = CS_TILE / CC_THREADS;      // the counting kernel
+constexpr int CS_BITS = 11;
+constexpr int CS_DIGITS = 1 << CS_BITS;
+constexpr int CS_WPT = CS_DIGITS / 2 / CS_THREADS;       // pairs of digits a thread
+
+struct SortPass {
+    int shift, bits;                       // the digit
+    int64_t ntiles;
+};
+
+__device__ __forceinline__ int64_t sort_tile(int64_t ntiles)
+{
+    const int64_t per = (ntiles + 7) / 8;
+    return (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+}
+
+enum { CS_BAD = 0, CS_POINTERS = 1, CS_REPEATS = 2, CS_COUNT = 3 };     // flags[]
+
+// hist[digit * ntiles + tile]: how often the tile's entries hold the digit.
+// The first pass reads the source, drops zeros and checks the coordinates and
+// the segment pointers; the others read the keys of the pass before.
+template <typename T, bool FIRST>
+__global__ __launch_bounds__(CC_THREADS) void sort_count_kernel(jlust_sparse src, int64_t nseg, int64_t major_dim,
+                                                                const uint32_t *__restrict__ keys, SortPass ps,
+                                                                int32_t *__restrict__ hist,
+                                                                int32_t *__restrict__ flags)
+{
+    __shared__ uint32_t h[CS_DIGITS];
+    const int64_t tile = sort_tile(ps.ntiles);
+    if (tile >= ps.ntiles) return;
+    const int nd = 1 << ps.bits, tid = threadIdx.x;
+    const int64_t n = FIRST ? src.nnz : (int64_t)flags[CS_COUNT];
+    for (int d = tid; d < nd; d += CC_THREADS) h[d] = 0;
+    __syncthreads();
+    bool bad = false;
+    if (tile * CS_TILE < n) {
+        // All loads first; threads past the end read the last entry.
+        const int64_t p0 = tile * CS_TILE + tid;
+        int64_t key[CC_ITEMS];
+        bool valid[CC_ITEMS];
+#pragma unroll
+        for (int j = 0; j < CC_ITEMS; ++j) {
+            const int64_t p = min(p0 + j * CC_THREADS, n - 1);
+            valid[j] = p0 + j * CC_THREADS < n;
+            if (FIRST) {
+                key[j] = (int64_t)src.crd2[p] - src.origin;
+                const bool inb = key[j] >= 0 && key[j] < major_dim;
+                bad = bad || !inb;
+                valid[j] = valid[j] && inb && static_cast<const T *>(src.val)[p] != T(0);  // no -0.0; NaN kept
+            } else {
+                key[j] = keys[p];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < CC_ITEMS; ++j)
+            if (valid[j]) atomicAdd(&h[(uint32_t)key[j] >> ps.shift & (nd - 1)], 1u);
+    }
+    if (FIRST) {
+        if (bad) flags[CS_BAD] = 1;
+        const int64_t per = (nseg + ps.ntiles - 1) / ps.ntiles;
+        bool off = tile == 0 && tid == 0 &&
+                   (src.pos2[0] != src.origin || (int64_t)src.pos2[nseg] != src.nnz + src.origin);
+        for (int64_t s = tile * per + tid; s < min((tile + 1) * per, nseg); s += CC_THREADS)
+            off = off || src.pos2[s + 1] < src.pos2[s];
+        if (off) flags[CS_POINTERS] = 1;
+    }
+    __syncthreads();
+    for (int d = tid; d < nd; d += CC_THREADS) hist[(int64_t)d * ps.ntiles + tile] = (int32_t)h[d];
+    if (tile == 0 && tid == 0) hist[(int64_t)nd * ps.ntiles] = 0;
+}
+
+// The last segment that starts at position p or before (0 if none), by a
+// whole wave; ends for any pointer array.
+__device__ __forceinline__ int32_t segment_of(const int32_t *__restrict__ ptr, int64_t nseg, int32_t origin, int64_t p)
+{
+    const int lane = threadIdx.x & 63;
+    int64_t lo = 0, hi = nseg;
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + 63) / 64, at = lo + lane * step;
+        const bool le = lane == 0 || (at < hi && (int64_t)ptr[at] - origin <= p);
+        lo += (63 - __builtin_clzll(__ballot(le))) * step;
+        hi = min(hi, lo + step);
+    }
+    return (int32_t)lo;
+}
+
+// One pass: the entries of each tile to their places by digit, hist holding
+// the exclusive scan of the counts.  okey gets the coordinate + kadd, ominor
+// the segment + madd (the target's index origin in the last pass).
+template <typename T, bool FIRST>
+__global__ __launch_bounds__(CS_THREADS, 4) void sort_move_kernel(jlust_sparse src, int64_t nseg, int64_t major_dim,
+                                                                  const uint32_t *__restrict__ ikey,
+                                                                  const uint32_t *__restrict__ iminor,
+                                                                  const T *__restrict__ ival, SortPass ps,
+                                                                  const int32_t *__restrict__ hist,
+                                                                  int32_t *__restrict__ flags,
+                                                                  uint32_t *__restrict__ okey,
+                                                                  uint32_t *__restrict__ ominor,
+                                                                  T *__restrict__ oval, uint32_t kadd, uint32_t madd)
+{
+    // In turn: segment marks, the waves' digit counts, the entries in order.
+    __shared__ __align__(16) char lds[CS_TILE * 8];
+    __shared__ int32_t delta[CS_DIGITS];
+    __shared__ int32_t wsum[CS_WAVES];
+    __shared__ int32_t seg01[2];
+    const int64_t tile = sort_tile(ps.ntiles);
+    if (tile >= ps.ntiles) return;
+    const int nd = 1 << ps.bits, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t n = FIRST ? src.nnz : (int64_t)flags[CS_COUNT];
+    const int64_t t0 = tile * CS_TILE, t1 = min(t0 + CS_TILE, n);
+    if (t0 >= n) return;
+    const int base = wave * (64 * CS_ITEMS) + lane;       // this thread's entries: base + 64 j
+    // An entry's value stays in memory until its place is known (the first
+    // pass reads it here too, to drop zeros).
+    const int last = (int)(t1 - t0) - 1;
+    const T *value = (FIRST ? static_cast<const T *>(src.val) : ival) + t0;
+    const uint32_t *keys = (FIRST ? reinterpret_cast<const uint32_t *>(src.crd2) : ikey) + t0;
+    uint32_t key[CS_ITEMS], minor[CS_ITEMS], valid = 0;
+    T val[CS_ITEMS];
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j) {
+        const uint32_t i = (uint32_t)min(base + 64 * j, last) & (CS_TILE - 1);
+        key[j] = keys[i];
+        if (FIRST) val[j] = value[i];
+    }
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j) {
+        if (FIRST) key[j] -= (uint32_t)src.origin;
+        const bool in = base + 64 * j <= last, ok = !FIRST | (((int64_t)key[j] < major_dim) & (val[j] != T(0)));
+        valid |= (uint32_t)(in & ok) << j;
+    }
+    if (FIRST) {
+        // The entries' segments: each segment marked at its first entry, then
+        // a running maximum.
+        int32_t *mark = reinterpret_cast<int32_t *>(lds);
+        if (wave < 2) {
+            const int32_t s = segment_of(src.pos2, nseg, src.origin, wave == 0 ? t0 : t1 - 1);
+            if (lane == 0) seg01[wave] = s;
+        }
+        for (int i = tid; i < CS_TILE; i += CS_THREADS) mark[i] = 0;
+        __syncthreads();
+        const int32_t s0 = seg01[0], s1 = seg01[1];
+        if (tid == 0) mark[0] = s0;
+        for (int64_t s = (int64_t)s0 + 1 + tid; s <= s1; s += CS_THREADS) {
+            const int64_t a = (int64_t)src.pos2[s] - src.origin, b = (int64_t)src.pos2[s + 1] - src.origin;
+            if (b > a && a > t0 && a < t1) mark[a - t0] = (int32_t)s;
+        }
+        __syncthreads();
+        int32_t m[CS_ITEMS];
+#pragma unroll
+        for (int j = 0; j < CS_ITEMS; ++j) {
+            m[j] = mark[tid * CS_ITEMS + j];
+            if (j) m[j] = max(m[j], m[j - 1]);
+        }
+        int32_t top = m[CS_ITEMS - 1];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int32_t o = __shfl_up(top, d, 64);
+            if (lane >= d) top = max(top, o);
+        }
+        if (lane == 63) wsum[wave] = top;
+        int32_t before = __shfl_up(top, 1, 64);
+        if (lane == 0) before = 0;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) before = max(before, wsum[w]);
+#pragma unroll
+        for (int j = 0; j < CS_ITEMS; ++j) mark[tid * CS_ITEMS + j] = max(m[j], before);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CS_ITEMS; ++j) minor[j] = (uint32_t)mark[base + 64 * j];
+        __syncthreads();
+    }
+    // Ranks: in its wave, by the wave's own count of each digit so far.
+    uint32_t *cnt2 = reinterpret_cast<uint32_t *>(lds);   // two digits a word
+    uint16_t *cnt = reinterpret_cast<uint16_t *>(lds) + wave * nd;
+    const int words = nd / 2;
+    for (int i = tid; i < CS_WAVES * words; i += CS_THREADS) cnt2[i] = 0;
+    int32_t place[CS_WPT][2];                             // of this thread's digits
+#pragma unroll
+    for (int q = 0; q < CS_WPT; ++q)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int d = 2 * (tid * CS_WPT + q) + e;
+            place[q][e] = d < nd ? hist[(int64_t)d * ps.ntiles + tile] : 0;
+        }
+    __syncthreads();
+    uint32_t at[CS_ITEMS];
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j) {
+        const bool v = valid >> j & 1;
+        const uint32_t d = key[j] >> ps.shift & (uint32_t)(nd - 1);
+        const uint64_t all = __ballot(v);
+        uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
+        for (int b = 0; b < ps.bits; ++b) {
+            const uint32_t on = (uint32_t)__builtin_amdgcn_sbfe((int)d, (uint32_t)b, 1u);   // 0 or all ones
+            const uint64_t m = __ballot(on != 0);
+            lo &= ~((uint32_t)m ^ on);
+            hi &= ~((uint32_t)(m >> 32) ^ on);
+        }
+        if (v) {
+            const uint32_t old = __hip_atomic_load(cnt + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            const uint32_t prior = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+            at[j] = old + prior;
+            if (prior == 0)
+                __hip_atomic_store(cnt + d, (uint16_t)(old + __builtin_popcount(lo) + __builtin_popcount(hi)),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // The tile's stretches, by each thread's digits.
+    uint32_t c[CS_WAVES][CS_WPT], sum[CS_WPT];
+    int32_t mine = 0;
+#pragma unroll
+    for (int q = 0; q < CS_WPT; ++q) {
+        sum[q] = 0;
+        if (tid * CS_WPT + q < words) {
+#pragma unroll
+            for (int w = 0; w < CS_WAVES; ++w) sum[q] += c[w][q] = cnt2[w * words + tid * CS_WPT + q];
+        }
+        mine += (int32_t)(sum[q] & 0xffff) + (int32_t)(sum[q] >> 16);
+    }
+    int32_t inc = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int32_t o = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += o;
+    }
+    if (lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    int32_t first = inc - mine, total = 0;
+#pragma unroll
+    for (int w = 0; w < CS_WAVES; ++w) {
+        const int32_t t = wsum[w];
+        if (w < wave) first += t;
+        total += t;
+    }
+#pragma unroll
+    for (int q = 0; q < CS_WPT; ++q) {
+        const int word = tid * CS_WPT + q;
+        if (word >= words) break;
+        const int32_t second = first + (int32_t)(sum[q] & 0xffff);
+        uint32_t run = (uint32_t)first | (uint32_t)second << 16;
+#pragma unroll
+        for (int w = 0; w < CS_WAVES; ++w) {
+            cnt2[w * words + word] = run;
+            run += c[w][q];
+        }
+        delta[2 * word] = place[q][0] - first;
+        delta[2 * word + 1] = place[q][1] - second;
+        first = second + (int32_t)(sum[q] >> 16);
+    }
+    if (FIRST && tile == 0 && tid == 0) flags[CS_COUNT] = hist[(int64_t)nd * ps.ntiles];
+    // (An index the compiler can't see through: loads moved up would spill.)
+    uint32_t here = (uint32_t)base;
+    asm volatile("" : "+v"(here));
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j) {
+        const uint32_t i = min(here + 64 * j, (uint32_t)last) & (CS_TILE - 1);
+        if (!FIRST) minor[j] = iminor[t0 + i];
+        val[j] = value[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j)
+        if (valid >> j & 1) at[j] += cnt[key[j] >> ps.shift & (uint32_t)(nd - 1)];
+    __syncthreads();
+    // Out in digit order, one array after the other through the same LDS.
+    uint32_t *box = reinterpret_cast<uint32_t *>(lds);
+    T *vbox = reinterpret_cast<T *>(lds);
+    uint32_t dst[CS_ITEMS];
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j)
+        if (valid >> j & 1) box[at[j]] = key[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j) {
+        const int i = tid + CS_THREADS * j;
+        if (i >= total) continue;
+        const uint32_t k = box[i];
+        dst[j] = (uint32_t)(delta[k >> ps.shift & (uint32_t)(nd - 1)] + i);
+        okey[dst[j]] = k + kadd;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j)
+        if (valid >> j & 1) box[at[j]] = minor[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j)
+        if (tid + CS_THREADS * j < total) ominor[dst[j]] = box[tid + CS_THREADS * j] + madd;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j)
+        if (valid >> j & 1) vbox[at[j]] = val[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CS_ITEMS; ++j)
+        if (tid + CS_THREADS * j < total) oval[dst[j]] = vbox[tid + CS_THREADS * j];
+}
+
+// Counts the sorted entries that repeat the coordinates before them, and
+// (head given) marks the others.
+__global__ __launch_bounds__(256) void sort_repeats_kernel(int64_t nmax, const uint32_t *__restrict__ key,
+                                                           const uint32_t *__restrict__ minor,
+                                                           int32_t *__restrict__ flags, int32_t *__restrict__ head)
+{
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    const int64_t n = min(nmax, (int64_t)flags[CS_COUNT]);
+    int repeats = 0;
+    if (i + 4 <= n) {
+        const uint4 k = *reinterpret_cast<const uint4 *>(key + i);
+        uint4 m;                            // the caller's, of any alignment
+        __builtin_memcpy(&m, minor + i, sizeof(m));
+        const uint32_t kp = i > 0 ? key[i - 1] : ~k.x, mp = i > 0 ? minor[i - 1] : 0;
+        const int r0 = kp == k.x && mp == m.x, r1 = k.x == k.y && m.x == m.y, r2 = k.y == k.z && m.y == m.z,
+                  r3 = k.z == k.w && m.z == m.w;
+        repeats = r0 + r1 + r2 + r3;
+        if (head) *reinterpret_cast<int4 *>(head + i) = make_int4(1 - r0, 1 - r1, 1 - r2, 1 - r3);
+    } else {
+        for (int64_t t = i; t < n; ++t) {
+            const int r = t > 0 && key[t] == key[t - 1] && minor[t] == minor[t - 1];
+            repeats += r;
+            if (head) head[t] = 1 - r;
+        }
+    }
+    if (head) return;
+    int sum = 0;                            // of the wave: each thread has 0 to 4
+    for (int b = 0; b < 3; ++b) sum += __popcll(__ballot(repeats >> b & 1)) << b;
+    if (sum > 0 && (threadIdx.x & 63) == 0) atomicAdd(&flags[CS_REPEATS], sum);
+}
+
+// The marked entries to their places (idx: the exclusive scan of the marks).
+template <typename T>
+__global__ __launch_bounds__(256) void sort_heads_kernel(int64_t n, const int32_t *__restrict__ head,
+                                                         const int32_t *__restrict__ idx,
+                                                         const uint32_t *__restrict__ key,
+                                                         const uint32_t *__restrict__ minor,
+                                                         const T *__restrict__ val, uint32_t *__restrict__ okey,
+                                                         uint32_t *__restrict__ ominor, T *__restrict__ oval)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n || !head[i]) return;
+    okey[idx[i]] = key[i];
+    ominor[idx[i]] = minor[i];
+    oval[idx[i]] = val[i];
+}
+
+// ptr[r] = origin + first i with key[i] >= r, r in [0, nmajor], of the first
+// *count keys.
+__global__ __launch_bounds__(256) void sort_ptr_kernel(const uint32_t *__restrict__ key,
+                                                       const int32_t *__restrict__ count, int64_t nmajor,
+                                                       int32_t origin, int32_t *__restrict__ ptr)
+{
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r > nmajor) return;
+    int64_t lo = 0, hi = *count;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if ((int64_t)key[mid] < r) lo = mid + 1;
+        else hi = mid;
+    }
+    ptr[r] = (int32_t)(lo + origin);
 }
 
 // ----------------------------------------------------------------- host
@@ -611,6 +1005,143 @@ int analyze(const jlust_sparse *src, jlust_convert *h, void *ws, const AnalyzeLa
     return JLUST_STATUS_SUCCESS;
 }
 
+// The passes and the workspace of a direct conversion; passes == 0: not one.
+struct DirectLayout {
+    int64_t nseg = 0, major_dim = 0, ntiles = 0;
+    int passes = 0, bits = 0;
+    size_t tmp = 0, hist = 0, bytes = 0;
+};
+
+int direct_layout(const jlust_sparse *src, int dst_format, size_t vsize, DirectLayout *out)
+{
+    *out = DirectLayout();
+    const bool csr = src->format == JLUST_FORMAT_CSR;
+    if (!(csr && dst_format == JLUST_FORMAT_CSC) &&
+        !(src->format == JLUST_FORMAT_CSC && (dst_format == JLUST_FORMAT_CSR || dst_format == JLUST_FORMAT_COO)))
+        return JLUST_STATUS_SUCCESS;
+    out->nseg = csr ? src->m : src->n;
+    out->major_dim = csr ? src->n : src->m;
+    // A tile walks its segments: where almost all are empty the general
+    // path's scan over the entries is the better one.
+    if (src->nnz == 0 || out->major_dim == 0 || out->nseg == 0 || out->nseg > 16 * src->nnz)
+        return JLUST_STATUS_SUCCESS;
+    const int bits = std::max(1, bits_for(out->major_dim));
+    out->passes = (bits + CS_BITS - 1) / CS_BITS;
+    out->bits = (bits + out->passes - 1) / out->passes;
+    out->ntiles = (src->nnz + CS_TILE - 1) / CS_TILE;
+    out->hist = ((size_t)1 << out->bits) * (size_t)out->ntiles + 1;
+    int32_t *v = nullptr;
+    size_t a = 0, b = 0;
+    JLUST_HIP_TRY(rocprim::exclusive_scan(nullptr, a, v, v, 0, out->hist, rocprim::plus<int32_t>(), (hipStream_t)0));
+    JLUST_HIP_TRY(rocprim::exclusive_scan(nullptr, b, v, v, 0, (size_t)src->nnz, rocprim::plus<int32_t>(),
+                                          (hipStream_t)0));
+    out->tmp = std::max(a, b);
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    const size_t n = (size_t)src->nnz, entry = up(vsize * n) + 2 * up(4 * n);
+    // flags, counts, scan; the entries after the first pass; marks and their
+    // scan, or the entries after the second of three; the target's majors.
+    out->bytes = 256 + up(4 * out->hist) + up(out->tmp) + entry + (out->passes > 2 ? entry : 2 * up(4 * n)) + up(4 * n);
+    return JLUST_STATUS_SUCCESS;
+}
+
+template <typename T>
+int direct_run(const jlust_sparse *src, const jlust_sparse *dst, const DirectLayout &dl, void *ws, int64_t *count,
+               hipStream_t st)
+{
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    const int64_t N = src->nnz;
+    const size_t n = (size_t)N;
+    char *b = (char *)ws;
+    auto take = [&](size_t bytes) { char *p = b; b += up(bytes); return p; };
+    struct Entries { uint32_t *key, *minor; T *val; };
+    auto entries = [&] { Entries e; e.val = (T *)take(sizeof(T) * n); e.key = (uint32_t *)take(4 * n);
+                         e.minor = (uint32_t *)take(4 * n); return e; };
+    int32_t *flags = (int32_t *)take(256);
+    int32_t *hist = (int32_t *)take(4 * dl.hist);
+    void *tmp = take(dl.tmp);
+    const Entries e1 = entries();
+    char *after = b;
+    Entries e2 = {nullptr, nullptr, nullptr};
+    int32_t *head = nullptr, *idx = nullptr;
+    if (dl.passes > 2) e2 = entries();
+    else b += 2 * up(4 * n);
+    head = (int32_t *)after;
+    idx = (int32_t *)(after + up(4 * n));
+    uint32_t *major = (uint32_t *)take(4 * n);
+    const bool coo = dst->format == JLUST_FORMAT_COO;
+    const uint32_t o = (uint32_t)dst->origin;
+    const Entries out = {coo ? (uint32_t *)dst->crd1 : major, (uint32_t *)dst->crd2, (T *)dst->val};
+    JLUST_HIP_TRY(hipMemsetAsync(flags, 0, 16 * sizeof(int32_t), st));
+    Entries in = {nullptr, nullptr, nullptr};
+    const dim3 grid((unsigned)((dl.ntiles + 7) / 8 * 8)), block(CS_THREADS);
+    for (int p = 0; p < dl.passes; ++p) {
+        const SortPass ps = {p * dl.bits, dl.bits, dl.ntiles};
+        const bool last = p == dl.passes - 1;
+        const Entries to = last ? out : p % 2 ? e2 : e1;
+        if (p == 0)
+            hipLaunchKernelGGL((sort_count_kernel<T, true>), grid, dim3(CC_THREADS), 0, st, *src, dl.nseg, dl.major_dim, in.key, ps,
+                               hist, flags);
+        else
+            hipLaunchKernelGGL((sort_count_kernel<T, false>), grid, dim3(CC_THREADS), 0, st, *src, dl.nseg, dl.major_dim, in.key,
+                               ps, hist, flags);
+        if (int e = check_launch("sort_count_kernel")) return e;
+        size_t need = dl.tmp;
+        JLUST_HIP_TRY(rocprim::exclusive_scan(tmp, need, hist, hist, 0, dl.hist, rocprim::plus<int32_t>(), st));
+        const uint32_t kadd = last && coo ? o : 0, madd = last ? o : 0;
+        if (p == 0)
+            hipLaunchKernelGGL((sort_move_kernel<T, true>), grid, block, 0, st, *src, dl.nseg, dl.major_dim, in.key,
+                               in.minor, in.val, ps, hist, flags, to.key, to.minor, to.val, kadd, madd);
+        else
+            hipLaunchKernelGGL((sort_move_kernel<T, false>), grid, block, 0, st, *src, dl.nseg, dl.major_dim, in.key,
+                               in.minor, in.val, ps, hist, flags, to.key, to.minor, to.val, kadd, madd);
+        if (int e = check_launch("sort_move_kernel")) return e;
+        in = to;
+    }
+    auto pointers = [&]() -> int {
+        hipLaunchKernelGGL(sort_ptr_kernel, dim3(cv_grid(dl.major_dim + 1)), dim3(256), 0, st, major, flags + CS_COUNT,
+                           dl.major_dim, dst->origin, dst->pos2);
+        return check_launch("sort_ptr_kernel");
+    };
+    if (!coo) {
+        hipLaunchKernelGGL(sort_repeats_kernel, dim3(cv_grid((N + 3) / 4)), dim3(256), 0, st, N, major,
+                           (uint32_t *)dst->crd2, flags, (int32_t *)nullptr);
+        if (int e = check_launch("sort_repeats_kernel")) return e;
+        if (int e = pointers()) return e;
+    }
+    int32_t got[4] = {0, 0, 0, 0};
+    JLUST_HIP_TRY(hipMemcpyAsync(got, flags, sizeof(got), hipMemcpyDeviceToHost, st));
+    JLUST_HIP_TRY(hipStreamSynchronize(st));
+    if (got[CS_POINTERS]) return JLUST_STATUS_SUCCESS;      // *count stays -1
+    if (got[CS_BAD])
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert: a stored coordinate lies outside the %lld x %lld extents",
+                    (long long)src->m, (long long)src->n);
+    int64_t C = got[CS_COUNT];
+    if (coo && dst->pos1) {
+        hipLaunchKernelGGL(pair_kernel, dim3(1), dim3(64), 0, st, dst->pos1, dst->origin, (int32_t)(C + dst->origin));
+        if (int e = check_launch("pair_kernel")) return e;
+    }
+    if (got[CS_REPEATS] > 0) {                              // unique levels keep the first of equal coordinates
+        hipLaunchKernelGGL(sort_repeats_kernel, dim3(cv_grid((C + 3) / 4)), dim3(256), 0, st, C, major,
+                           (uint32_t *)dst->crd2, flags, head);
+        if (int e = check_launch("sort_repeats_kernel")) return e;
+        size_t need = dl.tmp;
+        JLUST_HIP_TRY(rocprim::exclusive_scan(tmp, need, head, idx, 0, (size_t)C, rocprim::plus<int32_t>(), st));
+        hipLaunchKernelGGL(sort_heads_kernel<T>, dim3(cv_grid(C)), dim3(256), 0, st, C, head, idx, major,
+                           (uint32_t *)dst->crd2, (T *)dst->val, e1.key, e1.minor, e1.val);
+        if (int e = check_launch("sort_heads_kernel")) return e;
+        C -= got[CS_REPEATS];
+        got[CS_COUNT] = (int32_t)C;
+        JLUST_HIP_TRY(hipMemcpyAsync(major, e1.key, 4 * (size_t)C, hipMemcpyDeviceToDevice, st));
+        JLUST_HIP_TRY(hipMemcpyAsync(dst->crd2, e1.minor, 4 * (size_t)C, hipMemcpyDeviceToDevice, st));
+        JLUST_HIP_TRY(hipMemcpyAsync(dst->val, e1.val, sizeof(T) * (size_t)C, hipMemcpyDeviceToDevice, st));
+        JLUST_HIP_TRY(hipMemcpyAsync(flags + CS_COUNT, &got[CS_COUNT], 4, hipMemcpyHostToDevice, st));
+        if (int e = pointers()) return e;
+        JLUST_HIP_TRY(hipStreamSynchronize(st));            // `got` is read until here
+    }
+    *count = C;
+    return JLUST_STATUS_SUCCESS;
+}
+
 template <typename T>
 int fill(const jlust_convert *h, const jlust_sparse *d, hipStream_t st)
 {
@@ -816,6 +1347,46 @@ extern "C" int jlust_hip_convert_analyze_ws(const jlust_sparse *src, int32_t dst
         return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_analyze: workspace null or not 256-byte aligned");
     return convert_analyze(src, dst_format, dst_b1, dst_b2, dst_row_major_blocks, value_type, ws, (size_t)ws_bytes,
                            (hipStream_t)stream, out, dst_nnz, dst_nouter);
+}
+
+extern "C" int jlust_hip_convert_direct_workspace(const jlust_sparse *src, int32_t dst_format, int value_type,
+                                                  int64_t *bytes)
+{
+    clear_error();
+    if (!bytes) return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_direct: null output pointer");
+    KeyLayout L;
+    *bytes = 0;
+    if (dst_format == JLUST_FORMAT_BSR) return JLUST_STATUS_SUCCESS;
+    if (int st = analyze_args(src, dst_format, 1, 1, 1, value_type, &L)) return st;
+    if (int st = require_device(nullptr)) return st;
+    DirectLayout dl;
+    if (int st = direct_layout(src, dst_format, value_type == 0 ? 8 : 4, &dl)) return st;
+    *bytes = (int64_t)dl.bytes;
+    return JLUST_STATUS_SUCCESS;
+}
+
+extern "C" int jlust_hip_convert_direct(const jlust_sparse *src, const jlust_sparse *dst, int value_type, void *ws,
+                                        int64_t ws_bytes, jlust_stream_t stream, int64_t *count)
+{
+    clear_error();
+    if (!count || !dst) return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_direct: null argument");
+    *count = -1;
+    KeyLayout L;
+    if (dst->format == JLUST_FORMAT_BSR) return JLUST_STATUS_SUCCESS;
+    if (int st = analyze_args(src, dst->format, 1, 1, 1, value_type, &L)) return st;
+    if (int st = require_device(nullptr)) return st;
+    DirectLayout dl;
+    if (int st = direct_layout(src, dst->format, value_type == 0 ? 8 : 4, &dl)) return st;
+    if (dl.passes == 0) return JLUST_STATUS_SUCCESS;
+    if (!ws || (uintptr_t)ws % 256 || ws_bytes < (int64_t)dl.bytes)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_direct: workspace of %lld bytes, %zu needed at 256",
+                    (long long)ws_bytes, dl.bytes);
+    if (dst->origin != src->origin || dst->m != src->m || dst->n != src->n || dst->nnz != src->nnz)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_direct: target does not match the source");
+    if (!dst->val || !dst->crd2 || (dst->format == JLUST_FORMAT_COO ? !dst->crd1 : !dst->pos2))
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_direct: null device pointer");
+    return value_type == 0 ? direct_run<double>(src, dst, dl, ws, count, (hipStream_t)stream)
+                           : direct_run<float>(src, dst, dl, ws, count, (hipStream_t)stream);
 }
 
 extern "C" int jlust_hip_convert_fill(jlust_convert_t h, const jlust_sparse *dst, jlust_stream_t stream)

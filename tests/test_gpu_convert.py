@@ -291,3 +291,62 @@ def test_workspace_of_the_caller(J, CO, dst):
     assert run(None, need.value)[0] != 0
     got = J.convert_format(u, fmt_of(J, dst, 4, 2))
     assert got.val.numel() == own[1]
+
+
+@pytest.mark.parametrize("src,dst", [("CSR", "CSC"), ("CSC", "CSR"), ("CSC", "COO")])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("origin", [0, 1])
+def test_direct_equals_two_steps(J, src, dst, dtype, origin, monkeypatch):
+    """convert_direct against the two-step conversion, bit for bit: one to
+    three passes (coordinates below 2^11, 2^22, above), entries at the edges
+    of 8,192-entry tiles, segments over several tiles, empty ones at either
+    end, unordered and repeated coordinates, explicit zeros (-0.0), NaN, all
+    zeros, and pointers that do not cover the entries (two steps)."""
+    import torch
+    from jlust_amd import convert as CV
+    rng = np.random.default_rng(17)
+
+    def run(nseg, ncoord, lens, repeat=False, zeros=0.0, ptr=None):
+        ends = np.r_[0, np.cumsum(lens)]
+        n = int(ends[-1])
+        p = (ends if ptr is None else ptr) + origin
+        c = rng.integers(0, ncoord, n)
+        if not repeat:                                      # distinct in each segment where they fit
+            for s in np.flatnonzero(np.asarray(lens) <= ncoord):
+                a, b = int(ends[s]), int(ends[s + 1])
+                if b - a > 1 and ncoord < 100000:
+                    c[a:b] = rng.permutation(ncoord)[:b - a]
+        v = rng.standard_normal(n).astype(dtype)
+        v[rng.random(n) < zeros] = -0.0
+        if n > 3 and zeros < 1:
+            v[2] = np.nan
+        dims = (nseg, ncoord) if src == "CSR" else (ncoord, nseg)
+        og = J.OneBased() if origin else J.ZeroBased()
+        make = J.csr_tensor if src == "CSR" else CV.csc_tensor
+        u = make(*(torch.from_numpy(t).cuda() for t in (p.astype(np.int32), (c + origin).astype(np.int32), v)),
+                 dims, og)
+        out = []
+        for general in (False, True):
+            with monkeypatch.context() as mp:
+                if general:
+                    mp.setattr(CV, "_convert_direct", lambda *a: None)
+                out.append(J.convert_format(u, fmt_of(J, dst)))
+        a, b = out
+        assert a.val.numel() == b.val.numel()
+        it = torch.int64 if dtype == np.float64 else torch.int32
+        assert torch.equal(a.val.view(it), b.val.view(it))
+        for x, y in zip((*a.pos_buffers, *a.crd_buffers), (*b.pos_buffers, *b.crd_buffers)):
+            assert (x is None) == (y is None)
+            if x is not None:
+                assert torch.equal(x, y)
+
+    spread = lambda n, k: np.bincount(rng.integers(0, k, n), minlength=k)      # noqa: E731
+    for n, k, dim in ((1, 1, 1), (5, 3, 2), (8191, 700, 2048), (8192, 700, 2049), (8193, 9000, 100),
+                      (3 * 8192 + 5, 5000, 70000), (70001, 300, 5000000)):
+        run(k, dim, spread(n, k))
+        run(k, dim, spread(n, k), repeat=True, zeros=0.1)
+    run(40, 30000, np.r_[np.zeros(10, int), 20000, 0, 0, 9000, np.ones(16, int), np.zeros(10, int)])
+    run(5, 9000, np.r_[3, 8192 - 3, 8192, 1, 0])
+    run(3, 50, np.r_[20, 0, 30], zeros=1.0)
+    run(4, 60, np.r_[20, 0, 30, 5], ptr=np.array([3, 20, 20, 40, 52]))
+    run(4, 60, np.r_[20, 0, 30, 5], ptr=np.array([0, 30, 20, 50, 55]))
