@@ -975,6 +975,26 @@ int jlust_hip_convert_direct(const jlust_sparse *src, const jlust_sparse *dst,
                              int value_type, void *ws, int64_t ws_bytes,
                              jlust_stream_t stream, int64_t *count);
 
+/* CSR to BSR of blocks up to 8 x 8 without a sort, where each row's columns
+ * increase.  workspace: the device bytes of ws (256-byte aligned); 0: not a
+ * conversion of this kind.  count writes browptr (Int32[m/b1 + 1], origin of
+ * src) and *nnzb, the stored blocks; -1: columns that do not increase,
+ * pointers that are not canonical or block-rows past 8192 entries or 1024
+ * blocks: use the two steps.  It synchronises `stream`.  fill writes dst's
+ * block columns and values (nouter = *nnzb, pos2 the browptr of count, the
+ * same src and ws), stream-ordered.  Results as the two steps', bit for bit. */
+int jlust_hip_convert_blocks_workspace(const jlust_sparse *src, int32_t b1,
+                                       int32_t b2, int value_type,
+                                       int64_t *bytes);
+int jlust_hip_convert_blocks_count(const jlust_sparse *src, int32_t b1,
+                                   int32_t b2, int value_type, void *ws,
+                                   int64_t ws_bytes, jlust_stream_t stream,
+                                   int32_t *browptr, int64_t *nnzb);
+int jlust_hip_convert_blocks_fill(const jlust_sparse *src,
+                                  const jlust_sparse *dst, int value_type,
+                                  const void *ws, int64_t ws_bytes,
+                                  jlust_stream_t stream);
+
 /* Step 2: writes the target's buffers (caller-allocated with the sizes from
  * analyze; origin, extents and format equal to the source's and the analysed
  * target), stream-ordered. */

@@ -146,6 +146,9 @@ SIGNATURES = {
                                             ctypes.POINTER(_I64), ctypes.POINTER(_I64)]),
     "jlust_hip_convert_direct_workspace": (_INT, [_P, _I32, _INT, ctypes.POINTER(_I64)]),
     "jlust_hip_convert_direct": (_INT, [_P, _P, _INT, _P, _I64, _P, ctypes.POINTER(_I64)]),
+    "jlust_hip_convert_blocks_workspace": (_INT, [_P, _I32, _I32, _INT, ctypes.POINTER(_I64)]),
+    "jlust_hip_convert_blocks_count": (_INT, [_P, _I32, _I32, _INT, _P, _I64, _P, _P, ctypes.POINTER(_I64)]),
+    "jlust_hip_convert_blocks_fill": (_INT, [_P, _P, _INT, _P, _I64, _P]),
     "jlust_hip_convert_fill": (_INT, [_P, _P, _P]),
     "jlust_hip_convert_destroy": (_INT, [_P]),
     "jlust_hip_sparse_to_dense": (_INT, [_P, _INT, _P, _I64, _P]),

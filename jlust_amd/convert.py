@@ -135,6 +135,36 @@ def _convert_direct(u: USTensor, fmt: TensorFormat, src: Sparse, fid: int, dev):
     return USTensor((m, n), fmt, *out, None, u.origin)
 
 
+def _convert_blocks(u: USTensor, fmt: TensorFormat, src: Sparse, b1: int, b2: int, row_major: bool, dev):
+    """CSR to BSR of small blocks (jlust_hip_convert_blocks_*), or None where the
+    two steps of convert_format do it."""
+    L = _lib.lib()
+    vt = _VT[u.val.dtype]
+    need, nnzb = ctypes.c_int64(), ctypes.c_int64()
+    _lib.check(L.jlust_hip_convert_blocks_workspace(ctypes.byref(src), b1, b2, vt, ctypes.byref(need)),
+               "convert_blocks", fmt)
+    if need.value == 0:
+        return None
+    m, n = u.extents
+    i32 = dict(dtype=torch.int32, device=dev)
+    ws = torch.empty(need.value, dtype=torch.uint8, device=dev)
+    browptr = torch.empty(m // b1 + 1, **i32)
+    st = L.jlust_hip_convert_blocks_count(ctypes.byref(src), b1, b2, vt, _ptr(ws), need.value, _stream(dev),
+                                          browptr.data_ptr(), ctypes.byref(nnzb))
+    _lib.check(st, "convert_blocks", fmt)
+    no = nnzb.value
+    if no < 0:
+        return None
+    bcol, val = torch.empty(no, **i32), torch.empty(no * b1 * b2, dtype=u.val.dtype, device=dev)
+    dst = Sparse(format=FMT_BSR, origin=u.origin.offset, m=m, n=n, b1=b1, b2=b2, row_major_blocks=int(row_major),
+                 nnz=no * b1 * b2, nouter=no)
+    dst.val, dst.pos2, dst.crd2 = _ptr(val), browptr.data_ptr(), _ptr(bcol)
+    st = L.jlust_hip_convert_blocks_fill(ctypes.byref(src), ctypes.byref(dst), vt, _ptr(ws), need.value, _stream(dev))
+    _lib.check(st, "convert_blocks", fmt)
+    torch.cuda.current_stream(dev).synchronize()
+    return USTensor((m, n), fmt, (None, browptr, None, None), (None, bcol, None, None), val, None, u.origin)
+
+
 def convert_format(u: USTensor, fmt: TensorFormat, index_type=None, value_type=None) -> USTensor:
     """src/convert.jl:302-388 on the device: a new tensor in `fmt` with u's origin."""
     if index_type not in (None, torch.int32):
@@ -148,7 +178,8 @@ def convert_format(u: USTensor, fmt: TensorFormat, index_type=None, value_type=N
     fid, b1, b2, rm = _format_id(fmt)
     L = _lib.lib()
     with torch.cuda.device(dev):
-        direct = _convert_direct(u, fmt, src, fid, dev)
+        direct = (_convert_blocks(u, fmt, src, b1, b2, rm, dev) if fid == FMT_BSR else
+                  _convert_direct(u, fmt, src, fid, dev))
     if direct is not None:
         return direct
     h = ctypes.c_void_p()

@@ -16,8 +16,9 @@
 // max-scan), zero-drop compaction, stable LSD radix sort (rocPRIM) of packed
 // level keys with source positions as values, adjacent-key dedup, then the
 // target's pos/crd/val from the sorted keys.  CSR to CSC and CSC to CSR or COO
-// move whole entries by coordinate instead (convert_direct).  Integer work
-// only; values are moved as bits.
+// move whole entries by coordinate instead (convert_direct), and CSR to small
+// blocks goes by block-rows (convert_blocks).  Integer work only; values are
+// moved as bits.
 //
 // Also: sparse_to_dense (ext/KernelAbstractionsExt/ops/conversion.jl:47-65)
 // and the index shift of materialize's origin change (CUDAExt.jl:199-220).
@@ -684,6 +685,175 @@ __global__ __launch_bounds__(256) void sort_ptr_kernel(const uint32_t *__restric
     ptr[r] = (int32_t)(lo + origin);
 }
 
+// ------------------------------------------------- CSR to BSR, small blocks
+//
+// A block-row's entries are one stretch of a CSR's, and where each row's
+// columns increase its block columns are the union of a few sorted lists: no
+// sort.  The general path sorts every entry by a 64-bit key and fetches its
+// value by position.
+//
+// A wave takes a block-row.  bsr_heads_kernel finds each block's first stored
+// entry (no nonzero before it in its row's part of the block, and none in the
+// rows above, found by binary search), gathers their block columns in LDS,
+// puts them in order by counting and leaves them at the block-row's place in
+// heads.  bsr_blocks_kernel, after a scan of the counts, writes each entry to
+// its block, found by binary search among them.  Explicit zeros are dropped:
+// a block of nothing else is not stored.  Rows that do not increase, pointers
+// that do not cover the entries, block-rows past BR_ENTRIES entries or
+// BR_BLOCKS blocks go to the general path (a wave is too little for those).
+//
+// What bounds it: memory, the entries read twice and the blocks written once,
+// twice where zeros fill them up.
+constexpr int BR_WAVES = 4, BR_BLOCKS = 1024, BR_ENTRIES = 8192, BR_DIM = 8;
+
+// Orders a wave's LDS accesses (its lanes exchange values through LDS).
+__device__ __forceinline__ void br_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The least i in [lo, hi) with a[i] >= x, hi if none.
+__device__ __forceinline__ int br_lower(const int32_t *a, int lo, int hi, int x)
+{
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (a[mid] < x) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// flags[0] = 1: not for this path.  full[R]: the block-row's entries fill its
+// blocks.  count[mb] = 0.
+template <typename T, int B2>
+__global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse src, int64_t mb, int b1,
+                                                                  int32_t *__restrict__ heads,
+                                                                  int32_t *__restrict__ count,
+                                                                  uint8_t *__restrict__ full,
+                                                                  int32_t *__restrict__ flags)
+{
+    __shared__ int32_t lds[BR_WAVES][BR_BLOCKS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t R = (int64_t)blockIdx.x * BR_WAVES + wave;
+    if (R >= mb) {
+        if (R == mb && lane == 0) count[mb] = 0;
+        return;
+    }
+    int32_t *h = lds[wave];
+    const int32_t *ptr = src.pos2 + R * b1, *col = src.crd2;
+    const T *val = static_cast<const T *>(src.val);
+    const int32_t o = src.origin;
+    const int32_t at = (int32_t)((int64_t)ptr[min(lane, b1)] - o), next = __shfl_down(at, 1, 64);
+    const int32_t p0 = __builtin_amdgcn_readlane(at, 0), p1 = __builtin_amdgcn_readlane(at, b1);
+    const bool off = at < 0 || at > src.nnz || (lane < b1 && next < at) || (lane == 0 && R == 0 && at != 0) ||
+                     (lane == b1 && R == mb - 1 && at != src.nnz);
+    if (__ballot(off) != 0 || p1 - p0 > BR_ENTRIES) {
+        if (lane == 0) flags[0] = 1;
+        return;
+    }
+    int nb = 0, nz = 0;
+    bool bad = false;
+    for (int q0 = p0; q0 < p1; q0 += 64) {
+        const int p = q0 + lane;
+        bool head = false;
+        int bc = 0;
+        const bool in = p < p1;
+        int r = 0, rs = p0;
+        for (int i = 1; i < b1; ++i) {
+            const int32_t s = __builtin_amdgcn_readlane(at, i);
+            if (s <= p) {
+                r = i;
+                rs = s;
+            }
+        }
+        if (in) {
+            const int c = col[p] - o;
+            bad = bad || c < 0 || c >= src.n || (p > rs && col[p - 1] - o >= c);
+            bc = c / B2;
+            head = val[p] != T(0);
+            const int first = bc * B2 + o;                // the block's first column, as stored
+            nz += head;
+            // Nonzeros of the block before it: in its row, then in those above.
+            for (int q = p - 1; head && q >= rs && q > p - B2 && col[q] >= first; --q) head = val[q] == T(0);
+            int s = p0;
+            for (int i = 0; i < b1 - 1; ++i) {
+                const int e = __builtin_amdgcn_readlane(at, i + 1);
+                if (head && i < r) {
+                    int q = br_lower(col, s, e, first);
+                    for (; head && q < e && col[q] < first + B2; ++q) head = val[q] == T(0);
+                }
+                s = e;
+            }
+        }
+        const uint64_t m = __ballot(head);
+        const int k = nb + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        if (head && k < BR_BLOCKS) h[k] = bc;
+        nb += __popcll(m);
+    }
+    if (__ballot(bad) != 0 || nb > BR_BLOCKS) {
+        if (lane == 0) flags[0] = 1;
+        return;
+    }
+    br_wave_sync();
+    for (int i = lane; i < nb; i += 64) {
+        const int x = h[i];
+        int rank = 0;
+        for (int j = 0; j < nb; ++j) rank += h[j] < x;
+        heads[p0 + rank] = x;
+    }
+#pragma unroll
+    for (int d = 32; d; d >>= 1) nz += __shfl_xor(nz, d, 64);
+    if (lane == 0) {
+        count[R] = nb;
+        full[R] = nz == nb * b1 * B2;
+    }
+}
+
+template <typename T, int B2>
+__global__ __launch_bounds__(64 * BR_WAVES) void bsr_blocks_kernel(jlust_sparse src, int64_t mb, int b1, int row_major,
+                                                                   const int32_t *__restrict__ heads,
+                                                                   const uint8_t *__restrict__ full,
+                                                                   const int32_t *__restrict__ browptr, int64_t nnzb,
+                                                                   int32_t *__restrict__ bcol, T *__restrict__ out)
+{
+    __shared__ int32_t lds[BR_WAVES][BR_BLOCKS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t R = (int64_t)blockIdx.x * BR_WAVES + wave;
+    if (R >= mb) return;
+    int32_t *h = lds[wave];
+    const int32_t o = src.origin;
+    const int32_t *ptr = src.pos2 + R * b1, *col = src.crd2;
+    const T *val = static_cast<const T *>(src.val);
+    const int32_t at = ptr[min(lane, b1)] - o;
+    const int32_t p0 = __builtin_amdgcn_readlane(at, 0), p1 = __builtin_amdgcn_readlane(at, b1);
+    const int64_t base = (int64_t)browptr[R] - o, end = (int64_t)browptr[R + 1] - o;
+    if (base < 0 || end > nnzb || end < base || end - base > min(p1 - p0, BR_BLOCKS)) return;
+    const int nb = (int)(end - base), bb = b1 * B2;
+    for (int i = lane; i < nb; i += 64) {
+        const int x = heads[p0 + i];
+        h[i] = x;
+        bcol[base + i] = x + o;
+    }
+    T *blocks = out + base * bb;
+    if (!full[R]) {
+        for (int i = lane; i < nb * bb; i += 64) blocks[i] = T(0);
+        __threadfence_block();                            // these stores, then the entries'
+    }
+    br_wave_sync();
+    for (int q0 = p0; q0 < p1; q0 += 64) {
+        const int p = q0 + lane;
+        int r = 0;
+        for (int i = 1; i < b1; ++i) r += __builtin_amdgcn_readlane(at, i) <= p;
+        if (p >= p1) continue;
+        const int c = col[p] - o, bc = c / B2, cc = c - bc * B2;
+        const T v = val[p];
+        if (v == T(0)) continue;
+        const int k = br_lower(h, 0, nb, bc);
+        if (k < nb) blocks[(int64_t)k * bb + (row_major ? r * B2 + cc : cc * b1 + r)] = v;
+    }
+}
+
 // ----------------------------------------------------------------- host
 
 int check_format(int fmt) { return fmt >= JLUST_FORMAT_CSR && fmt <= JLUST_FORMAT_BSR; }
@@ -1142,6 +1312,98 @@ int direct_run(const jlust_sparse *src, const jlust_sparse *dst, const DirectLay
     return JLUST_STATUS_SUCCESS;
 }
 
+// CSR to BSR by block-rows: the workspace (bytes == 0: not a conversion of
+// this kind).
+struct BlocksLayout {
+    int64_t mb = 0;
+    size_t tmp = 0, bytes = 0;
+};
+
+int blocks_layout(const jlust_sparse *src, int b1, int b2, BlocksLayout *out)
+{
+    *out = BlocksLayout();
+    if (src->format != JLUST_FORMAT_CSR || b1 > BR_DIM || b2 > BR_DIM || src->nnz == 0 || src->m == 0)
+        return JLUST_STATUS_SUCCESS;
+    out->mb = src->m / b1;
+    // A wave to a block-row: where almost all are empty the general path's
+    // passes over the entries are the better ones.
+    if (out->mb > 16 * src->nnz) return JLUST_STATUS_SUCCESS;
+    int32_t *v = nullptr;
+    JLUST_HIP_TRY(rocprim::exclusive_scan(nullptr, out->tmp, v, v, 0, (size_t)out->mb + 1, rocprim::plus<int32_t>(),
+                                          (hipStream_t)0));
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    // flags, heads, counts, full, the scan's
+    out->bytes = 256 + up(4 * (size_t)src->nnz) + up(4 * ((size_t)out->mb + 1)) + up((size_t)out->mb) + up(out->tmp);
+    return JLUST_STATUS_SUCCESS;
+}
+
+struct BlocksWs {
+    int32_t *flags, *heads, *count;
+    uint8_t *full;
+    void *tmp;
+};
+
+BlocksWs blocks_ws(const jlust_sparse *src, const BlocksLayout &bl, void *ws)
+{
+    char *b = (char *)ws;
+    auto take = [&](size_t bytes) { char *p = b; b += (bytes + 255) / 256 * 256; return p; };
+    BlocksWs w;
+    w.flags = (int32_t *)take(256);
+    w.heads = (int32_t *)take(4 * (size_t)src->nnz);
+    w.count = (int32_t *)take(4 * ((size_t)bl.mb + 1));
+    w.full = (uint8_t *)take((size_t)bl.mb);
+    w.tmp = take(bl.tmp);
+    return w;
+}
+
+#define JLUST_BY_B2(b2, CALL)                                              \
+    switch (b2) {                                                          \
+    case 1: CALL(1); break;                                                \
+    case 2: CALL(2); break;                                                \
+    case 3: CALL(3); break;                                                \
+    case 4: CALL(4); break;                                                \
+    case 5: CALL(5); break;                                                \
+    case 6: CALL(6); break;                                                \
+    case 7: CALL(7); break;                                                \
+    default: CALL(8);                                                      \
+    }
+
+template <typename T>
+int blocks_count(const jlust_sparse *src, int b1, int b2, const BlocksLayout &bl, const BlocksWs &w, int32_t *browptr,
+                 int64_t *nnzb, hipStream_t st)
+{
+    JLUST_HIP_TRY(hipMemsetAsync(w.flags, 0, 256, st));
+    const dim3 grid((unsigned)(bl.mb / BR_WAVES + 1)), block(64 * BR_WAVES);
+#define JLUST_HEADS(B2)                                                                                          \
+    hipLaunchKernelGGL((bsr_heads_kernel<T, B2>), grid, block, 0, st, *src, bl.mb, b1, w.heads, w.count, w.full, \
+                       w.flags)
+    JLUST_BY_B2(b2, JLUST_HEADS)
+#undef JLUST_HEADS
+    if (int e = check_launch("bsr_heads_kernel")) return e;
+    int32_t bad = 0, total = 0;
+    JLUST_HIP_TRY(hipMemcpyAsync(&bad, w.flags, 4, hipMemcpyDeviceToHost, st));
+    size_t need = bl.tmp;
+    JLUST_HIP_TRY(rocprim::exclusive_scan(w.tmp, need, w.count, browptr, src->origin, (size_t)bl.mb + 1,
+                                          rocprim::plus<int32_t>(), st));
+    JLUST_HIP_TRY(hipMemcpyAsync(&total, browptr + bl.mb, 4, hipMemcpyDeviceToHost, st));
+    JLUST_HIP_TRY(hipStreamSynchronize(st));
+    if (!bad) *nnzb = (int64_t)total - src->origin;
+    return JLUST_STATUS_SUCCESS;
+}
+
+template <typename T>
+int blocks_fill(const jlust_sparse *src, const jlust_sparse *dst, const BlocksLayout &bl, const BlocksWs &w,
+                hipStream_t st)
+{
+    const dim3 grid((unsigned)((bl.mb + BR_WAVES - 1) / BR_WAVES)), block(64 * BR_WAVES);
+#define JLUST_BLOCKS(B2)                                                                                      \
+    hipLaunchKernelGGL((bsr_blocks_kernel<T, B2>), grid, block, 0, st, *src, bl.mb, dst->b1,                  \
+                       dst->row_major_blocks != 0, w.heads, w.full, dst->pos2, dst->nouter, dst->crd2, (T *)dst->val)
+    JLUST_BY_B2(dst->b2, JLUST_BLOCKS)
+#undef JLUST_BLOCKS
+    return check_launch("bsr_blocks_kernel");
+}
+
 template <typename T>
 int fill(const jlust_convert *h, const jlust_sparse *d, hipStream_t st)
 {
@@ -1387,6 +1649,64 @@ extern "C" int jlust_hip_convert_direct(const jlust_sparse *src, const jlust_spa
         return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_direct: null device pointer");
     return value_type == 0 ? direct_run<double>(src, dst, dl, ws, count, (hipStream_t)stream)
                            : direct_run<float>(src, dst, dl, ws, count, (hipStream_t)stream);
+}
+
+extern "C" int jlust_hip_convert_blocks_workspace(const jlust_sparse *src, int32_t b1, int32_t b2, int value_type,
+                                                  int64_t *bytes)
+{
+    clear_error();
+    if (!bytes) return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: null output pointer");
+    *bytes = 0;
+    KeyLayout L;
+    if (int st = analyze_args(src, JLUST_FORMAT_BSR, b1, b2, 1, value_type, &L)) return st;
+    if (int st = require_device(nullptr)) return st;
+    BlocksLayout bl;
+    if (int st = blocks_layout(src, b1, b2, &bl)) return st;
+    *bytes = (int64_t)bl.bytes;
+    return JLUST_STATUS_SUCCESS;
+}
+
+extern "C" int jlust_hip_convert_blocks_count(const jlust_sparse *src, int32_t b1, int32_t b2, int value_type, void *ws,
+                                              int64_t ws_bytes, jlust_stream_t stream, int32_t *browptr, int64_t *nnzb)
+{
+    clear_error();
+    if (!nnzb) return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: null output pointer");
+    *nnzb = -1;
+    KeyLayout L;
+    if (int st = analyze_args(src, JLUST_FORMAT_BSR, b1, b2, 1, value_type, &L)) return st;
+    if (int st = require_device(nullptr)) return st;
+    BlocksLayout bl;
+    if (int st = blocks_layout(src, b1, b2, &bl)) return st;
+    if (bl.bytes == 0) return JLUST_STATUS_SUCCESS;
+    if (!ws || (uintptr_t)ws % 256 || ws_bytes < (int64_t)bl.bytes || !browptr)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: workspace of %lld bytes, %zu needed at 256",
+                    (long long)ws_bytes, bl.bytes);
+    const BlocksWs w = blocks_ws(src, bl, ws);
+    return value_type == 0 ? blocks_count<double>(src, b1, b2, bl, w, browptr, nnzb, (hipStream_t)stream)
+                           : blocks_count<float>(src, b1, b2, bl, w, browptr, nnzb, (hipStream_t)stream);
+}
+
+extern "C" int jlust_hip_convert_blocks_fill(const jlust_sparse *src, const jlust_sparse *dst, int value_type,
+                                             const void *ws, int64_t ws_bytes, jlust_stream_t stream)
+{
+    clear_error();
+    if (!dst || dst->format != JLUST_FORMAT_BSR)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: null or other target");
+    KeyLayout L;
+    if (int st = analyze_args(src, JLUST_FORMAT_BSR, dst->b1, dst->b2, 1, value_type, &L)) return st;
+    if (int st = require_device(nullptr)) return st;
+    BlocksLayout bl;
+    if (int st = blocks_layout(src, dst->b1, dst->b2, &bl)) return st;
+    if (bl.bytes == 0 || !ws || (uintptr_t)ws % 256 || ws_bytes < (int64_t)bl.bytes)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: not this conversion, or its workspace");
+    if (dst->origin != src->origin || dst->m != src->m || dst->n != src->n || dst->nouter < 0 ||
+        dst->nnz != dst->nouter * dst->b1 * dst->b2)
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: target does not match the source");
+    if (!dst->pos2 || bad_ptr(dst->crd2, dst->nouter) || bad_ptr(dst->val, dst->nnz))
+        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert_blocks: null device pointer");
+    const BlocksWs w = blocks_ws(src, bl, const_cast<void *>(ws));
+    return value_type == 0 ? blocks_fill<double>(src, dst, bl, w, (hipStream_t)stream)
+                           : blocks_fill<float>(src, dst, bl, w, (hipStream_t)stream);
 }
 
 extern "C" int jlust_hip_convert_fill(jlust_convert_t h, const jlust_sparse *dst, jlust_stream_t stream)

@@ -350,3 +350,83 @@ def test_direct_equals_two_steps(J, src, dst, dtype, origin, monkeypatch):
     run(3, 50, np.r_[20, 0, 30], zeros=1.0)
     run(4, 60, np.r_[20, 0, 30, 5], ptr=np.array([3, 20, 20, 40, 52]))
     run(4, 60, np.r_[20, 0, 30, 5], ptr=np.array([0, 30, 20, 50, 55]))
+
+
+@pytest.mark.parametrize("b1,b2,rm", [(1, 1, True), (2, 2, False), (3, 3, True), (4, 4, True), (5, 2, False), (8, 8, True),
+                                      (1, 8, True), (7, 1, False)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("origin", [0, 1])
+def test_blocks_equal_two_steps(J, b1, b2, rm, dtype, origin, monkeypatch):
+    """convert_blocks against the two-step conversion, bit for bit: dense and
+    ragged blocks, explicit zeros (-0.0, whole blocks of them, the first entry
+    of a block), NaN, empty block-rows, block-rows of 0, 1, 63 to 65 entries and
+    more, the last block-row of a workgroup's four, and what it leaves to the
+    two steps: unordered and repeated columns, pointers that do not cover the
+    entries, block-rows past 8192 entries or 1024 blocks."""
+    import torch
+    from jlust_amd import convert as CV
+    rng = np.random.default_rng(23)
+    og = J.OneBased() if origin else J.ZeroBased()
+    taken = []
+    blocks = CV._convert_blocks
+
+    def counted(*a):
+        r = blocks(*a)
+        taken.append(r is not None)
+        return r
+
+    def check(mb, nb, rows, path=True, zeros=0.0, ptr=None):
+        """rows: the columns of each row, in storage order."""
+        assert len(rows) == mb * b1
+        ends = np.r_[0, np.cumsum([len(r) for r in rows])]
+        c = np.concatenate([np.asarray(r, np.int64) for r in rows]) if ends[-1] else np.zeros(0, np.int64)
+        v = rng.standard_normal(c.size).astype(dtype)
+        z = rng.random(c.size) < zeros
+        v[z] = 0.0
+        v[np.flatnonzero(z)[::2]] = -0.0
+        if c.size > 3 and zeros < 1:
+            v[2] = np.nan
+        p = (ends if ptr is None else ptr) + origin
+        u = J.csr_tensor(*(torch.from_numpy(t).cuda() for t in (p.astype(np.int32), (c + origin).astype(np.int32), v)),
+                         (mb * b1, nb * b2), og)
+        out = []
+        for f in (counted, lambda *a: None):
+            with monkeypatch.context() as mp:
+                mp.setattr(CV, "_convert_blocks", f)
+                out.append(J.convert_format(u, fmt_of(J, "BSR", b1, b2, rm)))
+        assert taken.pop() == path
+        x, y = out
+        it = torch.int64 if dtype == np.float64 else torch.int32
+        assert torch.equal(x.pos_buffers[1], y.pos_buffers[1]) and torch.equal(x.crd_buffers[1], y.crd_buffers[1])
+        assert torch.equal(x.val.view(it), y.val.view(it))
+
+    def pick(n, k):
+        return np.sort(rng.choice(n, min(k, n), replace=False))
+
+    def dense(mb, nb, k):
+        out = []
+        for _ in range(mb):
+            at = pick(nb, k)
+            out += [(at[:, None] * b2 + np.arange(b2)).reshape(-1)] * b1
+        return out
+
+    for mb, nb, k in ((1, 1, 1), (3, 9, 4), (4, 40, 27), (5, 300, 70), (41, 60, 16)):
+        check(mb, nb, dense(mb, nb, k))
+        check(mb, nb, dense(mb, nb, k), zeros=0.3)
+        check(mb, nb, [pick(nb * b2, int(rng.integers(0, 2 * k))) for _ in range(mb * b1 - 1)] + [[nb * b2 - 1]],
+              zeros=0.2)
+    for n in (63, 64, 65, 129):                             # entries of a block-row, all in its last row
+        check(3, 200, [[]] * (2 * b1 - 1) + [pick(200 * b2, n)] + [[]] * b1)
+    check(4, 20, dense(4, 20, 7), zeros=1.0)
+    wide = 1024
+    check(2, 1030, dense(1, 1030, wide if wide * b1 * b2 <= 8192 else 8192 // (b1 * b2)) + [[1]] * b1)
+    check(2, 1030, dense(1, 1030, 1025) + [[1]] * b1, path=False)
+    check(1, 9000, [pick(9000 * b2, 8193)] + [[]] * (b1 - 1), path=False)
+    r = dense(2, 20, 9)
+    r[0] = np.r_[3, 1] if b2 * 20 > 3 else r[0]
+    check(2, 20, r, path=False)
+    r = dense(2, 20, 9)
+    r[-1] = np.r_[4, 4]
+    check(2, 20, r, path=False)
+    r = [np.array([0, 5])] * (4 * b1)
+    check(4, 20, r, path=False, ptr=np.r_[1, np.arange(1, 4 * b1 + 1) * 2])
