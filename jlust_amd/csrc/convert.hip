@@ -313,11 +313,12 @@ __global__ void shift_kernel(int64_t n, int32_t *__restrict__ dst, const int32_t
 // neighbours, meet in one L2.
 //
 // 16M f64 entries of 1,000,003 columns (512 MB of traffic a pass): the first
-// pass' count 67 us, the second's 21, each move 166 (3.1 TB/s; 16 entries a
-// thread without spills, two tiles a CU; 1,024 threads of 8 in 64 registers
-// took 195, with spills 285), scans 18, repeats 24, pointers 28: a whole
-// conversion 556 us, 1,201 by the general path.  10,007 rows of 9: 126 us, 260
-// there, both mostly launches.
+// pass' count 28 us (67 when it read the values too, to drop zeros), the
+// second's 20, each move 163 (3.1 TB/s; 16 entries a thread without spills, two
+// tiles a CU; 1,024 threads of 8 in 64 registers took 195, with spills 285),
+// scans 18, repeats 24, pointers 28: a whole conversion 508 us, 1,196 by the
+// general path.  With 5 % of zeros, which cost a second run, 1,113 us against
+// 3,992.  10,007 rows of 9: 126 us, 260 there, both mostly launches.
 constexpr int CS_THREADS = 512, CS_WAVES = CS_THREADS / 64, CS_ITEMS = 16;
 constexpr int CS_TILE = CS_THREADS * CS_ITEMS;
 constexpr int CC_THREADS = 1024, CC_ITEMS = CS_TILE / CC_THREADS;      // the counting kernel
@@ -336,17 +337,22 @@ __device__ __forceinline__ int64_t sort_tile(int64_t ntiles)
     return (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
 }
 
-enum { CS_BAD = 0, CS_POINTERS = 1, CS_REPEATS = 2, CS_COUNT = 3 };     // flags[]
+enum { CS_BAD = 0, CS_POINTERS = 1, CS_REPEATS = 2, CS_COUNT = 3, CS_ZEROS = 4 };     // flags[]
+
+// The source of a pass: the entries of the pass before, the source's, or the
+// source's without its zeros.
+enum SortFrom { CS_ENTRIES, CS_SOURCE, CS_NONZEROS };
 
 // hist[digit * ntiles + tile]: how often the tile's entries hold the digit.
-// The first pass reads the source, drops zeros and checks the coordinates and
-// the segment pointers; the others read the keys of the pass before.
-template <typename T, bool FIRST>
+// The first pass reads the source and checks the coordinates and the segment
+// pointers; the others read the keys of the pass before.
+template <typename T, int FROM>
 __global__ __launch_bounds__(CC_THREADS) void sort_count_kernel(jlust_sparse src, int64_t nseg, int64_t major_dim,
                                                                 const uint32_t *__restrict__ keys, SortPass ps,
                                                                 int32_t *__restrict__ hist,
                                                                 int32_t *__restrict__ flags)
 {
+    constexpr bool FIRST = FROM != CS_ENTRIES;
     __shared__ uint32_t h[CS_DIGITS];
     const int64_t tile = sort_tile(ps.ntiles);
     if (tile >= ps.ntiles) return;
@@ -368,7 +374,9 @@ __global__ __launch_bounds__(CC_THREADS) void sort_count_kernel(jlust_sparse src
                 key[j] = (int64_t)src.crd2[p] - src.origin;
                 const bool inb = key[j] >= 0 && key[j] < major_dim;
                 bad = bad || !inb;
-                valid[j] = valid[j] && inb && static_cast<const T *>(src.val)[p] != T(0);  // no -0.0; NaN kept
+                valid[j] = valid[j] && inb;
+                if (FROM == CS_NONZEROS)                         // no -0.0; NaN kept
+                    valid[j] = valid[j] && static_cast<const T *>(src.val)[p] != T(0);
             } else {
                 key[j] = keys[p];
             }
@@ -409,7 +417,7 @@ __device__ __forceinline__ int32_t segment_of(const int32_t *__restrict__ ptr, i
 // One pass: the entries of each tile to their places by digit, hist holding
 // the exclusive scan of the counts.  okey gets the coordinate + kadd, ominor
 // the segment + madd (the target's index origin in the last pass).
-template <typename T, bool FIRST>
+template <typename T, int FROM>
 __global__ __launch_bounds__(CS_THREADS, 4) void sort_move_kernel(jlust_sparse src, int64_t nseg, int64_t major_dim,
                                                                   const uint32_t *__restrict__ ikey,
                                                                   const uint32_t *__restrict__ iminor,
@@ -420,6 +428,7 @@ __global__ __launch_bounds__(CS_THREADS, 4) void sort_move_kernel(jlust_sparse s
                                                                   uint32_t *__restrict__ ominor,
                                                                   T *__restrict__ oval, uint32_t kadd, uint32_t madd)
 {
+    constexpr bool FIRST = FROM != CS_ENTRIES;
     // In turn: segment marks, the waves' digit counts, the entries in order.
     __shared__ __align__(16) char lds[CS_TILE * 8];
     __shared__ int32_t delta[CS_DIGITS];
@@ -432,8 +441,8 @@ __global__ __launch_bounds__(CS_THREADS, 4) void sort_move_kernel(jlust_sparse s
     const int64_t t0 = tile * CS_TILE, t1 = min(t0 + CS_TILE, n);
     if (t0 >= n) return;
     const int base = wave * (64 * CS_ITEMS) + lane;       // this thread's entries: base + 64 j
-    // An entry's value stays in memory until its place is known (the first
-    // pass reads it here too, to drop zeros).
+    // An entry's value stays in memory until its place is known, except where
+    // zeros are dropped.
     const int last = (int)(t1 - t0) - 1;
     const T *value = (FIRST ? static_cast<const T *>(src.val) : ival) + t0;
     const uint32_t *keys = (FIRST ? reinterpret_cast<const uint32_t *>(src.crd2) : ikey) + t0;
@@ -443,12 +452,13 @@ __global__ __launch_bounds__(CS_THREADS, 4) void sort_move_kernel(jlust_sparse s
     for (int j = 0; j < CS_ITEMS; ++j) {
         const uint32_t i = (uint32_t)min(base + 64 * j, last) & (CS_TILE - 1);
         key[j] = keys[i];
-        if (FIRST) val[j] = value[i];
+        if (FROM == CS_NONZEROS) val[j] = value[i];
     }
 #pragma unroll
     for (int j = 0; j < CS_ITEMS; ++j) {
         if (FIRST) key[j] -= (uint32_t)src.origin;
-        const bool in = base + 64 * j <= last, ok = !FIRST | (((int64_t)key[j] < major_dim) & (val[j] != T(0)));
+        const bool in = base + 64 * j <= last,
+                   ok = !FIRST | (((int64_t)key[j] < major_dim) & (FROM != CS_NONZEROS || val[j] != T(0)));
         valid |= (uint32_t)(in & ok) << j;
     }
     if (FIRST) {
@@ -581,6 +591,12 @@ __global__ __launch_bounds__(CS_THREADS, 4) void sort_move_kernel(jlust_sparse s
         const uint32_t i = min(here + 64 * j, (uint32_t)last) & (CS_TILE - 1);
         if (!FIRST) minor[j] = iminor[t0 + i];
         val[j] = value[i];
+    }
+    if (FROM == CS_SOURCE) {
+        bool zero = false;
+#pragma unroll
+        for (int j = 0; j < CS_ITEMS; ++j) zero = zero || val[j] == T(0);
+        if (zero) flags[CS_ZEROS] = 1;
     }
     __syncthreads();
 #pragma unroll
@@ -1241,50 +1257,63 @@ int direct_run(const jlust_sparse *src, const jlust_sparse *dst, const DirectLay
     const bool coo = dst->format == JLUST_FORMAT_COO;
     const uint32_t o = (uint32_t)dst->origin;
     const Entries out = {coo ? (uint32_t *)dst->crd1 : major, (uint32_t *)dst->crd2, (T *)dst->val};
-    JLUST_HIP_TRY(hipMemsetAsync(flags, 0, 16 * sizeof(int32_t), st));
-    Entries in = {nullptr, nullptr, nullptr};
     const dim3 grid((unsigned)((dl.ntiles + 7) / 8 * 8)), block(CS_THREADS);
-    for (int p = 0; p < dl.passes; ++p) {
-        const SortPass ps = {p * dl.bits, dl.bits, dl.ntiles};
-        const bool last = p == dl.passes - 1;
-        const Entries to = last ? out : p % 2 ? e2 : e1;
-        if (p == 0)
-            hipLaunchKernelGGL((sort_count_kernel<T, true>), grid, dim3(CC_THREADS), 0, st, *src, dl.nseg, dl.major_dim, in.key, ps,
-                               hist, flags);
-        else
-            hipLaunchKernelGGL((sort_count_kernel<T, false>), grid, dim3(CC_THREADS), 0, st, *src, dl.nseg, dl.major_dim, in.key,
-                               ps, hist, flags);
-        if (int e = check_launch("sort_count_kernel")) return e;
-        size_t need = dl.tmp;
-        JLUST_HIP_TRY(rocprim::exclusive_scan(tmp, need, hist, hist, 0, dl.hist, rocprim::plus<int32_t>(), st));
-        const uint32_t kadd = last && coo ? o : 0, madd = last ? o : 0;
-        if (p == 0)
-            hipLaunchKernelGGL((sort_move_kernel<T, true>), grid, block, 0, st, *src, dl.nseg, dl.major_dim, in.key,
-                               in.minor, in.val, ps, hist, flags, to.key, to.minor, to.val, kadd, madd);
-        else
-            hipLaunchKernelGGL((sort_move_kernel<T, false>), grid, block, 0, st, *src, dl.nseg, dl.major_dim, in.key,
-                               in.minor, in.val, ps, hist, flags, to.key, to.minor, to.val, kadd, madd);
-        if (int e = check_launch("sort_move_kernel")) return e;
-        in = to;
-    }
+    // Zeros are to be dropped, and there are none as a rule: the first count
+    // reads the coordinates alone, and where a pass meets a zero all is done
+    // again without them.
+    auto passes = [&](bool nonzeros) -> int {
+        JLUST_HIP_TRY(hipMemsetAsync(flags, 0, 16 * sizeof(int32_t), st));
+        Entries in = {nullptr, nullptr, nullptr};
+        for (int p = 0; p < dl.passes; ++p) {
+            const SortPass ps = {p * dl.bits, dl.bits, dl.ntiles};
+            const bool last = p == dl.passes - 1;
+            const Entries to = last ? out : p % 2 ? e2 : e1;
+#define JLUST_COUNT(FROM)                                                                                         \
+            hipLaunchKernelGGL((sort_count_kernel<T, FROM>), grid, dim3(CC_THREADS), 0, st, *src, dl.nseg, dl.major_dim, \
+                               in.key, ps, hist, flags)
+#define JLUST_MOVE(FROM)                                                                                          \
+            hipLaunchKernelGGL((sort_move_kernel<T, FROM>), grid, block, 0, st, *src, dl.nseg, dl.major_dim, in.key,  \
+                               in.minor, in.val, ps, hist, flags, to.key, to.minor, to.val, kadd, madd)
+            if (p > 0) JLUST_COUNT(CS_ENTRIES);
+            else if (nonzeros) JLUST_COUNT(CS_NONZEROS);
+            else JLUST_COUNT(CS_SOURCE);
+            if (int e = check_launch("sort_count_kernel")) return e;
+            size_t need = dl.tmp;
+            JLUST_HIP_TRY(rocprim::exclusive_scan(tmp, need, hist, hist, 0, dl.hist, rocprim::plus<int32_t>(), st));
+            const uint32_t kadd = last && coo ? o : 0, madd = last ? o : 0;
+            if (p > 0) JLUST_MOVE(CS_ENTRIES);
+            else if (nonzeros) JLUST_MOVE(CS_NONZEROS);
+            else JLUST_MOVE(CS_SOURCE);
+#undef JLUST_COUNT
+#undef JLUST_MOVE
+            if (int e = check_launch("sort_move_kernel")) return e;
+            in = to;
+        }
+        return JLUST_STATUS_SUCCESS;
+    };
     auto pointers = [&]() -> int {
         hipLaunchKernelGGL(sort_ptr_kernel, dim3(cv_grid(dl.major_dim + 1)), dim3(256), 0, st, major, flags + CS_COUNT,
                            dl.major_dim, dst->origin, dst->pos2);
         return check_launch("sort_ptr_kernel");
     };
-    if (!coo) {
-        hipLaunchKernelGGL(sort_repeats_kernel, dim3(cv_grid((N + 3) / 4)), dim3(256), 0, st, N, major,
-                           (uint32_t *)dst->crd2, flags, (int32_t *)nullptr);
-        if (int e = check_launch("sort_repeats_kernel")) return e;
-        if (int e = pointers()) return e;
+    int32_t got[5] = {0, 0, 0, 0, 0};
+    for (int nonzeros = 0; nonzeros < 2; ++nonzeros) {
+        if (int e = passes(nonzeros != 0)) return e;
+        if (!coo) {
+            hipLaunchKernelGGL(sort_repeats_kernel, dim3(cv_grid((N + 3) / 4)), dim3(256), 0, st, N, major,
+                               (uint32_t *)dst->crd2, flags, (int32_t *)nullptr);
+            if (int e = check_launch("sort_repeats_kernel")) return e;
+            if (int e = pointers()) return e;
+        }
+        JLUST_HIP_TRY(hipMemcpyAsync(got, flags, sizeof(got), hipMemcpyDeviceToHost, st));
+        JLUST_HIP_TRY(hipStreamSynchronize(st));
+        if (got[CS_POINTERS]) return JLUST_STATUS_SUCCESS;      // *count stays -1
+        if (got[CS_BAD])
+            return fail(JLUST_STATUS_INVALID_ARGUMENT,
+                        "convert: a stored coordinate lies outside the %lld x %lld extents", (long long)src->m,
+                        (long long)src->n);
+        if (!got[CS_ZEROS]) break;
     }
-    int32_t got[4] = {0, 0, 0, 0};
-    JLUST_HIP_TRY(hipMemcpyAsync(got, flags, sizeof(got), hipMemcpyDeviceToHost, st));
-    JLUST_HIP_TRY(hipStreamSynchronize(st));
-    if (got[CS_POINTERS]) return JLUST_STATUS_SUCCESS;      // *count stays -1
-    if (got[CS_BAD])
-        return fail(JLUST_STATUS_INVALID_ARGUMENT, "convert: a stored coordinate lies outside the %lld x %lld extents",
-                    (long long)src->m, (long long)src->n);
     int64_t C = got[CS_COUNT];
     if (coo && dst->pos1) {
         hipLaunchKernelGGL(pair_kernel, dim3(1), dim3(64), 0, st, dst->pos1, dst->origin, (int32_t)(C + dst->origin));
