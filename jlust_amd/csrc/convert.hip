@@ -718,9 +718,12 @@ __global__ __launch_bounds__(256) void sort_ptr_kernel(const uint32_t *__restric
 // that do not cover the entries, block-rows past BR_ENTRIES entries or
 // BR_BLOCKS blocks go to the general path (a wave is too little for those).
 //
-// What bounds it: memory, the entries read twice and the blocks written once,
-// twice where zeros fill them up.
-constexpr int BR_WAVES = 4, BR_BLOCKS = 1024, BR_ENTRIES = 8192, BR_DIM = 8;
+// What bounds it: the searches and the serial loop of a wave in the first
+// kernel, memory in the second (entries read, blocks written, twice where zeros
+// fill them up).  Mesh of 59,200 nodes, 4 x 4 f64, 24M entries: 187 and 168 us, a
+// whole conversion 419 (2,038 by the general path); 3 x 3 f32, 24,000 nodes: 132
+// (762); 400k uniform rows of 8 to 8 x 8 blocks, mostly zeros: 623 (937).
+constexpr int BR_WAVES = 4, BR_BLOCKS = 1024, BR_ENTRIES = 8192, BR_STAGE = 2048, BR_DIM = 8;
 
 // Orders a wave's LDS accesses (its lanes exchange values through LDS).
 __device__ __forceinline__ void br_wave_sync()
@@ -740,23 +743,35 @@ __device__ __forceinline__ int br_lower(const int32_t *a, int lo, int hi, int x)
     return lo;
 }
 
+// flags[0] = 1 where a block-row is too long or the pointers do not cover the
+// entries: found before the others' entries are read.
+__global__ __launch_bounds__(256) void bsr_long_kernel(jlust_sparse src, int64_t mb, int b1, int32_t *__restrict__ flags)
+{
+    const int64_t R = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (R >= mb) return;
+    const int64_t a = (int64_t)src.pos2[R * b1] - src.origin, b = (int64_t)src.pos2[(R + 1) * b1] - src.origin;
+    if ((R == 0 && a != 0) || (R == mb - 1 && b != src.nnz) || b - a > BR_ENTRIES) flags[0] = 1;
+}
+
 // flags[0] = 1: not for this path.  full[R]: the block-row's entries fill its
-// blocks.  count[mb] = 0.
+// blocks.  count[mb] = 0.  stage: entries of a block-row that fit its LDS.
 template <typename T, int B2>
-__global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse src, int64_t mb, int b1,
+__global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse src, int64_t mb, int b1, int stage,
                                                                   int32_t *__restrict__ heads,
                                                                   int32_t *__restrict__ count,
                                                                   uint8_t *__restrict__ full,
                                                                   int32_t *__restrict__ flags)
 {
-    __shared__ int32_t lds[BR_WAVES][BR_BLOCKS];
+    extern __shared__ int32_t br_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t R = (int64_t)blockIdx.x * BR_WAVES + wave;
     if (R >= mb) {
         if (R == mb && lane == 0) count[mb] = 0;
         return;
     }
-    int32_t *h = lds[wave];
+    if (flags[0]) return;
+    int32_t *h = br_lds + wave * (stage + BR_BLOCKS);
+    uint32_t *staged = reinterpret_cast<uint32_t *>(h + BR_BLOCKS);
     const int32_t *ptr = src.pos2 + R * b1, *col = src.crd2;
     const T *val = static_cast<const T *>(src.val);
     const int32_t o = src.origin;
@@ -770,42 +785,76 @@ __global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse s
     }
     int nb = 0, nz = 0;
     bool bad = false;
-    for (int q0 = p0; q0 < p1; q0 += 64) {
-        const int p = q0 + lane;
-        bool head = false;
-        int bc = 0;
-        const bool in = p < p1;
-        int r = 0, rs = p0;
-        for (int i = 1; i < b1; ++i) {
-            const int32_t s = __builtin_amdgcn_readlane(at, i);
-            if (s <= p) {
-                r = i;
-                rs = s;
-            }
-        }
-        if (in) {
-            const int c = col[p] - o;
-            bad = bad || c < 0 || c >= src.n || (p > rs && col[p - 1] - o >= c);
-            bc = c / B2;
-            head = val[p] != T(0);
-            const int first = bc * B2 + o;                // the block's first column, as stored
-            nz += head;
-            // Nonzeros of the block before it: in its row, then in those above.
-            for (int q = p - 1; head && q >= rs && q > p - B2 && col[q] >= first; --q) head = val[q] == T(0);
-            int s = p0;
-            for (int i = 0; i < b1 - 1; ++i) {
-                const int e = __builtin_amdgcn_readlane(at, i + 1);
-                if (head && i < r) {
-                    int q = br_lower(col, s, e, first);
-                    for (; head && q < e && col[q] < first + B2; ++q) head = val[q] == T(0);
+    // entry(p): twice the column of entry p, plus one if it is a zero.
+    auto find = [&](auto entry) {
+        for (int q0 = p0; q0 < p1; q0 += 64) {
+            const int p = q0 + lane;
+            bool head = false;
+            int bc = 0, r = 0, rs = p0;
+            for (int i = 1; i < b1; ++i) {
+                const int32_t s = __builtin_amdgcn_readlane(at, i);
+                if (s <= p) {
+                    r = i;
+                    rs = s;
                 }
-                s = e;
             }
+            if (p < p1) {
+                const uint32_t e = entry(p), c = e >> 1;
+                bad = bad || c >= (uint64_t)src.n || (p > rs && (entry(p - 1) >> 1) >= c);
+                bc = (int)(c / B2);
+                head = !(e & 1);
+                nz += head;
+                const uint32_t first = 2 * (uint32_t)(bc * B2), past = first + 2 * B2;
+                // Nonzeros of the block before it: in its row, then in those above.
+                for (int q = p - 1; head && q >= rs && q > p - B2; --q) {
+                    const uint32_t f = entry(q);
+                    if (f < first) break;
+                    head = f & 1;
+                }
+                int s = p0;
+                for (int i = 0; i < b1 - 1; ++i) {
+                    const int end = __builtin_amdgcn_readlane(at, i + 1);
+                    if (head && i < r) {
+                        int lo = s, hi = end;
+                        while (lo < hi) {
+                            const int mid = (lo + hi) >> 1;
+                            if (entry(mid) < first) lo = mid + 1;
+                            else hi = mid;
+                        }
+                        for (; head && lo < end; ++lo) {
+                            const uint32_t f = entry(lo);
+                            if (f >= past) break;
+                            head = f & 1;
+                        }
+                    }
+                    s = end;
+                }
+            }
+            const uint64_t m = __ballot(head);
+            const int k =
+                nb + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+            if (head && k < BR_BLOCKS) h[k] = bc;
+            nb += __popcll(m);
         }
-        const uint64_t m = __ballot(head);
-        const int k = nb + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-        if (head && k < BR_BLOCKS) h[k] = bc;
-        nb += __popcll(m);
+    };
+    auto load = [&](int p) {
+        const int32_t c = col[p] - o;
+        bad = bad || c < 0;                               // would look like another one once doubled
+        return (uint32_t)c << 1 | (uint32_t)(val[p] == T(0));
+    };
+    if (p1 - p0 <= stage) {
+        for (int q = p0 + lane; q < p1; q += 256) {
+            uint32_t e[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) e[j] = load(min(q + 64 * j, p1 - 1));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (q + 64 * j < p1) staged[q + 64 * j - p0] = e[j];
+        }
+        br_wave_sync();
+        find([&](int p) { return staged[p - p0]; });
+    } else {
+        find(load);
     }
     if (__ballot(bad) != 0 || nb > BR_BLOCKS) {
         if (lane == 0) flags[0] = 1;
@@ -815,6 +864,7 @@ __global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse s
     for (int i = lane; i < nb; i += 64) {
         const int x = h[i];
         int rank = 0;
+#pragma unroll 4
         for (int j = 0; j < nb; ++j) rank += h[j] < x;
         heads[p0 + rank] = x;
     }
@@ -1403,9 +1453,17 @@ int blocks_count(const jlust_sparse *src, int b1, int b2, const BlocksLayout &bl
 {
     JLUST_HIP_TRY(hipMemsetAsync(w.flags, 0, 256, st));
     const dim3 grid((unsigned)(bl.mb / BR_WAVES + 1)), block(64 * BR_WAVES);
-#define JLUST_HEADS(B2)                                                                                          \
-    hipLaunchKernelGGL((bsr_heads_kernel<T, B2>), grid, block, 0, st, *src, bl.mb, b1, w.heads, w.count, w.full, \
-                       w.flags)
+    hipLaunchKernelGGL(bsr_long_kernel, dim3(cv_grid(bl.mb)), dim3(256), 0, st, *src, bl.mb, b1, w.flags);
+    if (int e = check_launch("bsr_long_kernel")) return e;
+    // LDS for block-rows of up to twice the mean, in steps of 64 entries: the
+    // searches read it instead of L1 (4 x 4 f64 mesh, 24M entries: 311 -> 187
+    // us); the others search in memory.
+    const int64_t mean = src->nnz / bl.mb + 1;
+    const int stage = (int)std::min((2 * mean + 63) / 64 * 64, (int64_t)BR_STAGE);
+    const size_t lds = 4 * BR_WAVES * (size_t)(stage + BR_BLOCKS);
+#define JLUST_HEADS(B2)                                                                                           \
+    hipLaunchKernelGGL((bsr_heads_kernel<T, B2>), grid, block, lds, st, *src, bl.mb, b1, stage, w.heads, w.count, \
+                       w.full, w.flags)
     JLUST_BY_B2(b2, JLUST_HEADS)
 #undef JLUST_HEADS
     if (int e = check_launch("bsr_heads_kernel")) return e;
