@@ -979,7 +979,7 @@ int jlust_hip_convert_direct(const jlust_sparse *src, const jlust_sparse *dst,
  * increase.  workspace: the device bytes of ws (256-byte aligned); 0: not a
  * conversion of this kind.  count writes browptr (Int32[m/b1 + 1], origin of
  * src) and *nnzb, the stored blocks; -1: columns that do not increase,
- * pointers that are not canonical or block-rows past 8192 entries or 1024
+ * pointers that are not canonical or block-rows past 2048 entries or 1024
  * blocks: use the two steps.  It synchronises `stream`.  fill writes dst's
  * block columns and values (nouter = *nnzb, pos2 the browptr of count, the
  * same src and ws), stream-ordered.  Results as the two steps', bit for bit. */

@@ -723,7 +723,10 @@ __global__ __launch_bounds__(256) void sort_ptr_kernel(const uint32_t *__restric
 // fill them up).  Mesh of 59,200 nodes, 4 x 4 f64, 24M entries: 187 and 168 us, a
 // whole conversion 419 (2,038 by the general path); 3 x 3 f32, 24,000 nodes: 132
 // (762); 400k uniform rows of 8 to 8 x 8 blocks, mostly zeros: 623 (937).
-constexpr int BR_WAVES = 4, BR_BLOCKS = 1024, BR_ENTRIES = 8192, BR_STAGE = 2048, BR_DIM = 8;
+// Past 2,048 entries a wave is the whole kernel's tail, and they are found before
+// the others are read: 400k power-law rows of 16 into 4 x 4 blocks, which the
+// general path takes, 1,263 us (1,195 there; 1,651 with 8,192 allowed).
+constexpr int BR_WAVES = 4, BR_BLOCKS = 1024, BR_ENTRIES = 2048, BR_STAGE = 2048, BR_DIM = 8;
 
 // Orders a wave's LDS accesses (its lanes exchange values through LDS).
 __device__ __forceinline__ void br_wave_sync()

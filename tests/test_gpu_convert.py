@@ -362,7 +362,7 @@ def test_blocks_equal_two_steps(J, b1, b2, rm, dtype, origin, monkeypatch):
     of a block), NaN, empty block-rows, block-rows of 0, 1, 63 to 65 entries and
     more, the last block-row of a workgroup's four, and what it leaves to the
     two steps: unordered and repeated columns, pointers that do not cover the
-    entries, block-rows past 8192 entries or 1024 blocks."""
+    entries, block-rows past 2048 entries or 1024 blocks."""
     import torch
     from jlust_amd import convert as CV
     rng = np.random.default_rng(23)
@@ -411,17 +411,18 @@ def test_blocks_equal_two_steps(J, b1, b2, rm, dtype, origin, monkeypatch):
         return out
 
     for mb, nb, k in ((1, 1, 1), (3, 9, 4), (4, 40, 27), (5, 300, 70), (41, 60, 16)):
-        check(mb, nb, dense(mb, nb, k))
-        check(mb, nb, dense(mb, nb, k), zeros=0.3)
+        full = min(k, 2048 // (b1 * b2))
+        check(mb, nb, dense(mb, nb, full))
+        check(mb, nb, dense(mb, nb, full), zeros=0.3)
         check(mb, nb, [pick(nb * b2, int(rng.integers(0, 2 * k))) for _ in range(mb * b1 - 1)] + [[nb * b2 - 1]],
               zeros=0.2)
     for n in (63, 64, 65, 129):                             # entries of a block-row, all in its last row
         check(3, 200, [[]] * (2 * b1 - 1) + [pick(200 * b2, n)] + [[]] * b1)
     check(4, 20, dense(4, 20, 7), zeros=1.0)
     wide = 1024
-    check(2, 1030, dense(1, 1030, wide if wide * b1 * b2 <= 8192 else 8192 // (b1 * b2)) + [[1]] * b1)
+    check(2, 1030, dense(1, 1030, min(wide, 2048 // (b1 * b2))) + [[1]] * b1)
     check(2, 1030, dense(1, 1030, 1025) + [[1]] * b1, path=False)
-    check(1, 9000, [pick(9000 * b2, 8193)] + [[]] * (b1 - 1), path=False)
+    check(1, 9000, [pick(9000 * b2, 2049)] + [[]] * (b1 - 1), path=False)
     r = dense(2, 20, 9)
     r[0] = np.r_[3, 1] if b2 * 20 > 3 else r[0]
     check(2, 20, r, path=False)
