@@ -814,19 +814,19 @@ int jlust_hip_bsr_spmm_small_f32_i32(int64_t mb, int64_t nb, int64_t b1, int64_t
  * contract, ext/CUDAExt/ops/spmm.jl:8-70: analysis and workspace once,
  * execute many times, update_values! for new values of the same pattern).
  * 16 x 16 blocks keep the MFMA kernels (fp32, with 16-byte aligned values
- * for BSRRight, or fp64) and read the caller's buffers in place, and so do
- * square blocks of 2 to 8 rows whose longest block-row holds at most 64 blocks
- * or 4 times the mean (k >= 2; the plan owns a copy of B).  Any other
- * b1 x b2 shape is expanded to CSR once (jlust_hip_bsr_expand_csr_i32's
- * layout; the plan owns it) and runs through a CSR SpMM plan over it for k
- * columns.  create synchronises `stream` (browptr's ends are read back and
- * the CSR plan analyses its rows); update_values re-expands only the values,
- * stream-ordered, on the expansion path, and is a pointer swap on the other
- * two.  execute: B (nb*b2) x k (ldb), C (mb*b1) x k (ldc), column-major;
+ * for BSRRight, or fp64) and read the caller's buffers in place.  Square
+ * blocks of 2 to 8 rows whose longest block-row holds at most 64 blocks or 4
+ * times the mean run as stored (k >= 2; the plan owns a copy of the values and
+ * one of B).  Any other b1 x b2 shape is expanded to CSR once
+ * (jlust_hip_bsr_expand_csr_i32's layout; the plan owns it) and runs through a
+ * CSR SpMM plan over it for k columns.  create synchronises `stream` (browptr
+ * is read back and the CSR plan analyses its rows); update_values re-reads only
+ * the values, stream-ordered, and is a pointer swap on the MFMA path.
+ * execute: B (nb*b2) x k (ldb), C (mb*b1) x k (ldc), column-major;
  * C = alpha*A*B + beta*C (beta == 0: C write-only).  info: path 0 = MFMA,
  * 1 = CSR expansion, 2 = small square blocks as stored.  The plan keeps
- * browptr, bcolind (and, on paths 0 and 2, the values) by pointer: the caller
- * keeps them alive.
+ * browptr, bcolind (and, on path 0, the values) by pointer: the caller keeps
+ * them alive.
  */
 int jlust_hip_bsr_spmm_plan_create(int64_t mb, int64_t nb, int64_t b1,
                                    int64_t b2, int64_t nnzb, int32_t origin,

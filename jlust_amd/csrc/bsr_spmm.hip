@@ -2645,11 +2645,13 @@ extern "C" int jlust_hip_bsr_expand_csr_i32(int64_t mb, int64_t b1, int64_t b2, 
 // A prepared BSR SpMM (the analyse-once handle of the C ABI; the cuSPARSE SpMM
 // handle contract, ext/CUDAExt/ops/spmm.jl:8-70, for BSR).  16 x 16 blocks,
 // Float32 or Float64, keep the MFMA kernels and the caller's buffers
-// (update_values swaps the value pointer), and so do square blocks of 2 to 8
-// rows whose block-rows are of even length (bsr_small.hip; the plan owns the
-// copy of B).  Any other block shape is expanded to CSR once (the plan owns
-// the expansion) and runs through a CSR SpMM plan over it; update_values
-// re-expands the values only, on the stream.
+// (update_values swaps the value pointer).  Square blocks of 2 to 8 rows whose
+// block-rows are of even length run as stored (bsr_small.hip); any other block
+// shape is expanded to CSR once and runs through a CSR SpMM plan over it.
+// Which of the two a shape takes depends on its pattern, so both keep the
+// values in memory of the plan's own: a caller may reuse or free its buffer
+// after create and after update_values, which copies or re-expands the values
+// on the stream (199 MB of 4 x 4 f64 blocks: 75 us).
 static size_t bsr_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 struct jlust_bsr_plan {
@@ -2660,10 +2662,11 @@ struct jlust_bsr_plan {
     const int32_t *bcolind = nullptr;
     const void *val = nullptr;
     bool mfma = false, small = false;
-    void *mem = nullptr;                // expansion: rowptr | colind | values; or B's copy (small)
+    void *mem = nullptr;                // expansion: rowptr | colind | values; small: values | B's copy
     int32_t *rowptr = nullptr;
     int32_t *colind = nullptr;
-    void *cval = nullptr;
+    void *cval = nullptr;               // the plan's own values (not on the MFMA path)
+    void *Bt = nullptr;                 // small: B's copy
     jlust_spmm_plan_t csr = nullptr;
 };
 
@@ -2711,7 +2714,17 @@ static int bsr_spmm_plan_create_body(int64_t mb, int64_t nb, int64_t b1, int64_t
     if (!p->mfma && bsr_small_shape(nb, b1, b2, k, tsz))
         if (int st = bsr_small_pattern(mb, nnzb, origin, browptr, (hipStream_t)stream, &p->small)) return st;
     if (p->small) {
-        JLUST_HIP_TRY(hipMalloc(&p->mem, bsr_small_copy_bytes(nb, b1, k, tsz)));
+        const size_t sz_v = bsr_align_up(tsz * (size_t)total, 256);
+        JLUST_HIP_TRY(hipMalloc(&p->mem, sz_v + bsr_small_copy_bytes(nb, b1, k, tsz)));
+        p->cval = p->mem;
+        p->Bt = (char *)p->mem + sz_v;
+        hipStream_t s = (hipStream_t)stream;
+        hipError_t e = hipMemcpyAsync(p->cval, val, tsz * (size_t)total, hipMemcpyDeviceToDevice, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);     // the plan may then run on any stream
+        if (e != hipSuccess) {
+            (void)hipFree(p->mem);
+            return hip_fail(e, "bsr_spmm_plan_create");
+        }
     } else if (!p->mfma) {
         const size_t nz = (size_t)(total > 0 ? total : 1);
         const size_t sz_rp = bsr_align_up(sizeof(int32_t) * (size_t)(mb * b1 + 1), 256);
@@ -2757,12 +2770,18 @@ extern "C" int jlust_hip_bsr_spmm_plan_update_values(jlust_bsr_plan_t plan, cons
     if (plan->mfma && plan->value_type == 1 && plan->row_major && (uintptr_t)val % 16 != 0)
         return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_spmm_plan_update_values: block values must be 16-byte aligned");
     plan->val = val;
-    if (plan->mfma || plan->small) return JLUST_STATUS_SUCCESS;     // the kernels read the values in place
+    if (plan->mfma) return JLUST_STATUS_SUCCESS;     // the kernels read the values in place
     int dev = 0;
     if (int st = require_device(&dev)) return st;
     if (dev != plan->device)
         return fail(JLUST_STATUS_INVALID_ARGUMENT,
                     "bsr_spmm_plan_update_values: plan belongs to device %d, current device is %d", plan->device, dev);
+    if (plan->small) {
+        const size_t tsz = plan->value_type == 0 ? sizeof(double) : sizeof(float);
+        JLUST_HIP_TRY(hipMemcpyAsync(plan->cval, val, tsz * (size_t)total, hipMemcpyDeviceToDevice,
+                                     (hipStream_t)stream));
+        return JLUST_STATUS_SUCCESS;
+    }
     return bsr_expand_entries(plan->mb, plan->b1, plan->b2, plan->nnzb, plan->origin, plan->browptr, plan->bcolind,
                               val, plan->value_type, plan->row_major, nullptr, plan->cval, (hipStream_t)stream);
 }
@@ -2791,8 +2810,8 @@ static int bsr_small_execute(jlust_bsr_plan_t p, T alpha, const T *B, int64_t ld
     if (dev != p->device)
         return fail(JLUST_STATUS_INVALID_ARGUMENT,
                     "bsr_spmm_plan_execute: plan belongs to device %d, current device is %d", p->device, dev);
-    return bsr_small_spmm<T>(p->mb, p->nb, p->b1, p->origin, p->browptr, p->bcolind, (const T *)p->val, p->row_major,
-                             p->k, alpha, B, ldb, beta, C, ldc, (T *)p->mem, (hipStream_t)stream);
+    return bsr_small_spmm<T>(p->mb, p->nb, p->b1, p->origin, p->browptr, p->bcolind, (const T *)p->cval, p->row_major,
+                             p->k, alpha, B, ldb, beta, C, ldc, (T *)p->Bt, (hipStream_t)stream);
 }
 
 template <typename T>

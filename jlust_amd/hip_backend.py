@@ -1496,9 +1496,10 @@ class HIPBSRSpMMHandle(AbstractKernelHandle):
     blocks of 2 to 8 rows in block-rows of even length a kernel of their own;
     any other block shape is expanded to CSR once and runs through a CSR SpMM
     plan over the expansion.  A's values are read as they are at the
-    call: on the expansion path, values written in place through torch since
-    the plan last read them (the value tensor's version counter moved) are
-    expanded again, in stream order, before the product.  B with another
+    call: where the plan has values of its own (all but the MFMA kernels),
+    values written in place through torch since it last read them (the value
+    tensor's version counter moved) are read again, in stream order, before the
+    product.  B with another
     number of columns than the plan's rebuilds the plan."""
 
     def __init__(self, u_A: USTensor, n_cols=None):

@@ -733,3 +733,46 @@ def test_bsr_spmv_runs_of_items(J, O, b, dtype, row_major):
             absref = O.csr_spmv_absref(rp, ci, v, x, alpha, beta, yb, origin)
             assert_within(ys[0], ref, absref, dtype, f"{name}, beta={beta}")
             np.testing.assert_array_equal(ys[1], ys[0], err_msg=f"{name}, plan")
+
+
+@pytest.mark.parametrize("b,long_row,path", [(4, 0, 2), (3, 0, 2), (4, 200, 1), (5, 200, 1)])
+@pytest.mark.parametrize("vt,dtype", [(0, np.float64), (1, np.float32)])
+def test_bsr_plan_owns_its_values(J, O, b, long_row, path, vt, dtype):
+    """A C caller's value buffer is its own again after create and after
+    update_values, whichever of the two paths with values of the plan's own the
+    pattern takes: what the buffer holds later does not reach the product."""
+    import ctypes
+    import torch
+    from jlust_amd import _lib
+    L = _lib.lib()
+    rng = np.random.default_rng(b)
+    mb, nb, k = 40, 250, 6
+    counts = rng.integers(1, 6, mb)
+    if long_row:
+        counts[3] = long_row
+    bc = (np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in counts]) + 1).astype(np.int32)
+    bp = (np.r_[0, np.cumsum(counts)] + 1).astype(np.int32)
+    first, second = (rng.integers(-4, 5, bc.size * b * b).astype(dtype) for _ in range(2))
+    B = np.asfortranarray(rng.integers(-3, 4, (nb * b, k)).astype(dtype))
+    want = [O.bsr_spmm(bp, bc, v, b, B, 1.0, 0.0, np.zeros((mb * b, k), dtype, order="F"), b2=b)
+            for v in (first, second)]
+    dbp, dbc, buf, Bd = dev(bp), dev(bc), dev(first), dev(B)
+    C = J.dense_matrix(mb * b, k, dtype=buf.dtype)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    plan, got_path = ctypes.c_void_p(), ctypes.c_int32(-1)
+    ok = lambda st: _lib.check(st, "bsr plan")      # noqa: E731
+    ok(L.jlust_hip_bsr_spmm_plan_create(mb, nb, b, b, bc.size, 1, vt, 1, dbp.data_ptr(), dbc.data_ptr(),
+                                        buf.data_ptr(), k, stream, ctypes.byref(plan)))
+    try:
+        ok(L.jlust_hip_bsr_spmm_plan_info(plan, ctypes.byref(got_path)))
+        assert got_path.value == path
+        run = L.jlust_hip_bsr_spmm_plan_execute_f32 if vt else L.jlust_hip_bsr_spmm_plan_execute_f64
+        for i in range(2):
+            if i:
+                buf.copy_(dev(second))
+                ok(L.jlust_hip_bsr_spmm_plan_update_values(plan, buf.data_ptr(), stream))
+            buf.fill_(float("nan"))
+            ok(run(plan, 1.0, Bd.data_ptr(), nb * b, 0.0, C.data_ptr(), mb * b, stream))
+            np.testing.assert_array_equal(host(C), want[i])
+    finally:
+        L.jlust_hip_bsr_spmm_plan_destroy(plan)
