@@ -793,8 +793,9 @@ int jlust_hip_bsr_expand_csr_i32(int64_t mb, int64_t b1, int64_t b2,
  * C = alpha*A*B + beta*C for square blocks of 2 to 8 rows on the blocks as
  * stored: *taken = 1 if the product ran, 0 if it is left to
  * jlust_hip_bsr_expand_csr_i32 + the CSR entry points (another shape, k < 2,
- * a copy of B past 4 GiB, block-rows far longer than the mean, or a browptr
- * that is not canonical).  Arguments as jlust_hip_bsr_spmm_*.  Reads the
+ * 24 columns of B past 4 GiB, no memory for B's copy, block-rows far longer
+ * than the mean, or a browptr that is not canonical).  B's copy is in the
+ * stream's scratch buffer, up to 1 GB of it or 16 columns.  Arguments as jlust_hip_bsr_spmm_*.  Reads the
  * longest block-row back, so it synchronises `stream` (not capturable; a plan
  * is).
  */

@@ -6,7 +6,8 @@
 // rows), without the expansion: one column index per block instead of one per
 // entry, and every gathered row of B used for all of the block's rows.
 //
-// B is re-laid row-major (spmm_row_major_copy).  A wave's 64 lanes form NG =
+// B is re-laid row-major (spmm_row_major_copy), in passes of columns where the
+// copy would be large (small_kchunk).  A wave's 64 lanes form NG =
 // 64 / L groups; a group takes a block-row, each lane CPL columns of C for its
 // B block-row rows in registers.  A group's next SB blocks are loaded by its
 // own lanes, a stage ahead, and kept in LDS column by column, from where every
@@ -262,16 +263,31 @@ int launch_cpl(int cpl, const SmallShape &sh, const int32_t *browptr, const int3
 
 }  // namespace
 
+// Columns per pass: as few passes of about equal width as keep B's copy within
+// 512 MB, or 1 GB for blocks past 4 x 4, whose values are the larger part of
+// what a further pass reads again; 16 columns at least.  us per product, copy
+// within 256 MB / 512 MB / 1 GB: 4 x 4 f64 on a band, 2M rows, k = 48: 1311 /
+// 1250 / 1433; 2 x 2 f64 mesh of 1M nodes, k = 48: 2139 / 2175 / 2762; 3 x 3
+// f32 mesh of 1M nodes, k = 128: 5227 / 4344 / 4380 (one pass: 4932); 4 x 4 f64
+// mesh of 422k nodes, k = 24: 1224 / 961 / 954; 8 x 8: 3944 / 3940 / 2969.
+static int64_t small_kchunk(int64_t nb, int64_t b, int64_t k, size_t tsz)
+{
+    const size_t budget = (size_t)(b <= 4 ? 512 : 1024) << 20;
+    const int64_t passes = (int64_t)(((size_t)k * (size_t)(nb * b) * tsz + budget - 1) / budget);
+    if (passes <= 1) return k;
+    return std::min(k, std::max<int64_t>(16, ((k + passes - 1) / passes + 7) / 8 * 8));
+}
+
 bool bsr_small_shape(int64_t nb, int64_t b1, int64_t b2, int64_t k, size_t tsz)
 {
     if (b1 != b2 || b1 < 2 || b1 > 8 || k < 2) return false;
     // Offsets into B's copy are 32-bit.
-    return (uint64_t)(nb * b2 + 1) * (uint64_t)(k + 8) * tsz < 0xff000000ull;
+    return (uint64_t)(nb * b2 + 1) * (uint64_t)(small_kchunk(nb, b2, k, tsz) + 8) * tsz < 0xff000000ull;
 }
 
 size_t bsr_small_copy_bytes(int64_t nb, int64_t b, int64_t k, size_t tsz)
 {
-    return tsz * (size_t)(nb * b + 1) * (size_t)((k + 7) / 8 * 8);
+    return tsz * (size_t)(nb * b + 1) * (size_t)((small_kchunk(nb, b, k, tsz) + 7) / 8 * 8);
 }
 
 int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *browptr, hipStream_t s, bool *even)
@@ -294,12 +310,12 @@ int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *b
     return JLUST_STATUS_SUCCESS;
 }
 
+// One pass: its k columns.
 template <typename T>
-int bsr_small_spmm(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int32_t *browptr, const int32_t *bcolind,
-                   const T *val, int row_major, int64_t k, T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
-                   T *Bt, hipStream_t s)
+static int small_pass(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int32_t *browptr,
+                      const int32_t *bcolind, const T *val, int row_major, int64_t k, T alpha, const T *B, int64_t ldb,
+                      T beta, T *C, int64_t ldc, T *Bt, hipStream_t s)
 {
-    if (mb == 0 || k == 0) return JLUST_STATUS_SUCCESS;
     const int cpl = small_cpl<T>(k);
     SmallShape sh{};
     sh.mb = mb;
@@ -321,6 +337,20 @@ int bsr_small_spmm(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int3
     }
 #undef JLUST_B
     return fail(JLUST_STATUS_INVALID_ARGUMENT, "bsr_small_spmm: block size %lld", (long long)b);
+}
+
+template <typename T>
+int bsr_small_spmm(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int32_t *browptr, const int32_t *bcolind,
+                   const T *val, int row_major, int64_t k, T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                   T *Bt, hipStream_t s)
+{
+    if (mb == 0) return JLUST_STATUS_SUCCESS;
+    const int64_t kc = small_kchunk(nb, b, k, sizeof(T));
+    for (int64_t c0 = 0; c0 < k; c0 += kc)
+        if (int st = small_pass<T>(mb, nb, b, origin, browptr, bcolind, val, row_major, std::min(kc, k - c0), alpha,
+                                   B + c0 * ldb, ldb, beta, C + c0 * ldc, ldc, Bt, s))
+            return st;
+    return JLUST_STATUS_SUCCESS;
 }
 
 template int bsr_small_spmm<double>(int64_t, int64_t, int64_t, int32_t, const int32_t *, const int32_t *,

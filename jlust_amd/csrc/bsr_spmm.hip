@@ -2715,7 +2715,14 @@ static int bsr_spmm_plan_create_body(int64_t mb, int64_t nb, int64_t b1, int64_t
         if (int st = bsr_small_pattern(mb, nnzb, origin, browptr, (hipStream_t)stream, &p->small)) return st;
     if (p->small) {
         const size_t sz_v = bsr_align_up(tsz * (size_t)total, 256);
-        JLUST_HIP_TRY(hipMalloc(&p->mem, sz_v + bsr_small_copy_bytes(nb, b1, k, tsz)));
+        if (hipMalloc(&p->mem, sz_v + bsr_small_copy_bytes(nb, b1, k, tsz)) != hipSuccess) {
+            (void)hipGetLastError();         // the expansion's copy of B may be smaller
+            p->mem = nullptr;
+            p->small = false;
+        }
+    }
+    if (p->small) {
+        const size_t sz_v = bsr_align_up(tsz * (size_t)total, 256);
         p->cval = p->mem;
         p->Bt = (char *)p->mem + sz_v;
         hipStream_t s = (hipStream_t)stream;
@@ -2839,7 +2846,11 @@ static int bsr_small_call(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_
     if (!even) return JLUST_STATUS_SUCCESS;
     if (int st = bsr_small_dense_args(mb * b1, nb * b2, k, B, ldb, C, ldc)) return st;
     void *Bt = nullptr;
-    if (int st = scratch(stream, bsr_small_copy_bytes(nb, b1, k, sizeof(T)), &Bt)) return st;
+    if (scratch(stream, bsr_small_copy_bytes(nb, b1, k, sizeof(T)), &Bt) != JLUST_STATUS_SUCCESS) {
+        (void)hipGetLastError();             // the expansion's copy of B may be smaller
+        clear_error();
+        return JLUST_STATUS_SUCCESS;
+    }
     *taken = 1;
     return bsr_small_spmm<T>(mb, nb, b1, origin, browptr, bcolind, val, row_major_blocks ? 1 : 0, k, alpha, B, ldb,
                              beta, C, ldc, (T *)Bt, s);

@@ -127,7 +127,7 @@ int spmm_row_major_copy(int value_type, int64_t n, int64_t k, const void *B, int
                         hipStream_t s);
 
 // BSR SpMM on small square blocks (bsr_small.hip): whether a shape is one of
-// its; the bytes of B's copy (Bt); whether browptr runs from the origin to
+// its; the bytes of B's copy of one pass (Bt); whether browptr runs from the origin to
 // nnzb + origin without decreasing and has no block-row much longer than the
 // others (*even; synchronises s); the product.
 bool bsr_small_shape(int64_t nb, int64_t b1, int64_t b2, int64_t k, size_t tsz);

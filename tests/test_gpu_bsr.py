@@ -776,3 +776,37 @@ def test_bsr_plan_owns_its_values(J, O, b, long_row, path, vt, dtype):
             np.testing.assert_array_equal(host(C), want[i])
     finally:
         L.jlust_hip_bsr_spmm_plan_destroy(plan)
+
+
+@pytest.mark.parametrize("call", ["plain", "plan"])
+@pytest.mark.parametrize("k", [17, 40])
+def test_bsr_small_blocks_column_passes(J, k, call):
+    """A B past 512 MB goes through its row-major copy 16 columns at a time:
+    a last pass of one column, and of eight; exact on integers."""
+    import torch
+    b, nb, mb = 2, 2_050_000, 301
+    rng = np.random.default_rng(k)
+    counts = rng.integers(0, 9, mb)
+    bc = np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in counts])
+    bc[-1] = nb - 1
+    bp = np.r_[0, np.cumsum(counts)]
+    gen = torch.Generator("cuda").manual_seed(k)
+    vals = torch.randint(-4, 5, (bc.size, b, b), generator=gen, device="cuda").double()
+    B = torch.randint(-3, 4, (k, nb * b), generator=gen, device="cuda").double().t()
+    C = torch.randint(-3, 4, (k, mb * b), generator=gen, device="cuda").double().t()
+    A = J.bsr_tensor(dev((bp + 1).astype(np.int32)), dev((bc + 1).astype(np.int32)), vals.reshape(-1),
+                     (mb * b, nb * b), (b, b), True)
+    X = B[(torch.from_numpy(bc).cuda()[:, None] * b + torch.arange(b, device="cuda")).reshape(-1)].view(-1, b, k)
+    part = sum(vals[:, :, j, None] * X[:, j, None, :] for j in range(b))
+    rows = torch.from_numpy(np.repeat(np.arange(mb), counts)).cuda()
+    want = -1.0 * C + 2.0 * torch.zeros(mb, b, k, dtype=torch.float64, device="cuda").index_add_(0, rows, part).view(
+        mb * b, k)
+    free = torch.cuda.mem_get_info()[0]
+    if call == "plain":
+        J.execute(J.SpMMOp, A, B, C, alpha=2.0, beta=-1.0)
+    else:
+        h = J.prepare(J.HIPBackend(), J.SpMMOp, A, n_cols=k)
+        assert h.info()["path"] == "blocks"
+        assert free - torch.cuda.mem_get_info()[0] < 600 << 20      # a copy of 16 columns: 525 MB
+        J.execute(h, B, C, alpha=2.0, beta=-1.0)
+    assert torch.equal(C, want)
