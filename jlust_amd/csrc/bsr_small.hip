@@ -54,13 +54,19 @@ struct SmallShape {
     int sb;                              // blocks per stage
     int gs;                              // values of a group's stage in LDS
     int wave_vals;                       // values of a wave's stage or result tile in LDS
+    int sums_at;                         // where a wave's further sums start
     int wave_stride;                     // values from one wave's LDS to the next
     int32_t origin;
     int row_major;
     unsigned run;                        // consecutive workgroups per XCD
 };
 
-template <typename T, int B, int CPL>
+// LV sums per row and column: a block's product goes into the first, in a
+// register, which goes into the next, in LDS, after four blocks (LV = 2) or
+// three, that one into a third after three of those (small_levels).  In
+// registers they cost waves (8 x 8 f64, k = 2: 190 registers, 115 us against
+// 66).
+template <typename T, int B, int CPL, int LV>
 __global__ __launch_bounds__(BS_BLOCK) void bsr_small_spmm_kernel(
     SmallShape sh, const int32_t *__restrict__ browptr, const int32_t *__restrict__ bcolind,
     const T *__restrict__ val, const T *__restrict__ Bt0, T alpha, T beta, int beta_zero, T *__restrict__ C,
@@ -71,17 +77,19 @@ __global__ __launch_bounds__(BS_BLOCK) void bsr_small_spmm_kernel(
     constexpr int AW = B <= 2 ? 2 : V16 < 4 ? 2 : 4;       // values per read of A
     constexpr int BP = (B + AW - 1) / AW * AW;             // a block row in LDS
     constexpr int BB = B * B;
+    constexpr int HALF = B < 5 || LV == 1 ? B : (B + 1) / 2;   // a block row's product in two halves
     extern __shared__ __attribute__((aligned(16))) char s_mem[];
 
     const unsigned x = blockIdx.x % NUM_XCD, i0 = blockIdx.x / NUM_XCD;
     const int64_t wg = (int64_t)(i0 / sh.run * NUM_XCD + x) * sh.run + i0 % sh.run;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int L = sh.L, NG = 64 / L;
     const int64_t R0 = (wg * BS_WAVES + wave) * NG;
     if (R0 >= sh.mb) return;
     const int grp = lane / L, sub = lane - grp * L;
     T *const s_a = reinterpret_cast<T *>(s_mem) + wave * sh.wave_stride;
     uint32_t *const s_off = reinterpret_cast<uint32_t *>(s_a + sh.wave_vals);
+    T *const s_sum = s_a + sh.sums_at + lane;              // sum h, row r, column c: [((h - 1) * B + r) * CPL + c][lane]
     const int c0 = (int)blockIdx.y * sh.cols;
     const int kk = min(sh.cols, sh.k - c0);
     const uint32_t col = (uint32_t)(c0 + min(sub * CPL, (int)sh.ldt - c0 - CPL)) * (uint32_t)sizeof(T);
@@ -127,6 +135,24 @@ __global__ __launch_bounds__(BS_BLOCK) void bsr_small_spmm_kernel(
     for (int r = 0; r < B; ++r)
 #pragma unroll
         for (int c = 0; c < CPL; ++c) acc[r][c] = T(0);
+#pragma unroll
+    for (int i = 0; i < (LV - 1) * B * CPL; ++i) s_sum[i * 64] = T(0);
+    auto carry = [&](int h) {                              // sum h into the next
+#pragma unroll
+        for (int r = 0; r < B; ++r)
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) {
+                T *const up = s_sum + ((h * B + r) * CPL + c) * 64;
+                if (h == 0) {
+                    *up += acc[r][c];
+                    acc[r][c] = T(0);
+                } else {
+                    *up += *(up - B * CPL * 64);
+                    *(up - B * CPL * 64) = T(0);
+                }
+            }
+    };
+    int filled0 = 0, filled1 = 0;
 
     load_stage(0);
     for (int s0 = 0; __any(s0 < n); s0 += sh.sb) {
@@ -136,37 +162,66 @@ __global__ __launch_bounds__(BS_BLOCK) void bsr_small_spmm_kernel(
         load_stage(s0 + sh.sb);
         const int top = min(sh.sb, n - s0);
         for (int u = 0; __any(u < top); ++u) {
-            if (u >= top) continue;
-            const char *const bp = reinterpret_cast<const char *>(Bt0);
-            const uint32_t off = s_off[grp * sh.sb + u] + col;
-            Pack<T, W> b[B][CPL / W];
+            if (u < top) {
+                const char *const bp = reinterpret_cast<const char *>(Bt0);
+                const uint32_t off = s_off[grp * sh.sb + u] + col;
+                Pack<T, W> b[B][CPL / W];
 #pragma unroll
-            for (int jj = 0; jj < B; ++jj)
+                for (int jj = 0; jj < B; ++jj)
 #pragma unroll
-                for (int v = 0; v < CPL / W; ++v)
-                    b[jj][v] = *reinterpret_cast<const Pack<T, W> *>(
-                        bp + (off + (uint32_t)jj * row_bytes + (uint32_t)(v * W * sizeof(T))));
-            // A row of the block's own product first, then into the row's sum: a
-            // chain of one rounding per block (as few as the expanded rows'
-            // split sums).
+                    for (int v = 0; v < CPL / W; ++v)
+                        b[jj][v] = *reinterpret_cast<const Pack<T, W> *>(
+                            bp + (off + (uint32_t)jj * row_bytes + (uint32_t)(v * W * sizeof(T))));
+                // A row of the block's own product first, then into the row's sum.
 #pragma unroll
-            for (int r = 0; r < B; ++r) {
-                T a[BP];
+                for (int r = 0; r < B; ++r) {
+                    T a[BP];
 #pragma unroll
-                for (int v = 0; v < BP / AW; ++v) {
-                    const Pack<T, AW> p = *reinterpret_cast<const Pack<T, AW> *>(a_dst + (u * B + r) * BP + v * AW);
+                    for (int v = 0; v < BP / AW; ++v) {
+                        const Pack<T, AW> p = *reinterpret_cast<const Pack<T, AW> *>(a_dst + (u * B + r) * BP + v * AW);
 #pragma unroll
-                    for (int e = 0; e < AW; ++e) a[v * AW + e] = p.v[e];
+                        for (int e = 0; e < AW; ++e) a[v * AW + e] = p.v[e];
+                    }
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) {
+                        T t = a[0] * b[0][c / W].v[c % W];
+#pragma unroll
+                        for (int jj = 1; jj < HALF; ++jj) t += a[jj] * b[jj][c / W].v[c % W];
+                        if constexpr (HALF < B) {
+                            T t2 = a[HALF] * b[HALF][c / W].v[c % W];
+#pragma unroll
+                            for (int jj = HALF + 1; jj < B; ++jj) t2 += a[jj] * b[jj][c / W].v[c % W];
+                            t += t2;
+                        }
+                        acc[r][c] += t;
+                    }
                 }
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) {
-                    T t = a[0] * b[0][c / W].v[c % W];
-#pragma unroll
-                    for (int jj = 1; jj < B; ++jj) t += a[jj] * b[jj][c / W].v[c % W];
-                    acc[r][c] += t;
+            }
+            // All groups together: a sum of a finished row stays what it is, now
+            // or below.
+            if constexpr (LV > 1) {
+                if (++filled0 == (LV == 2 ? 4 : 3)) {
+                    filled0 = 0;
+                    carry(0);
+                    if constexpr (LV > 2) {
+                        if (++filled1 == 3) {
+                            filled1 = 0;
+                            carry(1);
+                        }
+                    }
                 }
             }
         }
+    }
+    if constexpr (LV > 1) {
+#pragma unroll
+        for (int r = 0; r < B; ++r)
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) {
+                T *const up = s_sum + (r * CPL + c) * 64;
+                acc[r][c] += *up;
+                if constexpr (LV > 2) acc[r][c] += up[B * CPL * 64];
+            }
     }
 
     // Column c of every lane: the wave's rows, one run per column of C.
@@ -221,7 +276,22 @@ int small_cpl(int64_t k)
     return c;
 }
 
-template <typename T, int B, int CPL>
+// Sums per row and column.  The expansion's kernels hold S = 64 / p sums of a
+// column's products for k <= 32 columns (p the power of two at k or above), one
+// beyond.  One chain of the blocks' products rounds as little as those below S =
+// b, two levels below 3b, three from there: counted over rows of 3 to 32 blocks,
+// 0.53-1.02 times the error of the S sums, where one chain made up to 1.34.
+// Measured, f32, 27 blocks a row: 2 x 2, k = 2, 1.01 (one chain 1.53); 3 x 3, k =
+// 12, 0.83 (1.14).
+inline int small_levels(int64_t b, int64_t k)
+{
+    int64_t p = 1;
+    while (p < k) p *= 2;
+    const int64_t S = p <= 32 ? 64 / p : 1;
+    return S >= 3 * b ? 3 : S >= b ? 2 : 1;
+}
+
+template <typename T, int B, int CPL, int LV>
 int launch(const SmallShape &base, const int32_t *browptr, const int32_t *bcolind, const T *val, const T *Bt, T alpha,
            T beta, T *C, int64_t ldc, hipStream_t s)
 {
@@ -237,13 +307,14 @@ int launch(const SmallShape &base, const int32_t *browptr, const int32_t *bcolin
     sh.gs = (sh.sb * B * BP + V16 - 1) / V16 * V16;
     if (sh.gs / V16 % 2 == 0) sh.gs += V16;
     sh.wave_vals = (max(NG * sh.gs, sh.L * (NG * B + 1)) + V16 - 1) / V16 * V16;
-    sh.wave_stride = (sh.wave_vals + NG * sh.sb * 4 / (int)sizeof(T) + V16) / V16 * V16;
+    sh.sums_at = (sh.wave_vals + NG * sh.sb * 4 / (int)sizeof(T) + V16) / V16 * V16;
+    sh.wave_stride = sh.sums_at + (LV - 1) * B * CPL * 64;
     const size_t per_wave = sizeof(T) * (size_t)sh.wave_stride;
     const int64_t wgs = (sh.mb + (int64_t)BS_WAVES * NG - 1) / (BS_WAVES * NG);
     sh.run = (unsigned)((wgs + 4 * NUM_XCD - 1) / (4 * NUM_XCD));
     const dim3 grid((unsigned)((wgs + (int64_t)sh.run * NUM_XCD - 1) / ((int64_t)sh.run * NUM_XCD) * sh.run * NUM_XCD),
                     (unsigned)ny);
-    hipLaunchKernelGGL((bsr_small_spmm_kernel<T, B, CPL>), grid, dim3(BS_BLOCK), per_wave * BS_WAVES, s, sh, browptr,
+    hipLaunchKernelGGL((bsr_small_spmm_kernel<T, B, CPL, LV>), grid, dim3(BS_BLOCK), per_wave * BS_WAVES, s, sh, browptr,
                        bcolind, val, Bt, alpha, beta, beta == T(0), C, ldc);
     return check_launch("bsr_small_spmm_kernel");
 }
@@ -253,12 +324,26 @@ int launch_cpl(int cpl, const SmallShape &sh, const int32_t *browptr, const int3
                const T *Bt, T alpha, T beta, T *C, int64_t ldc, hipStream_t s)
 {
     constexpr int M = MAX_COLS<T>;
-#define JLUST_CPL(N) \
-    if (cpl == N) return launch<T, B, (N <= M ? N : M)>(sh, browptr, bcolind, val, Bt, alpha, beta, C, ldc, s);
-    JLUST_CPL(4)
-    JLUST_CPL(2)
-#undef JLUST_CPL
-    return launch<T, B, 1>(sh, browptr, bcolind, val, Bt, alpha, beta, C, ldc, s);
+    const int lv = small_levels(B, sh.k);
+    // Only what small_cpl and small_levels can ask for together.
+#define JLUST_LAUNCH(N, LV) \
+    return launch<T, B, (N <= M ? N : M), LV>(sh, browptr, bcolind, val, Bt, alpha, beta, C, ldc, s)
+    if (cpl == 4) {                                        // 13 columns or more
+        if constexpr (B <= 4) {
+            if (lv == 2) JLUST_LAUNCH(4, 2);
+        }
+        JLUST_LAUNCH(4, 1);
+    }
+    if (cpl == 2) {                                        // 7 or more
+        if constexpr (B == 2) {
+            if (lv == 3) JLUST_LAUNCH(2, 3);
+        }
+        if (lv == 2) JLUST_LAUNCH(2, 2);
+        JLUST_LAUNCH(2, 1);
+    }
+    if (lv == 3) JLUST_LAUNCH(1, 3);                       // 6 or fewer
+    JLUST_LAUNCH(1, 2);
+#undef JLUST_LAUNCH
 }
 
 }  // namespace

@@ -68,3 +68,17 @@ def sample_rows(rowptr, colind, val, rows, origin=1):
     idx = np.concatenate([np.arange(a, b) for a, b in zip(lo, hi)]) if rows.size else \
         np.zeros(0, np.int64)
     return (rp + origin).astype(np.int32), colind[idx], val[idx], idx
+
+
+def split_sums_f32(a, b, sums):
+    """sum_j a[..., j] * b[..., j] in float32 over `sums` (a power of two)
+    strided partial sums, fused multiply-adds in order, added as a tree: what
+    a group of that many lanes computes."""
+    n = a.shape[-1]
+    acc = [np.zeros(a.shape[:-1], np.float32) for _ in range(sums)]
+    for j in range(n):
+        p = a[..., j].astype(np.float64) * b[..., j].astype(np.float64)
+        acc[j % sums] = (acc[j % sums].astype(np.float64) + p).astype(np.float32)
+    while len(acc) > 1:
+        acc = [acc[i] + acc[i + 1] for i in range(0, len(acc), 2)]
+    return acc[0]
