@@ -240,9 +240,12 @@ __device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 // k = 20: 107 -> 34; 200k uniform rows of 16 (bound by the fabric), f64, k = 8:
 // 69 -> 63, k = 64: 291 -> 297.
 // 5 waves per SIMD at least, as many as the LDS of 5 blocks leaves (the f64 mesh
-// at k = 20: 71 us at 4).
+// at k = 20: 71 us at 4); 4 where the sums and the entries in flight take more
+// registers than that leaves (f64, 2 columns a lane, 12 of both: 9 to 24 spilled
+// at 5; mesh below, k = 8: 50 -> 46 us with twice the sums, band of 30 a row, k =
+// 16: 18.1 -> 15.9).
 template <typename T, int VEC, int U, int ACC, bool BIG>
-__global__ __launch_bounds__(SPMM_BLOCK, 5) void csr_spmm_rows_kernel(
+__global__ __launch_bounds__(SPMM_BLOCK, (ACC + U) * VEC * sizeof(T) > 160 ? 4 : 5) void csr_spmm_rows_kernel(
     SpmmJob<T> ja, SpmmJob<T> jb, SpmmShape sh, int32_t origin, const int32_t *__restrict__ colind,
     const T *__restrict__ val, const T *__restrict__ Bt0)
 {
@@ -295,11 +298,11 @@ __global__ __launch_bounds__(SPMM_BLOCK, 5) void csr_spmm_rows_kernel(
 
     const int ss = sh.slice_log2, S = 1 << ss;
 
-    // N steps of every group: entries p + s .. p + s + N - 1, those with s + u < n.
-    // ACC sums per column, entry u of a step into sum u mod ACC.
+    // N steps of every group: entries p + s .. p + s + N - 1, those with s + u < n,
+    // entry u into sum (FIRST + u) mod ACC of ACC sums per column.
     T acc[ACC][VEC];
-    auto steps = [&](auto N, int p, int s, int n) {
-        constexpr int NS = decltype(N)::value;
+    auto steps = [&](auto N, auto FIRST, int p, int s, int n) {
+        constexpr int NS = decltype(N)::value, F = decltype(FIRST)::value;
         uint32_t off[NS];
         T a[NS];
         V b[NS];
@@ -319,14 +322,30 @@ __global__ __launch_bounds__(SPMM_BLOCK, 5) void csr_spmm_rows_kernel(
 #pragma unroll
         for (int u = 0; u < NS; ++u)
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[u % ACC][e] += a[u] * b[u].v[e];
+            for (int e = 0; e < VEC; ++e) acc[(F + u) % ACC][e] += a[u] * b[u].v[e];
     };
+    using I0 = std::integral_constant<int, 0>;
+    using I2 = std::integral_constant<int, 2>;
+    using I4 = std::integral_constant<int, 4>;
     auto row_sum = [&](int p, int n) {
         int s = 0;
-        if (U == 8)
-            for (; __any(s + 4 < n); s += 8) steps(std::integral_constant<int, 8>(), p, s, n);
-        for (; __any(s + 2 < n); s += 4) steps(std::integral_constant<int, 4>(), p, s, n);
-        if (__any(s < n)) steps(std::integral_constant<int, 2>(), p, s, n);
+        if constexpr (ACC == 8) {
+            for (; __any(s + 6 < n); s += 8) {
+                steps(I4(), I0(), p, s, n);
+                steps(I4(), I4(), p, s + 4, n);
+            }
+            if (__any(s + 2 < n)) {
+                steps(I4(), I0(), p, s, n);
+                s += 4;
+                if (__any(s < n)) steps(I2(), I4(), p, s, n);
+                return;
+            }
+        } else {
+            if constexpr (U == 8)
+                for (; __any(s + 4 < n); s += 8) steps(std::integral_constant<int, 8>(), I0(), p, s, n);
+            for (; __any(s + 2 < n); s += 4) steps(I4(), I0(), p, s, n);
+        }
+        if (__any(s < n)) steps(I2(), I0(), p, s, n);
     };
 
     int a = whole ? bcast_i(lo, 0) : wave_min(empty ? INT_MAX : lo);
@@ -410,7 +429,8 @@ __global__ __launch_bounds__(SPMM_BLOCK, 5) void csr_spmm_rows_kernel(
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
                     T v = acc[0][e] + acc[1][e];
-                    if (ACC == 4) v += acc[ACC - 2][e] + acc[ACC - 1][e];
+                    if constexpr (ACC >= 4) v += acc[2][e] + acc[3][e];
+                    if constexpr (ACC == 8) v += (acc[4][e] + acc[5][e]) + (acc[6][e] + acc[7][e]);
                     dst[e] = v;
                 }
             }
@@ -609,19 +629,32 @@ int spmm_rows_launch(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, i
     // 8 entries in flight per group for long f64 rows (27-point mesh, k = 128:
     // 558 -> 523 us), else 4: short rows would load past their ends (1M
     // power-law rows of 5, f64, k = 64: 827 -> 752 us), and f32 gains nothing.
-    // Four sums per column up to 16 columns, else two: as many roundings in a
-    // chain as the kernels before had or fewer (27 entries, f32: 6.2e-8 relative
-    // error with four, 7.2e-8 with two, 9.4e-8 with one; four cost the f64 mesh
-    // at k = 20 8 % in registers).
+    // Eight sums per column up to 8 columns, four up to 16, else two: counted
+    // over rows of 32 entries and fewer, no more error than the 64 / p sums of
+    // a row split over a wave's lanes (p the power of two at the columns or
+    // above; four sums for 8 columns made 1.09 times that).
 #define JLUST_ROWS(U, ACC, BIG)                                                                               \
     hipLaunchKernelGGL((csr_spmm_rows_kernel<T, VEC, U, ACC, BIG>), grid, dim3(SPMM_BLOCK), lds, s, ja, jb, sh, \
                        origin, colind, val, Bt)
-    const bool deep = sizeof(T) == 8 && mean_a > 20, wide = kk > 16;
-    if ((uint64_t)(n + 1) * (uint64_t)ldt * sizeof(T) > 0xffffff00ull) JLUST_ROWS(4, 4, true);
-    else if (deep && wide) JLUST_ROWS(8, 2, false);
-    else if (deep) JLUST_ROWS(8, 4, false);
-    else if (wide) JLUST_ROWS(4, 2, false);
-    else JLUST_ROWS(4, 4, false);
+    // Only what spmm_chunk_kind's columns per lane leave to choose from.
+    constexpr bool SOME8 = VEC <= 2, SOME4 = VEC >= 2;
+    constexpr int DEEP = sizeof(T) == 8 ? 8 : 4;
+    const bool big = (uint64_t)(n + 1) * (uint64_t)ldt * sizeof(T) > 0xffffff00ull;
+    const bool deep = DEEP == 8 && mean_a > 20;
+    if constexpr (SOME8) {
+        if (!SOME4 || kk <= 8) {
+            if (big) JLUST_ROWS(4, 8, true);
+            else JLUST_ROWS(4, 8, false);
+            return check_launch("csr_spmm_rows_kernel");
+        }
+    }
+    if constexpr (SOME4) {
+        if (big) JLUST_ROWS(4, 4, true);
+        else if (kk <= 16 && deep) JLUST_ROWS(DEEP, 4, false);
+        else if (kk <= 16) JLUST_ROWS(4, 4, false);
+        else if (deep) JLUST_ROWS(DEEP, 2, false);
+        else JLUST_ROWS(4, 2, false);
+    }
 #undef JLUST_ROWS
     return check_launch("csr_spmm_rows_kernel");
 }
