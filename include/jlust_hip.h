@@ -25,8 +25,9 @@
  *  - Work is enqueued on `stream` (a hipStream_t; NULL = the null stream) and
  *    returns without synchronising.  Entry points are reentrant.  The library
  *    keeps one scratch buffer per (device, stream) for the SpMV/SpMM partial
- *    results, so concurrent calls must use different streams.  The buffer
- *    grows on demand and an outgrown one is kept, never freed, so work already
+ *    results and copies of B, so concurrent calls must use different streams
+ *    (the COO and CSC SDDMM have one of their own and order themselves).  The
+ *    buffer grows on demand and an outgrown one is kept, never freed, so work already
  *    queued and HIP graphs that captured a call stay valid.  Capturing a call
  *    in a graph: make one call of the same size on the capturing stream first
  *    (no allocation may happen inside a capture); prepared plans own their
@@ -593,7 +594,11 @@ int jlust_hip_csr_sddmm_f32_i32(int64_t m, int64_t n, int64_t K, int64_t nnz,
  * mask's storage order.  Replaces the COO case of execute(::EmitterBackend,
  * ::Op{:SDDMM}) (ext/KernelAbstractionsExt/ops/sddmm.jl:49-65; reference
  * answer test/test_emitter.jl:289-307).  No analysis: a group of lanes per
- * entry reads A's row with stride lda; a prepared plan (below) puts the
+ * entry, over a row-major copy of A where K is 16 bytes to 1 KB, the mask has
+ * m entries or more and the copy stays within 1 GB.  The copy is in a scratch
+ * buffer per (device, stream), kept like the others; without the memory for it,
+ * and in a call under capture (which needs no warm-up), A is read with stride
+ * lda, with the same results bit for bit.  A prepared plan (below) puts the
  * entries in row order once and runs the CSR kernel instead.
  */
 int jlust_hip_coo_sddmm_f64_i32(int64_t m, int64_t n, int64_t K, int64_t nnz,

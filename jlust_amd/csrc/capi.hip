@@ -3,6 +3,7 @@
 #include <cstdarg>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -96,21 +97,21 @@ struct ScratchBuf {
     size_t bytes = 0;
 };
 static std::mutex g_scratch_mu;
-static std::map<std::pair<int, jlust_stream_t>, ScratchBuf> g_scratch;
+static std::map<std::tuple<int, jlust_stream_t, int>, ScratchBuf> g_scratch;
 // Buffers outgrown by a later call.  They are kept until the process ends:
 // work already queued may still read them, and so may any HIP graph that
 // captured a call on that stream and is replayed later.  Growth is by at
 // least a quarter, so the kept buffers stay within a few times the largest.
 static std::vector<void *> g_scratch_retired;
 
-int scratch(jlust_stream_t stream, size_t bytes, void **out)
+int scratch(jlust_stream_t stream, size_t bytes, void **out, int kind)
 {
     int dev = 0;
     int st = require_device(&dev);
     if (st) return st;
     return host_guard("scratch", [&]() -> int {
         std::lock_guard<std::mutex> lk(g_scratch_mu);
-        ScratchBuf &b = g_scratch[{dev, stream}];
+        ScratchBuf &b = g_scratch[{dev, stream, kind}];
         if (b.bytes < bytes) {
             const size_t want = bytes + bytes / 4 + 4096;
             if (b.ptr) g_scratch_retired.reserve(g_scratch_retired.size() + 1);   // before the hipMalloc

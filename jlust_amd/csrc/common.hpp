@@ -71,7 +71,9 @@ const DeviceInfo &device_info(int device);
 // private to (current device, stream).  It grows on demand; an outgrown
 // buffer is kept until process exit, since queued work or a captured graph
 // may still read it.
-int scratch(jlust_stream_t stream, size_t bytes, void **out);
+// kind: 0 = what the calls share that must not run at once on one stream; 1 =
+// the COO SDDMM's, which may (coo_sddmm orders its own).
+int scratch(jlust_stream_t stream, size_t bytes, void **out, int kind = 0);
 
 // out[i] = sum(in[0..i)) over n int32 counts (in == out allowed); stream-ordered.
 // Uses the stream's scratch buffer for chunk sums.

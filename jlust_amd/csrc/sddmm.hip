@@ -21,6 +21,7 @@
 // so K = 1 puts 64 nonzeros on a wave per load instead of 8.
 #include <algorithm>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -97,6 +98,19 @@ __device__ __forceinline__ void load_slices(int q, int K, const T *col, U16<T> (
         } else {
             b[st] = *reinterpret_cast<const U16<T> *>(col + at);
         }
+    }
+}
+
+// The same elements of a row whose elements lie ld apart.
+template <typename T, int G, int KS>
+__device__ __forceinline__ void load_slices_strided(int q, int K, const T *row, int64_t ld, U16<T> (&b)[KS])
+{
+    constexpr int NE = V16<T>::N;
+#pragma unroll
+    for (int st = 0; st < KS; ++st) {
+        const int k0 = (st * G + q) * NE, at = st == KS - 1 ? min(k0, K - NE) : k0;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) b[st].v[e] = row[(at + e) * ld];
     }
 }
 
@@ -293,15 +307,17 @@ __global__ __launch_bounds__(SD_BLOCK) void coo_sddmm_kernel(
     }
 }
 
-// COO mask over a row-major copy of A (At, rows of lda_t elements, 16-byte
+// COO mask over a row-major copy of A (A, rows of lda elements, 16-byte
 // aligned): a group of G lanes per stored entry in storage order, both rows
 // read as vectors with every load issued first.  A's row from column-major
 // memory takes a line per element instead (the kernel above): 27-point mesh of
-// 69k rows, K = 128, with the copy: f32 261 -> 96 us, f64 483 -> 155 us.
-template <typename T, int G, int U, int KS>
+// 69k rows, K = 128, with the copy: f32 261 -> 96 us, f64 483 -> 155 us.  Not
+// COPY: A itself, the same sums bit for bit, where the copy may not be made (in a
+// graph: f32 205 us with the kernel above, 169 here; f64 380, 334).
+template <typename T, int G, int U, int KS, bool COPY>
 __global__ __launch_bounds__(SD_BLOCK) void coo_sddmm_rows_kernel(
     int64_t nnz, int K, int32_t origin, const int32_t *__restrict__ rows, const int32_t *__restrict__ cols, T alpha,
-    const T *__restrict__ At, int64_t ld_t, const T *__restrict__ B, int64_t ldb, T beta, int beta_zero, T *Cval,
+    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb, T beta, int beta_zero, T *Cval,
     const T *mask)
 {
     constexpr int GROUPS = SD_BLOCK / G;
@@ -312,7 +328,8 @@ __global__ __launch_bounds__(SD_BLOCK) void coo_sddmm_rows_kernel(
         for (int u = 0; u < U; ++u) {
             const int64_t p = p0 + u * GROUPS < nnz ? p0 + u * GROUPS : p0;
             const int64_t i = (int64_t)rows[p] - origin, j = (int64_t)cols[p] - origin;
-            load_slices<T, SD_ANY, G, KS>(q, K, At + i * ld_t, av[u]);
+            if (COPY) load_slices<T, SD_ANY, G, KS>(q, K, A + i * lda, av[u]);
+            else load_slices_strided<T, G, KS>(q, K, A + i, lda, av[u]);
             load_slices<T, SD_ANY, G, KS>(q, K, B + j * ldb, bv[u]);
         }
 #pragma unroll
@@ -464,6 +481,64 @@ int dcsr_sddmm(int64_t m, int64_t n, int64_t K, int64_t nout, int64_t nnz, int32
                            nullptr, rows, m, (hipStream_t)stream);
 }
 
+template <typename T, bool COPY>
+int coo_sddmm_rows_launch(int64_t K, int64_t nnz, int32_t origin, const int32_t *rows, const int32_t *cols, T alpha,
+                          const T *A, int64_t lda, const T *B, int64_t ldb, T beta, T *Cval, const T *mask,
+                          hipStream_t s)
+{
+    constexpr int64_t N = V16<T>::N;
+    const int64_t slices = (K + N - 1) / N;
+#define JLUST_COO(G, U, KS)                                                                                      \
+    hipLaunchKernelGGL((coo_sddmm_rows_kernel<T, G, U, KS, COPY>),                                               \
+                       dim3((unsigned)std::min<int64_t>((nnz + SD_BLOCK / G * U - 1) / (SD_BLOCK / G * U),       \
+                                                        SD_GRID_MAX)),                                           \
+                       dim3(SD_BLOCK), 0, s, nnz, (int)K, origin, rows, cols, alpha, A, lda, B, ldb, beta,       \
+                       (int)(beta == T(0)), Cval, mask)
+    if (slices <= 1) JLUST_COO(1, 4, 1);
+    else if (slices <= 2) JLUST_COO(2, 4, 1);
+    else if (slices <= 4) JLUST_COO(4, 2, 1);
+    else if (slices <= 8) JLUST_COO(8, 1, 1);
+    else if (slices <= 16) JLUST_COO(8, 1, 2);
+    else if (slices <= 24) JLUST_COO(8, 1, 3);
+    else if (slices <= 32) JLUST_COO(8, 1, 4);
+    else if (slices <= 40) JLUST_COO(8, 1, 5);
+    else if (slices <= 48) JLUST_COO(8, 1, 6);
+    else if (slices <= 56) JLUST_COO(8, 1, 7);
+    else JLUST_COO(8, 1, 8);
+#undef JLUST_COO
+    return check_launch("coo_sddmm_rows_kernel");
+}
+
+// Over a row-major copy of A, in a scratch buffer of these calls alone: a call
+// on a stream that another thread uses too has its copy and its product in turn
+// under the lock, as one launch would be.  A itself where the stream is being
+// captured (a replay may run beside other calls, and no buffer grows in a
+// capture) and where there is no memory for the copy.
+template <typename T>
+int coo_sddmm_rows(int64_t m, int64_t K, int64_t nnz, int32_t origin, const int32_t *rows, const int32_t *cols,
+                   T alpha, const T *A, int64_t lda, int64_t ld_t, const T *B, int64_t ldb, T beta, T *Cval,
+                   const T *mask, hipStream_t s)
+{
+    static std::mutex locks[16];
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;
+    }
+    if (cap == hipStreamCaptureStatusNone) {
+        std::lock_guard<std::mutex> lk(locks[(uintptr_t)s / 64 % 16]);
+        void *ws = nullptr;
+        if (scratch((jlust_stream_t)s, sizeof(T) * (size_t)((m + 1) * ld_t), &ws, 1) == JLUST_STATUS_SUCCESS) {
+            if (int st = spmm_row_major_copy(sizeof(T) == 8 ? 0 : 1, m, K, A, lda, ws, ld_t, s)) return st;
+            return coo_sddmm_rows_launch<T, true>(K, nnz, origin, rows, cols, alpha, (const T *)ws, ld_t, B, ldb, beta,
+                                                  Cval, mask, s);
+        }
+        (void)hipGetLastError();
+        clear_error();
+    }
+    return coo_sddmm_rows_launch<T, false>(K, nnz, origin, rows, cols, alpha, A, lda, B, ldb, beta, Cval, mask, s);
+}
+
 template <typename T>
 int coo_sddmm(int64_t m, int64_t n, int64_t K, int64_t nnz, int32_t origin, const int32_t *rows,
               const int32_t *cols, T alpha, const T *A, int64_t lda, const T *B, int64_t ldb, T beta, T *Cval,
@@ -479,38 +554,12 @@ int coo_sddmm(int64_t m, int64_t n, int64_t K, int64_t nnz, int32_t origin, cons
     if (int st = require_device(nullptr)) return st;
     if (nnz == 0) return JLUST_STATUS_SUCCESS;
     // A row-major copy of A where K is whole loads of a group and the mask has
-    // more entries than a copy costs; the scratch buffer it takes cannot grow
-    // while the stream is being captured.
+    // more entries than a copy costs.
     constexpr int64_t N = V16<T>::N;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    JLUST_HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cap));
     const int64_t ld_t = (K + N - 1) / N * N;
-    if (K >= N && K <= 64 * N && nnz >= m && cap == hipStreamCaptureStatusNone &&
-        (m + 1) * ld_t * (int64_t)sizeof(T) <= (int64_t)1 << 30) {
-        void *ws = nullptr;
-        if (int st = scratch(stream, sizeof(T) * (size_t)((m + 1) * ld_t), &ws)) return st;
-        if (int st = spmm_row_major_copy(sizeof(T) == 8 ? 0 : 1, m, K, A, lda, ws, ld_t, (hipStream_t)stream)) return st;
-        const int64_t slices = ld_t / N;
-#define JLUST_COO(G, U, KS)                                                                                      \
-    hipLaunchKernelGGL((coo_sddmm_rows_kernel<T, G, U, KS>),                                                     \
-                       dim3((unsigned)std::min<int64_t>((nnz + SD_BLOCK / G * U - 1) / (SD_BLOCK / G * U),       \
-                                                        SD_GRID_MAX)),                                           \
-                       dim3(SD_BLOCK), 0, (hipStream_t)stream, nnz, (int)K, origin, rows, cols, alpha, (T *)ws,  \
-                       ld_t, B, ldb, beta, (int)(beta == T(0)), Cval, mask)
-        if (slices <= 1) JLUST_COO(1, 4, 1);
-        else if (slices <= 2) JLUST_COO(2, 4, 1);
-        else if (slices <= 4) JLUST_COO(4, 2, 1);
-        else if (slices <= 8) JLUST_COO(8, 1, 1);
-        else if (slices <= 16) JLUST_COO(8, 1, 2);
-        else if (slices <= 24) JLUST_COO(8, 1, 3);
-        else if (slices <= 32) JLUST_COO(8, 1, 4);
-        else if (slices <= 40) JLUST_COO(8, 1, 5);
-        else if (slices <= 48) JLUST_COO(8, 1, 6);
-        else if (slices <= 56) JLUST_COO(8, 1, 7);
-        else JLUST_COO(8, 1, 8);
-#undef JLUST_COO
-        return check_launch("coo_sddmm_rows_kernel");
-    }
+    if (K >= N && K <= 64 * N && nnz >= m && (m + 1) * ld_t * (int64_t)sizeof(T) <= (int64_t)1 << 30)
+        return coo_sddmm_rows<T>(m, K, nnz, origin, rows, cols, alpha, A, lda, ld_t, B, ldb, beta, Cval, mask,
+                                 (hipStream_t)stream);
     hipLaunchKernelGGL((coo_sddmm_kernel<T>),
                        dim3((unsigned)std::min<int64_t>((nnz + SD_GROUPS - 1) / SD_GROUPS, SD_GRID_MAX)), dim3(SD_BLOCK),
                        0, (hipStream_t)stream, nnz, K, origin, rows, cols, alpha, A, lda, B, ldb, beta,

@@ -249,3 +249,38 @@ def test_graph_bsr_plan(J, b1, b2, dtype):
     C = J.dense_matrix(mb * b1, k, dtype=tdt)
     C0 = torch.randn(k, mb * b1, dtype=tdt, device="cuda").t()
     check_replays(lambda: J.execute(J.SpMMOp, h, B, C, alpha=0.75, beta=1.5), B, C, C0)
+
+
+@pytest.mark.parametrize("K", [3, 17, 40, 100, 256])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_graph_coo_sddmm(J, dtype, K):
+    """The plain COO SDDMM captured: no copy of A there, and the bits of the
+    eager call, which makes one."""
+    import torch
+    m, n = 900, 700
+    tdt = torch.float64 if dtype == np.float64 else torch.float32
+    rowptr, colind, val = random_csr(m, n, lengths=np.random.default_rng(3).integers(0, 9, m), seed=4, dtype=dtype)
+    rows = np.repeat(np.arange(m, dtype=np.int32), np.diff(rowptr)) + 1
+    perm = np.random.default_rng(5).permutation(rows.size)
+    out = dev(val[perm].copy())
+    Cs = J.coo_tensor(dev(rows[perm]), dev(colind[perm]), out, (m, n))
+    A = torch.zeros(K, m, dtype=tdt, device="cuda").t()
+    Bm = torch.randn(n, K + 1, dtype=tdt, device="cuda").t()[:K]
+    check_replays(lambda: J.execute(J.SDDMMOp, A, Bm, Cs, alpha=0.5, beta=2.0), A, out, out.clone())
+
+
+def test_graph_bsr_small_plan(J):
+    """The prepared SpMM plan on small square blocks captured and replayed."""
+    import torch
+    mb, nb, b, k = 60, 50, 4, 24
+    rng = np.random.default_rng(17)
+    counts = rng.integers(0, 6, mb)
+    bc = (np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in counts]) + 1).astype(np.int32)
+    A = J.bsr_tensor(dev((np.r_[0, np.cumsum(counts)] + 1).astype(np.int32)), dev(bc),
+                     dev(rng.standard_normal(bc.size * b * b)), (mb * b, nb * b), (b, b))
+    h = J.prepare(J.HIPBackend(), J.SpMMOp, A, n_cols=k)
+    assert h.info()["path"] == "blocks"
+    B = J.dense_matrix(nb * b, k, dtype=torch.float64)
+    C = J.dense_matrix(mb * b, k, dtype=torch.float64)
+    C0 = torch.randn(k, mb * b, dtype=torch.float64, device="cuda").t()
+    check_replays(lambda: J.execute(J.SpMMOp, h, B, C, alpha=0.75, beta=1.5), B, C, C0)

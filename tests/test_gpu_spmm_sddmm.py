@@ -458,3 +458,39 @@ def test_sddmm_every_width(J, O, dtype, pad):
                 gbad = host(J.nonzeros(C))
                 np.testing.assert_array_equal(gbad[~hit], got[~hit], err_msg=f"{name} {call} K={K}")
                 assert not np.isfinite(gbad[hit]).any()
+
+
+def test_coo_sddmm_threads_on_one_stream(J):
+    """Two threads call the plain COO SDDMM on the same stream, each with an A
+    of its own: neither sees the other's copy."""
+    import threading
+
+    import torch
+    m, n, K, nnz, calls = 3000, 2500, 64, 9000, 200
+    gen = torch.Generator("cuda").manual_seed(8)
+    rows = torch.randint(1, m + 1, (nnz,), generator=gen, device="cuda", dtype=torch.int32)
+    cols = torch.randint(1, n + 1, (nnz,), generator=gen, device="cuda", dtype=torch.int32)
+    B = torch.randn(n, K, generator=gen, device="cuda").t()
+    As = [torch.randn(K, m, generator=gen, device="cuda").t() for _ in range(2)]
+    Cs = [[J.coo_tensor(rows, cols, torch.empty(nnz, device="cuda"), (m, n)) for _ in range(calls)] for _ in range(2)]
+    want = []
+    for A in As:
+        C = J.coo_tensor(rows, cols, torch.empty(nnz, device="cuda"), (m, n))
+        J.execute(J.SDDMMOp, A, B, C)
+        want.append(J.nonzeros(C).clone())
+    torch.cuda.synchronize()
+    start = threading.Barrier(2)
+
+    def work(i):
+        start.wait()
+        for C in Cs[i]:
+            J.execute(J.SDDMMOp, As[i], B, C)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(J.nonzeros(C), want[i]) for C in Cs[i])
