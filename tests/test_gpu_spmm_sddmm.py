@@ -494,3 +494,26 @@ def test_coo_sddmm_threads_on_one_stream(J):
     torch.cuda.synchronize()
     for i in range(2):
         assert all(torch.equal(J.nonzeros(C), want[i]) for C in Cs[i])
+
+
+@pytest.mark.parametrize("fmt", ["csr", "coo"])
+@pytest.mark.parametrize("K", [5, 9, 13, 17, 18, 25, 31, 39, 45, 70, 101, 255])
+def test_sddmm_rounding(J, K, fmt):
+    """Dot products of a width that is no whole vector are no further from 64
+    bits than sums over 8 lanes, an element each in turn.  Over these seeds the
+    ratio is 0.82 to 1.018; one sum a lane over whole vectors makes 1.029 at
+    K = 39."""
+    rng = np.random.default_rng(K)
+    m, n, per = 600, 500, 100
+    cols = np.sort(np.argsort(rng.random((m, n)), axis=1)[:, :per], axis=1).astype(np.int32)
+    A, B = rng.standard_normal((m, K)).astype(np.float32), rng.standard_normal((K, n)).astype(np.float32)
+    out = dev(np.zeros(m * per, np.float32))
+    rows = np.repeat(np.arange(m, dtype=np.int32), per)
+    C = (J.csr_tensor(dev((np.arange(m + 1) * per + 1).astype(np.int32)), dev(cols.reshape(-1) + 1), out, (m, n))
+         if fmt == "csr" else J.coo_tensor(dev(rows + 1), dev(cols.reshape(-1) + 1), out, (m, n)))
+    J.execute(J.SDDMMOp, dev(A), dev(B), C)
+    a, b = A[rows], B.T[cols.reshape(-1)]
+    exact = (a.astype(np.float64) * b).sum(-1)
+    rms = lambda c: np.sqrt(((c - exact) ** 2).mean())     # noqa: E731
+    got, want = rms(host(J.nonzeros(C))), rms(split_sums_f32(a, b, 8))
+    assert got <= 1.02 * want, f"{got / want:.3f}"
