@@ -431,3 +431,44 @@ def test_blocks_equal_two_steps(J, b1, b2, rm, dtype, origin, monkeypatch):
     check(2, 20, r, path=False)
     r = [np.array([0, 5])] * (4 * b1)
     check(4, 20, r, path=False, ptr=np.r_[1, np.arange(1, 4 * b1 + 1) * 2])
+
+
+@pytest.mark.parametrize("src,dst", [("CSR", "CSC"), ("CSC", "CSR"), ("CSC", "COO")])
+@pytest.mark.parametrize("gap", [4 * 8192 - 20, 4 * 8192 + 20, 20_000_000])
+def test_direct_over_empty_segments(J, src, dst, gap, monkeypatch):
+    """A long run of empty segments inside one tile of entries: bit for bit the
+    two-step conversion, in a time of its order (a workgroup that walked 20M
+    segments would take over 30 times as long)."""
+    import time
+
+    import torch
+    from jlust_amd import convert as CV
+    rng = np.random.default_rng(31)
+    side = 700_000                                          # entries on either side, 1 or 2 a segment
+    lens = np.concatenate([np.full(side // 2, 2), np.zeros(gap, np.int64), np.ones(side, np.int64), [0, 0]])
+    ncoord = 90_000
+    n = int(lens.sum())
+    p, c = np.r_[0, np.cumsum(lens)] + 1, rng.integers(0, ncoord, n) + 1
+    c[:side:2], c[1:side:2] = np.minimum(c[:side:2], ncoord - 1), np.minimum(c[:side:2], ncoord - 1) + 1
+    dims = (lens.size, ncoord) if src == "CSR" else (ncoord, lens.size)
+    make = J.csr_tensor if src == "CSR" else CV.csc_tensor
+    u = make(*(torch.from_numpy(t).cuda() for t in (p.astype(np.int32), c.astype(np.int32), rng.standard_normal(n))),
+             dims)
+    direct, out, took = CV._convert_direct, [], []
+    for general in (False, True):
+        monkeypatch.setattr(CV, "_convert_direct", (lambda *a: None) if general else direct)
+        best = 1e9
+        for _ in range(3):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            r = J.convert_format(u, fmt_of(J, dst))
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t)
+        out.append(r)
+        took.append(best)
+    monkeypatch.setattr(CV, "_convert_direct", direct)
+    assert CV._convert_direct(u, fmt_of(J, dst), CV._descriptor(u), CV._format_id(fmt_of(J, dst))[0], u.val.device)
+    a, b = out
+    for x, y in zip((*a.pos_buffers, *a.crd_buffers, a.val), (*b.pos_buffers, *b.crd_buffers, b.val)):
+        assert (x is None) == (y is None) and (x is None or torch.equal(x, y))
+    assert took[0] < 4 * took[1] + 1e-3
