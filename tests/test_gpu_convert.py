@@ -305,6 +305,12 @@ def test_direct_equals_two_steps(J, src, dst, dtype, origin, monkeypatch):
     import torch
     from jlust_amd import convert as CV
     rng = np.random.default_rng(17)
+    direct, taken = CV._convert_direct, []
+
+    def recorded(*a):
+        r = direct(*a)
+        taken.append(r is not None)
+        return r
 
     def run(nseg, ncoord, lens, repeat=False, zeros=0.0, ptr=None):
         ends = np.r_[0, np.cumsum(lens)]
@@ -328,9 +334,9 @@ def test_direct_equals_two_steps(J, src, dst, dtype, origin, monkeypatch):
         out = []
         for general in (False, True):
             with monkeypatch.context() as mp:
-                if general:
-                    mp.setattr(CV, "_convert_direct", lambda *a: None)
+                mp.setattr(CV, "_convert_direct", (lambda *a: None) if general else recorded)
                 out.append(J.convert_format(u, fmt_of(J, dst)))
+        assert taken.pop() == (ptr is None)
         a, b = out
         assert a.val.numel() == b.val.numel()
         it = torch.int64 if dtype == np.float64 else torch.int32
