@@ -25,6 +25,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "wave.hpp"
 
 namespace jlust {
 namespace {
@@ -37,13 +38,6 @@ template <typename T, int N>
 struct alignas(sizeof(T) * N < 16 ? sizeof(T) * N : 16) Pack {
     T v[N];
 };
-
-// Orders a wave's LDS accesses (its lanes exchange values through LDS).
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 struct SmallShape {
     int64_t mb;

@@ -30,6 +30,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "common.hpp"
+#include "wave.hpp"
 
 namespace jlust {
 namespace {
@@ -747,13 +748,6 @@ __global__ __launch_bounds__(256) void sort_ptr_kernel(const uint32_t *__restric
 // general path takes, 1,263 us (1,195 there; 1,651 with 8,192 allowed).
 constexpr int BR_WAVES = 4, BR_BLOCKS = 1024, BR_ENTRIES = 2048, BR_STAGE = 2048, BR_DIM = 8;
 
-// Orders a wave's LDS accesses (its lanes exchange values through LDS).
-__device__ __forceinline__ void br_wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // The least i in [lo, hi) with a[i] >= x, hi if none.
 __device__ __forceinline__ int br_lower(const int32_t *a, int lo, int hi, int x)
 {
@@ -873,7 +867,7 @@ __global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse s
             for (int j = 0; j < 4; ++j)
                 if (q + 64 * j < p1) staged[q + 64 * j - p0] = e[j];
         }
-        br_wave_sync();
+        wave_sync();
         find([&](int p) { return staged[p - p0]; });
     } else {
         find(load);
@@ -882,7 +876,7 @@ __global__ __launch_bounds__(64 * BR_WAVES) void bsr_heads_kernel(jlust_sparse s
         if (lane == 0) flags[0] = 1;
         return;
     }
-    br_wave_sync();
+    wave_sync();
     for (int i = lane; i < nb; i += 64) {
         const int x = h[i];
         int rank = 0;
@@ -928,7 +922,7 @@ __global__ __launch_bounds__(64 * BR_WAVES) void bsr_blocks_kernel(jlust_sparse 
         for (int i = lane; i < nb * bb; i += 64) blocks[i] = T(0);
         __threadfence_block();                            // these stores, then the entries'
     }
-    br_wave_sync();
+    wave_sync();
     for (int q0 = p0; q0 < p1; q0 += 64) {
         const int p = q0 + lane;
         int r = 0;

@@ -27,21 +27,6 @@ constexpr int SPMM_BLOCK = 256;
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 constexpr int SPMM_ROWS = 32;
 
-template <typename T>
-__device__ __forceinline__ T bcast(T v, int lane);
-template <>
-__device__ __forceinline__ float bcast<float>(float v, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-template <>
-__device__ __forceinline__ double bcast<double>(double v, int lane)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 __device__ __forceinline__ int bcast_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 
 template <typename T, int VEC> struct Vec;
@@ -214,7 +199,8 @@ __device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 
 // Row-split SpMM over the row-major copy of B.  A wave's 64 lanes form
 // NG = 64 / L groups; a group takes a row, each lane VEC columns of B's row per
-// entry, so one vector load of a wave serves NG entries of NG rows and no sum crosses lanes.  What bounds it is the gathers: L1 and L2 where rows share
+// entry, so one vector load of a wave serves NG entries of NG rows and no sum
+// crosses lanes.  What bounds it is the gathers: L1 and L2 where rows share
 // columns, the fabric behind the L2s where they do not.
 //   - The block's entries (colind turned into an offset into Bt, and val) are
 //     staged in LDS with coalesced loads and read back by the groups: a load
@@ -695,9 +681,13 @@ int spmm_group_launch(int64_t m, int64_t kk, int64_t nnz_rows, int32_t origin, c
         else if (steps <= 4) JLUST_GROUP_U(KV, 4);                                                     \
         else JLUST_GROUP_U(KV, 8);                                                                     \
     } while (0)
-    if (kk == 1) JLUST_GROUP(1);
-    else if (kk == 2) JLUST_GROUP(2);
-    else JLUST_GROUP(4);
+    if (kk == 1) {
+        JLUST_GROUP(1);
+    } else if (kk == 2) {
+        JLUST_GROUP(2);
+    } else {
+        if constexpr (sizeof(T) == 4) JLUST_GROUP(4);   // f64: 2 columns at most (spmm_chunk_kind)
+    }
 #undef JLUST_GROUP
 #undef JLUST_GROUP_U
     return check_launch("csr_spmm_group_kernel");

@@ -1,5 +1,5 @@
-// wave.hpp -- wave64 cross-lane helpers (DPP segmented scan) shared by the
-// SpMV kernels.
+// wave.hpp -- wave64 cross-lane helpers: a DPP segmented scan, and the order of
+// a wave's LDS accesses.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -7,6 +7,13 @@
 #include <cstdint>
 
 namespace jlust {
+
+// Orders a wave's LDS accesses (its lanes exchange values through LDS).
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // ---- wave64 DPP (GFX9 controls): row_shr:n = 0x110+n, row_bcast:15 = 0x142,
 // row_bcast:31 = 0x143, wave_shr:1 = 0x138.  Lanes without a source keep `old`.
