@@ -966,7 +966,7 @@ int jlust_hip_convert_analyze_ws(const jlust_sparse *src, int32_t dst_format,
                                  int64_t *dst_nnz, int64_t *dst_nouter);
 
 /* CSR to CSC, CSC to CSR and CSC to COO in one call, without a handle: the
- * entries move to the target's buffers in two or three passes.  workspace
+ * entries move to the target's buffers in one to three passes.  workspace
  * reports the device bytes of ws (256-byte aligned); 0: not a conversion of
  * this kind, or one the two steps do better.  dst: origin and extents of src,
  * nnz = src->nnz, its buffers allocated for that many entries.  *count: the

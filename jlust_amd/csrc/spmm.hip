@@ -200,8 +200,10 @@ __device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 // Row-split SpMM over the row-major copy of B.  A wave's 64 lanes form
 // NG = 64 / L groups; a group takes a row, each lane VEC columns of B's row per
 // entry, so one vector load of a wave serves NG entries of NG rows and no sum
-// crosses lanes.  What bounds it is the gathers: L1 and L2 where rows share
-// columns, the fabric behind the L2s where they do not.
+// crosses lanes.  What bounds it is the gathers: L1 where rows share columns (the
+// f64 mesh below: an access in 94 % of its cycles), the fabric behind the L2s
+// where they do not (200k power-law rows below: L2 hits 14 %, 6.7 TB/s past it;
+// 1M uniform rows, 64 columns: 4 %, 7.6 TB/s).
 //   - The block's entries (colind turned into an offset into Bt, and val) are
 //     staged in LDS with coalesced loads and read back by the groups: a load
 //     of col and val by each group would take as many address cycles as the
@@ -512,10 +514,10 @@ __global__ void spmm_long_reduce_kernel(int64_t nlong, int64_t kk, const int32_t
 //     567 us).
 //   - The group kernel for one column, and for 2 to 4 (f64: 2) where rows hold
 //     more than 48 entries on average: so few columns leave the rows kernel's
-//     slices too few for its groups (200 entries a row, band of +-150, f32:
-//     k = 2 86.9 against 50.9 us, k = 4 99.4 against 74.7 us; f64: k = 2 92.8
-//     against 68.6, k = 4 107.7 against 125.9; with 27 entries, f32, k = 4,
-//     27.6 against 54.2 us).
+//     slices too few for its groups (100k rows of 200, band of +-150, f32:
+//     k = 2 79.7 against 47.5 us, k = 4 92.4 against 72.3 us; f64: k = 2 92.3
+//     against 65.2, k = 4 106 against 126; with 27 entries, f32, k = 4, 27.6
+//     against 54.2 us).
 struct SpmmChunk {
     bool group;                          // the group kernel
     bool direct;                         // B's own column, no copy
