@@ -525,6 +525,8 @@ int coo_sddmm_rows_launch(int64_t K, int64_t nnz, int32_t origin, const int32_t 
     return check_launch("coo_sddmm_rows_kernel");
 }
 
+std::mutex g_coo_locks[16];            // by stream, for both value types
+
 // Over a row-major copy of A, in a scratch buffer of these calls alone: a call
 // on a stream that another thread uses too has its copy and its product in turn
 // under the lock, as one launch would be.  A itself where the stream is being
@@ -535,14 +537,13 @@ int coo_sddmm_rows(int64_t m, int64_t K, int64_t nnz, int32_t origin, const int3
                    T alpha, const T *A, int64_t lda, int64_t ld_t, const T *B, int64_t ldb, T beta, T *Cval,
                    const T *mask, hipStream_t s)
 {
-    static std::mutex locks[16];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
         (void)hipGetLastError();
         cap = hipStreamCaptureStatusActive;
     }
     if (cap == hipStreamCaptureStatusNone) {
-        std::lock_guard<std::mutex> lk(locks[(uintptr_t)s / 64 % 16]);
+        std::lock_guard<std::mutex> lk(g_coo_locks[(uintptr_t)s / 64 % 16]);
         void *ws = nullptr;
         if (scratch((jlust_stream_t)s, sizeof(T) * (size_t)((m + 1) * ld_t), &ws, 1) == JLUST_STATUS_SUCCESS) {
             if (int st = spmm_row_major_copy(sizeof(T) == 8 ? 0 : 1, m, K, A, lda, ws, ld_t, s)) return st;

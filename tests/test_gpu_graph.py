@@ -284,3 +284,25 @@ def test_graph_bsr_small_plan(J):
     C = J.dense_matrix(mb * b, k, dtype=torch.float64)
     C0 = torch.randn(k, mb * b, dtype=torch.float64, device="cuda").t()
     check_replays(lambda: J.execute(J.SpMMOp, h, B, C, alpha=0.75, beta=1.5), B, C, C0)
+
+
+def test_graph_bsr_small_update(J):
+    """New values of a plan on small square blocks, read and used inside a graph."""
+    import torch
+    mb, nb, b, k = 60, 50, 3, 24
+    rng = np.random.default_rng(18)
+    counts = rng.integers(0, 6, mb)
+    bc = (np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in counts]) + 1).astype(np.int32)
+    vals = dev(rng.standard_normal(bc.size * b * b))
+    A = J.bsr_tensor(dev((np.r_[0, np.cumsum(counts)] + 1).astype(np.int32)), dev(bc), vals, (mb * b, nb * b), (b, b))
+    h = J.prepare(J.HIPBackend(), J.SpMMOp, A, n_cols=k)
+    assert h.info()["path"] == "blocks"
+    B = torch.randn(k, nb * b, dtype=torch.float64, device="cuda").t()
+    C = J.dense_matrix(mb * b, k, dtype=torch.float64)
+    C0 = torch.randn(k, mb * b, dtype=torch.float64, device="cuda").t()
+
+    def run():
+        J.update_values_(h, A)
+        J.execute(J.SpMMOp, h, B, C, alpha=0.75, beta=1.5)
+
+    check_replays(run, vals, C, C0)

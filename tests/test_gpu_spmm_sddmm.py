@@ -460,7 +460,8 @@ def test_sddmm_every_width(J, O, dtype, pad):
                 assert not np.isfinite(gbad[hit]).any()
 
 
-def test_coo_sddmm_threads_on_one_stream(J):
+@pytest.mark.parametrize("types", ["f32 f32", "f32 f64"])
+def test_coo_sddmm_threads_on_one_stream(J, types):
     """Two threads call the plain COO SDDMM on the same stream, each with an A
     of its own: neither sees the other's copy."""
     import threading
@@ -470,12 +471,14 @@ def test_coo_sddmm_threads_on_one_stream(J):
     gen = torch.Generator("cuda").manual_seed(8)
     rows = torch.randint(1, m + 1, (nnz,), generator=gen, device="cuda", dtype=torch.int32)
     cols = torch.randint(1, n + 1, (nnz,), generator=gen, device="cuda", dtype=torch.int32)
-    B = torch.randn(n, K, generator=gen, device="cuda").t()
-    As = [torch.randn(K, m, generator=gen, device="cuda").t() for _ in range(2)]
-    Cs = [[J.coo_tensor(rows, cols, torch.empty(nnz, device="cuda"), (m, n)) for _ in range(calls)] for _ in range(2)]
+    dts = [torch.float64 if t == "f64" else torch.float32 for t in types.split()]
+    Bs = [torch.randn(n, K, generator=gen, device="cuda", dtype=dt).t() for dt in dts]
+    As = [torch.randn(K, m, generator=gen, device="cuda", dtype=dt).t() for dt in dts]
+    Cs = [[J.coo_tensor(rows, cols, torch.empty(nnz, device="cuda", dtype=dt), (m, n)) for _ in range(calls)]
+          for dt in dts]
     want = []
-    for A in As:
-        C = J.coo_tensor(rows, cols, torch.empty(nnz, device="cuda"), (m, n))
+    for A, B, dt in zip(As, Bs, dts):
+        C = J.coo_tensor(rows, cols, torch.empty(nnz, device="cuda", dtype=dt), (m, n))
         J.execute(J.SDDMMOp, A, B, C)
         want.append(J.nonzeros(C).clone())
     torch.cuda.synchronize()
@@ -484,7 +487,7 @@ def test_coo_sddmm_threads_on_one_stream(J):
     def work(i):
         start.wait()
         for C in Cs[i]:
-            J.execute(J.SDDMMOp, As[i], B, C)
+            J.execute(J.SDDMMOp, As[i], Bs[i], C)
 
     threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
     for t in threads:
