@@ -798,8 +798,8 @@ int jlust_hip_bsr_expand_csr_i32(int64_t mb, int64_t b1, int64_t b2,
  * C = alpha*A*B + beta*C for square blocks of 2 to 8 rows on the blocks as
  * stored: *taken = 1 if the product ran, 0 if it is left to
  * jlust_hip_bsr_expand_csr_i32 + the CSR entry points (another shape, k < 2,
- * 24 columns of B past 4 GiB, no memory for B's copy, block-rows far longer
- * than the mean, or a browptr that is not canonical).  B's copy is in the
+ * 24 columns of B past 4 GiB, no memory for B's copy, a block-row that
+ * one group of lanes would be too long at, or a browptr that is not canonical).  B's copy is in the
  * stream's scratch buffer, up to 1 GB of it or 16 columns.  Arguments as jlust_hip_bsr_spmm_*.  Reads the
  * longest block-row back, so it synchronises `stream` (not capturable; a plan
  * is).
@@ -821,8 +821,8 @@ int jlust_hip_bsr_spmm_small_f32_i32(int64_t mb, int64_t nb, int64_t b1, int64_t
  * execute many times, update_values! for new values of the same pattern).
  * 16 x 16 blocks keep the MFMA kernels (fp32, with 16-byte aligned values
  * for BSRRight, or fp64) and read the caller's buffers in place.  Square
- * blocks of 2 to 8 rows whose longest block-row holds at most 64 blocks or 4
- * times the mean run as stored (k >= 2; the plan owns a copy of the values and
+ * blocks of 2 to 8 rows whose longest block-row is no tail of its own (40 blocks,
+ * or more where the product is large enough to cover it) run as stored (k >= 2; the plan owns a copy of the values and
  * one of B).  Any other b1 x b2 shape is expanded to CSR once
  * (jlust_hip_bsr_expand_csr_i32's layout; the plan owns it) and runs through a
  * CSR SpMM plan over it for k columns.  create synchronises `stream` (browptr

@@ -371,7 +371,29 @@ size_t bsr_small_copy_bytes(int64_t nb, int64_t b, int64_t k, size_t tsz)
     return tsz * (size_t)(nb * b + 1) * (size_t)((small_kchunk(nb, b, k, tsz) + 7) / 8 * 8);
 }
 
-int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *browptr, hipStream_t s, bool *even)
+// The longest block-row that the kernel takes.  A group of lanes walks its
+// block-row alone, 0.5 (2 x 2) to 1.6 us (8 x 8) a block, about 0.2 * b; the
+// expansion shares long rows among the card and takes an entry in the time of
+// its k values, 64 bytes at least, at 8 TB/s, a plain call 132 bytes more for
+// making it.  So a row may have as many blocks as pass while the expansion's
+// entries do; 40 in a plan and 512 / b in a plain call, whose expansion takes 90
+// us and more, in any case; and 64 or 4 times the mean at most.  us, this kernel /
+// the expansion, plan, 4 x 4 f64, k = 24: 512 block-rows of 1024 blocks 644 /
+// 196, 2048 of 64 59 / 43, 4096 of 64 59 / 59, 8192 of 128 103 / 193; 8 x 8:
+// 1024 of 128 232 / 123, 4096 of 128 281 / 449; f32: 2 x 2, k = 8, 2048 of 1024
+// 514 / 75, 16384 of 128 74 / 70; 4 x 4, k = 6, 16384 of 128 105 / 237.  Plain, 4
+// x 4 f64, k = 24: 512 of 256 233 / 191, 2048 of 256 224 / 309; 2 x 2 f32, k = 8,
+// 4096 of 512 314 / 276, 8192 of 512 302 / 421.  8 block-rows of 65,536 4 x 4
+// blocks: 47 ms here, 0.4 by the expansion.
+static int64_t small_longest(int64_t mb, int64_t nnzb, int64_t b, int64_t k, size_t tsz, bool plan)
+{
+    const double entry = std::max(64.0, (double)k * (double)tsz) + (plan ? 0.0 : 132.0);
+    const double most = std::max(plan ? 40.0 : 512.0 / (double)b, (double)nnzb * (double)b * entry / 1.6e6);
+    return (int64_t)std::min(most, (double)std::max<int64_t>(64, 4 * nnzb / mb));
+}
+
+int bsr_small_pattern(int64_t mb, int64_t nnzb, int64_t b, int64_t k, size_t tsz, bool plan, int32_t origin,
+                      const int32_t *browptr, hipStream_t s, bool *even)
 {
     *even = false;
     if (mb == 0 || nnzb == 0) return JLUST_STATUS_SUCCESS;
@@ -387,7 +409,7 @@ int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *b
     JLUST_HIP_TRY(hipMemcpyAsync(&ends[1], browptr + mb, 4, hipMemcpyDeviceToHost, s));
     JLUST_HIP_TRY(hipStreamSynchronize(s));
     if (ends[0] != origin || (int64_t)ends[1] - origin != nnzb || h[1]) return JLUST_STATUS_SUCCESS;
-    *even = h[0] <= std::max<int64_t>(64, 4 * nnzb / mb);
+    *even = h[0] <= small_longest(mb, nnzb, b, k, tsz, plan);
     return JLUST_STATUS_SUCCESS;
 }
 

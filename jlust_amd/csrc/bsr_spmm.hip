@@ -2646,7 +2646,7 @@ extern "C" int jlust_hip_bsr_expand_csr_i32(int64_t mb, int64_t b1, int64_t b2, 
 // handle contract, ext/CUDAExt/ops/spmm.jl:8-70, for BSR).  16 x 16 blocks,
 // Float32 or Float64, keep the MFMA kernels and the caller's buffers
 // (update_values swaps the value pointer).  Square blocks of 2 to 8 rows whose
-// block-rows are of even length run as stored (bsr_small.hip); any other block
+// longest block-row is short enough run as stored (bsr_small.hip); any other block
 // shape is expanded to CSR once and runs through a CSR SpMM plan over it.
 // Which of the two a shape takes depends on its pattern, so both keep the
 // values in memory of the plan's own: a caller may reuse or free its buffer
@@ -2712,7 +2712,8 @@ static int bsr_spmm_plan_create_body(int64_t mb, int64_t nb, int64_t b1, int64_t
               (value_type == 0 || !row_major_blocks || (uintptr_t)val % 16 == 0);
     const size_t tsz = value_type == 0 ? sizeof(double) : sizeof(float);
     if (!p->mfma && bsr_small_shape(nb, b1, b2, k, tsz))
-        if (int st = bsr_small_pattern(mb, nnzb, origin, browptr, (hipStream_t)stream, &p->small)) return st;
+        if (int st = bsr_small_pattern(mb, nnzb, b1, k, tsz, true, origin, browptr, (hipStream_t)stream, &p->small))
+            return st;
     if (p->small) {
         const size_t sz_v = bsr_align_up(tsz * (size_t)total, 256);
         if (hipMalloc(&p->mem, sz_v + bsr_small_copy_bytes(nb, b1, k, tsz)) != hipSuccess) {
@@ -2842,7 +2843,7 @@ static int bsr_small_call(int64_t mb, int64_t nb, int64_t b1, int64_t b2, int64_
     if (!bsr_small_shape(nb, b1, b2, k, sizeof(T))) return JLUST_STATUS_SUCCESS;
     hipStream_t s = (hipStream_t)stream;
     bool even = false;
-    if (int st = bsr_small_pattern(mb, nnzb, origin, browptr, s, &even)) return st;
+    if (int st = bsr_small_pattern(mb, nnzb, b1, k, sizeof(T), false, origin, browptr, s, &even)) return st;
     if (!even) return JLUST_STATUS_SUCCESS;
     if (int st = bsr_small_dense_args(mb * b1, nb * b2, k, B, ldb, C, ldc)) return st;
     void *Bt = nullptr;

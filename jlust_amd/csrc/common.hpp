@@ -130,11 +130,12 @@ int spmm_row_major_copy(int value_type, int64_t n, int64_t k, const void *B, int
 
 // BSR SpMM on small square blocks (bsr_small.hip): whether a shape is one of
 // its; the bytes of B's copy of one pass (Bt); whether browptr runs from the origin to
-// nnzb + origin without decreasing and has no block-row much longer than the
-// others (*even; synchronises s); the product.
+// nnzb + origin without decreasing and has no block-row too long for the kernel
+// (*even; synchronises s); the product.
 bool bsr_small_shape(int64_t nb, int64_t b1, int64_t b2, int64_t k, size_t tsz);
 size_t bsr_small_copy_bytes(int64_t nb, int64_t b, int64_t k, size_t tsz);
-int bsr_small_pattern(int64_t mb, int64_t nnzb, int32_t origin, const int32_t *browptr, hipStream_t s, bool *even);
+int bsr_small_pattern(int64_t mb, int64_t nnzb, int64_t b, int64_t k, size_t tsz, bool plan, int32_t origin,
+                      const int32_t *browptr, hipStream_t s, bool *even);
 template <typename T>
 int bsr_small_spmm(int64_t mb, int64_t nb, int64_t b, int32_t origin, const int32_t *browptr, const int32_t *bcolind,
                    const T *val, int row_major, int64_t k, T alpha, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,

@@ -1493,7 +1493,7 @@ class HIPBSRSpMMHandle(AbstractKernelHandle):
     SpMMOp, A::BSR; n_cols=k) -> execute(h, B, C) -> update_values!(h, A), the
     cuSPARSE SpMM handle contract (ext/CUDAExt/ops/spmm.jl:8-70) for BSR.
     16 x 16 blocks run the MFMA kernels (fp32 or fp64) on A's buffers, square
-    blocks of 2 to 8 rows in block-rows of even length a kernel of their own;
+    blocks of 2 to 8 rows without overlong block-rows a kernel of their own;
     any other block shape is expanded to CSR once and runs through a CSR SpMM
     plan over the expansion.  A's values are read as they are at the
     call: where the plan has values of its own (all but the MFMA kernels),

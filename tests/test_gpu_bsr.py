@@ -842,3 +842,34 @@ def test_bsr_small_blocks_rounding(J, b, k):
         rms = lambda c: np.sqrt(((c.reshape(exact.shape) - exact) ** 2).mean())     # noqa: E731
         got, want = rms(host(C)), rms(split_sums_f32(a, x, sums))
         assert got <= 1.09 * want, f"{blocks} blocks: {got / want:.3f}"
+
+
+@pytest.mark.parametrize("mb,per,path", [(8, 4096, "csr_expansion"), (1, 3000, "csr_expansion"), (700, 41, "csr_expansion"),
+                                         (700, 40, "blocks"), (2100, 100, "blocks"), (2000, 100, "csr_expansion")])
+@pytest.mark.parametrize("call", ["plain", "plan"])
+def test_bsr_small_blocks_long_rows(J, mb, per, path, call):
+    """Block-rows that are all long: one group of lanes would walk each alone,
+    so few of them go to the expansion (8 rows of 4096 blocks took 2.5 ms), many
+    stay; exact on integers."""
+    import torch
+    b, k, nb = 4, 24, 6000
+    gen = torch.Generator("cuda").manual_seed(per)
+    bc = torch.rand(mb, nb, generator=gen, device="cuda").argsort(1)[:, :per].sort(1).values
+    vals = torch.randint(-4, 5, (mb * per, b, b), generator=gen, device="cuda").double()
+    B = torch.randint(-3, 4, (k, nb * b), generator=gen, device="cuda").double().t()
+    A = J.bsr_tensor((torch.arange(mb + 1, device="cuda") * per + 1).int(), (bc.reshape(-1) + 1).int(), vals.reshape(-1),
+                     (mb * b, nb * b), (b, b), True)
+    C = J.dense_matrix(mb * b, k, dtype=torch.float64, fill=float("nan"))
+    if call == "plain":
+        J.execute(J.SpMMOp, A, B, C)
+    else:
+        h = J.prepare(J.HIPBackend(), J.SpMMOp, A, n_cols=k)
+        assert h.info()["path"] == path
+        J.execute(h, B, C)
+    Bb = B.contiguous().view(nb, b, k)
+    want = torch.zeros(mb, b, k, dtype=torch.float64, device="cuda")
+    for j in range(b):
+        for s in range(0, per, 50):
+            e = min(per, s + 50)
+            want += (vals.view(mb, per, b, b)[:, s:e, :, j, None] * Bb[bc[:, s:e], j][:, :, None, :]).sum(1)
+    assert torch.equal(C, want.view(mb * b, k))
