@@ -307,7 +307,7 @@ int launch(const SmallShape &base, const int32_t *browptr, const int32_t *bcolin
     sh.wave_stride = sh.sums_at + (LV - 1) * B * CPL * 64;
     const size_t per_wave = sizeof(T) * (size_t)sh.wave_stride;
     const int64_t wgs = (sh.mb + (int64_t)BS_WAVES * NG - 1) / (BS_WAVES * NG);
-    sh.run = (unsigned)((wgs + 4 * NUM_XCD - 1) / (4 * NUM_XCD));
+    sh.run = xcd_run(wgs);
     const dim3 grid((unsigned)((wgs + (int64_t)sh.run * NUM_XCD - 1) / ((int64_t)sh.run * NUM_XCD) * sh.run * NUM_XCD),
                     (unsigned)ny);
     hipLaunchKernelGGL((bsr_small_spmm_kernel<T, B, CPL, LV>), grid, dim3(BS_BLOCK), per_wave * BS_WAVES, s, sh, browptr,

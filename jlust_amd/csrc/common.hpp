@@ -128,6 +128,19 @@ int spmm_plan_adopt_reorder(jlust_spmm_plan_t plan, void *mem, const int32_t *pe
 int spmm_row_major_copy(int value_type, int64_t n, int64_t k, const void *B, int64_t ldb, void *Bt, int64_t ldt,
                         hipStream_t s);
 
+// Consecutive workgroups per XCD of a launch of n that numbers them in such runs,
+// so that neighbours share an L2: 8 runs an XCD, and 16 workgroups a run where
+// that leaves four.  With four long runs an XCD, rows whose entries lie in one
+// eighth of them (a graph ordered by degree) kept four XCDs busy: 100k rows, 128
+// entries in each of the first eighth, f64, k = 100: 474 us, 218 with 8.  Meshes
+// lose by shorter ones (f32, 262k rows, k = 24: 55 us with 4 and 8, 58 with 16).
+inline unsigned xcd_run(int64_t n)
+{
+    auto runs = [&](int64_t per) { return (n + per * NUM_XCD - 1) / (per * NUM_XCD); };
+    const int64_t few = runs(4) < 16 ? runs(4) : 16, run = runs(8) > few ? runs(8) : few;
+    return (unsigned)(run > 0 ? run : 1);
+}
+
 // BSR SpMM on small square blocks (bsr_small.hip): whether a shape is one of
 // its; the bytes of B's copy of one pass (Bt); whether browptr runs from the origin to
 // nnzb + origin without decreasing and has no block-row too long for the kernel

@@ -604,8 +604,7 @@ int spmm_rows_launch(int64_t n, int64_t kk, int64_t nnz_rows, int64_t nnz_seg, i
     ja.R = spmm_rows_per_block<T>(ja.rows, mean_a, ngb, sh.slice_log2, sh.cld);
     jb.R = spmm_rows_per_block<T>(jb.rows, mean_b, ngb, sh.slice_log2, sh.cld);
     const int64_t nb = (ja.rows + ja.R - 1) / ja.R;
-    ja.run = (unsigned)((nb + 4 * NUM_XCD - 1) / (4 * NUM_XCD));
-    if (ja.run == 0) ja.run = 1;
+    ja.run = xcd_run(nb);
     ja.blocks = (unsigned)((nb + ja.run * NUM_XCD - 1) / (ja.run * NUM_XCD) * (ja.run * NUM_XCD));
     jb.blocks = (unsigned)((jb.rows + jb.R - 1) / jb.R);
     sh.rmax = max(ja.R, jb.rows ? jb.R : 1);
