@@ -596,9 +596,9 @@ int jlust_hip_csr_sddmm_f32_i32(int64_t m, int64_t n, int64_t K, int64_t nnz,
  * answer test/test_emitter.jl:289-307).  No analysis: a group of lanes per
  * entry, over a row-major copy of A where K is 16 bytes to 1 KB, the mask has
  * m entries or more and the copy stays within 1 GB.  The copy is in a scratch
- * buffer per (device, stream), kept like the others; without the memory for it,
- * and in a call under capture (which needs no warm-up), A is read with stride
- * lda, with the same results bit for bit.  A prepared plan (below) puts the
+ * buffer per (device, stream), kept like the others; in small calls, without the
+ * memory for it, and in a call under capture (which needs no warm-up), A is read
+ * with stride lda, with the same results bit for bit.  A prepared plan (below) puts the
  * entries in row order once and runs the CSR kernel instead.
  */
 int jlust_hip_coo_sddmm_f64_i32(int64_t m, int64_t n, int64_t K, int64_t nnz,

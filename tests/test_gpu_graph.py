@@ -251,13 +251,14 @@ def test_graph_bsr_plan(J, b1, b2, dtype):
     check_replays(lambda: J.execute(J.SpMMOp, h, B, C, alpha=0.75, beta=1.5), B, C, C0)
 
 
-@pytest.mark.parametrize("K", [3, 17, 40, 100, 256])
+@pytest.mark.parametrize("K", [3, 17, 40, 70, 100, 128, 150, 190, 220, 256])
+@pytest.mark.parametrize("m", [900, 40_000])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-def test_graph_coo_sddmm(J, dtype, K):
+def test_graph_coo_sddmm(J, dtype, m, K):
     """The plain COO SDDMM captured: no copy of A there, and the bits of the
-    eager call, which makes one."""
+    eager call, which makes one for the larger mask."""
     import torch
-    m, n = 900, 700
+    n = 700
     tdt = torch.float64 if dtype == np.float64 else torch.float32
     rowptr, colind, val = random_csr(m, n, lengths=np.random.default_rng(3).integers(0, 9, m), seed=4, dtype=dtype)
     rows = np.repeat(np.arange(m, dtype=np.int32), np.diff(rowptr)) + 1

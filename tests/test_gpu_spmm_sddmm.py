@@ -467,7 +467,7 @@ def test_coo_sddmm_threads_on_one_stream(J, types):
     import threading
 
     import torch
-    m, n, K, nnz, calls = 3000, 2500, 64, 9000, 200
+    m, n, K, nnz, calls = 3000, 2500, 64, 90000, 100
     gen = torch.Generator("cuda").manual_seed(8)
     rows = torch.randint(1, m + 1, (nnz,), generator=gen, device="cuda", dtype=torch.int32)
     cols = torch.randint(1, n + 1, (nnz,), generator=gen, device="cuda", dtype=torch.int32)
