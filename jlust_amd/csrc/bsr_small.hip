@@ -241,18 +241,21 @@ __global__ __launch_bounds__(BS_BLOCK) void bsr_small_spmm_kernel(
     }
 }
 
-// longest[0] = the longest block-row, longest[1] set where browptr decreases.
-__global__ void block_row_longest_kernel(int64_t mb, const int32_t *__restrict__ browptr, int32_t *__restrict__ longest)
+// out[0] = the longest block-row, out[1] set where browptr decreases, out[2] and
+// out[3] its ends: one copy to the host, which costs a plain call more than the
+// kernel does.
+__global__ void block_row_longest_kernel(int64_t mb, const int32_t *__restrict__ browptr, int32_t *__restrict__ out)
 {
     int32_t len = 0;
     for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < mb; r += (int64_t)gridDim.x * blockDim.x) {
         const int64_t d = (int64_t)browptr[r + 1] - browptr[r];
-        if (d < 0) longest[1] = 1;
+        if (d < 0) out[1] = 1;
         len = max(len, (int32_t)min(d, (int64_t)INT32_MAX));
     }
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) len = max(len, __shfl_xor(len, off, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(longest, len);
+    if ((threadIdx.x & 63) == 0) atomicMax(out, len);
+    if (blockIdx.x == 0 && threadIdx.x < 2) out[2 + threadIdx.x] = browptr[threadIdx.x * mb];
 }
 
 __global__ void clear_pair_kernel(int32_t *p)
@@ -399,16 +402,14 @@ int bsr_small_pattern(int64_t mb, int64_t nnzb, int64_t b, int64_t k, size_t tsz
     if (mb == 0 || nnzb == 0) return JLUST_STATUS_SUCCESS;
     void *ws = nullptr;
     if (int st = scratch((jlust_stream_t)s, 64, &ws)) return st;
-    int32_t *d = (int32_t *)ws, h[2] = {0, 0}, ends[2] = {0, 0};
+    int32_t *d = (int32_t *)ws, h[4] = {0, 0, 0, 0};
     hipLaunchKernelGGL(clear_pair_kernel, dim3(1), dim3(64), 0, s, d);
     hipLaunchKernelGGL(block_row_longest_kernel, dim3((unsigned)min((mb + 255) / 256, (int64_t)512)), dim3(256), 0, s,
                        mb, browptr, d);
     if (int st = check_launch("block_row_longest_kernel")) return st;
     JLUST_HIP_TRY(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
-    JLUST_HIP_TRY(hipMemcpyAsync(&ends[0], browptr, 4, hipMemcpyDeviceToHost, s));
-    JLUST_HIP_TRY(hipMemcpyAsync(&ends[1], browptr + mb, 4, hipMemcpyDeviceToHost, s));
     JLUST_HIP_TRY(hipStreamSynchronize(s));
-    if (ends[0] != origin || (int64_t)ends[1] - origin != nnzb || h[1]) return JLUST_STATUS_SUCCESS;
+    if (h[2] != origin || (int64_t)h[3] - origin != nnzb || h[1]) return JLUST_STATUS_SUCCESS;
     *even = h[0] <= small_longest(mb, nnzb, b, k, tsz, plan);
     return JLUST_STATUS_SUCCESS;
 }
