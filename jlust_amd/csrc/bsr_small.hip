@@ -297,8 +297,13 @@ int launch(const SmallShape &base, const int32_t *browptr, const int32_t *bcolin
     SmallShape sh = base;
     const int64_t ny = (sh.k + 64 * CPL - 1) / (64 * CPL);
     sh.cols = (int)(((sh.k + ny - 1) / ny + CPL - 1) / CPL * CPL);
-    // Lanes beyond the columns where a stage would not hold a block otherwise.
-    sh.L = max(sh.cols / CPL, (B * B + BS_STAGE - 1) / BS_STAGE);
+    // Lanes beyond the columns where a stage would not hold a block otherwise; for
+    // blocks up to 4 x 4, four values a lane: with eight, two lanes hold a block and
+    // 32 block-rows' blocks, a line or more apart, make up each load.  Mesh of 27
+    // blocks a row, 38^3, k = 2, against eight: 4 x 4 f32 70 -> 34 us, f64 57 -> 45;
+    // 3 x 3 f32 50 -> 36, f64 52 -> 37; against the expansion 52, 94, 43, 59.
+    // Larger blocks fill their loads with eight (8 x 8 f64: 74 us, 98 with four).
+    sh.L = max(sh.cols / CPL, (B * B + (B <= 4 ? 4 : BS_STAGE) - 1) / (B <= 4 ? 4 : BS_STAGE));
     const int NG = 64 / sh.L;
     constexpr int V16 = 16 / (int)sizeof(T), AW = B <= 2 ? 2 : V16 < 4 ? 2 : 4, BP = (B + AW - 1) / AW * AW;
     sh.sb = max(1, min(min(8, sh.L), BS_STAGE * sh.L / (B * B)));
